@@ -226,6 +226,68 @@ def test_backward_kernel_equals_tensor_operations(sorted_rows, n_cells):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("asked_for", ["distances", "vectors", "both"])
+@pytest.mark.parametrize("n_pairs", [1, 63, 65, 511, 512, 513, 262_144, 524_289])
+def test_backward_at_the_edges_of_its_workgroups(n_pairs, asked_for):
+    """Numbers of rows around a wave, a workgroup's round and the lists where a workgroup takes more rows, of points in
+    runs of neighbouring indices (17 per run: groups of eight slots that are full, and one begun), with either
+    gradient missing. A sum of m terms in another order differs by m ulp of the sum of their magnitudes at most."""
+    import ctypes
+
+    from vesin_amd._c_api import VesinCUDA, VesinDevice, get_library
+
+    n_points = 40_013
+    generator = torch.Generator(device="cuda:0").manual_seed(n_pairs)
+    rows = torch.arange(n_pairs, device="cuda:0")
+    i = (rows // 40) % n_points
+    j = (i + 17 * torch.randint(0, 30, (n_pairs,), device="cuda:0", generator=generator) + rows % 17) % n_points
+    pairs = torch.stack([i, j], dim=1)
+    shifts = torch.randint(-2, 3, (n_pairs, 3), dtype=torch.int32, device="cuda:0", generator=generator)
+    vectors = torch.randn((n_pairs, 3), dtype=torch.float64, device="cuda:0", generator=generator)
+    distances = vectors.norm(dim=1)
+    distances_grad = torch.randn(n_pairs, dtype=torch.float64, device="cuda:0", generator=generator)
+    vectors_grad = torch.randn((n_pairs, 3), dtype=torch.float64, device="cuda:0", generator=generator)
+    distances_grad *= asked_for != "vectors"
+    vectors_grad *= asked_for != "distances"
+    points_grad = torch.zeros((n_points, 3), dtype=torch.float64, device="cuda:0")
+    box_grad = torch.zeros((3, 3), dtype=torch.float64, device="cuda:0")
+    message = ctypes.c_char_p()
+    status = get_library().vesin_hip_pairs_backward(
+        pairs.data_ptr(), shifts.data_ptr(), distances.data_ptr(), vectors.data_ptr(), n_pairs,
+        None if asked_for == "vectors" else distances_grad.data_ptr(),
+        None if asked_for == "distances" else vectors_grad.data_ptr(), n_points, VesinDevice(VesinCUDA, 0),
+        points_grad.data_ptr(), box_grad.data_ptr(), None, ctypes.byref(message),
+    )
+    assert status == 0, message.value
+    expected_points, expected_box = _backward_with_tensor_operations(
+        pairs, shifts, distances, vectors, distances_grad, vectors_grad, n_points
+    )
+    magnitudes = vectors_grad.abs() + (distances_grad / distances)[:, None].abs() * vectors.abs()
+    of_points = torch.zeros_like(points_grad).index_add(0, j, magnitudes).index_add(0, i, magnitudes)
+    terms = torch.bincount(pairs.flatten(), minlength=n_points)[:, None]
+    ulp = 2.0**-52
+    assert bool(((points_grad - expected_points).abs() <= (terms + 4) * ulp * of_points).all())
+    of_box = shifts.abs().to(torch.float64).t() @ magnitudes
+    assert bool(((box_grad - expected_box).abs() <= (n_pairs + 4) * ulp * of_box).all())
+
+
+@pytest.mark.gpu
+def test_an_output_without_a_gradient_of_its_own_adds_nothing():
+    """Energies of the distances or of the vectors only: the gradient of the output that was not used is not there,
+    and both together are the sum."""
+    points = torch.rand((300, 3), dtype=torch.float64, device="cuda:0", generator=torch.Generator("cuda:0").manual_seed(2))
+    points = (8.0 * points).requires_grad_()
+    box = (8.0 * torch.eye(3, dtype=torch.float64, device="cuda:0")).requires_grad_()
+    d, D = NeighborList(cutoff=3.0, full_list=True, sorted=True).compute(points, box, True, "dD")
+    weights = torch.tensor([0.3, -1.1, 0.7], dtype=torch.float64, device="cuda:0")
+    of_d = torch.autograd.grad((d**2).sum(), (points, box), retain_graph=True)
+    of_D = torch.autograd.grad((D @ weights).sum(), (points, box), retain_graph=True)
+    of_both = torch.autograd.grad((d**2).sum() + (D @ weights).sum(), (points, box))
+    for one, other, both in zip(of_d, of_D, of_both):
+        assert float((one + other - both).abs().max()) <= 1e-12 * float(both.abs().max())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n_points", [7, 3000, 200_000])
 def test_backward_with_rows_in_no_order(n_points):
     """Rows that name points at random: with many points a workgroup meets more of them than its table in LDS

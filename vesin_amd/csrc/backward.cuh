@@ -16,7 +16,11 @@
 
 namespace vesin_hip {
 
-constexpr int BACKWARD_THREADS = 256;
+// Bound by reading the rows (56 bytes with a gradient of the distances only, 92 with everything). The table of sums fills
+// 58 KB of LDS, so two workgroups share a compute unit: with 256 threads each, too few loads are in flight, with 1024
+// the waves wait for each other where the table is filled and emptied (89 M rows, gradient of the distances: 1484 /
+// 1056 / 1115 us with 256 / 512 / 1024 threads).
+constexpr int BACKWARD_THREADS = 512;
 
 struct BackwardArgs {
     const size_t (*pairs)[2];
@@ -30,6 +34,7 @@ struct BackwardArgs {
     double* points_grad;           // [n_points][3] or nullptr
     double* box_grad;              // [3][3] or nullptr
     uint32_t* bad_index;           // set to 1 when a pair names a point that does not exist
+    size_t rows_per_block;         // a multiple of BACKWARD_THREADS (see backward_rows_per_block)
 };
 
 /// Sum over the 64 lanes of a wave, result in every lane.
@@ -63,29 +68,54 @@ __device__ inline void sum_runs(uint64_t heads, double& gx, double& gy, double& 
 /// Sums of one workgroup, by point, in LDS: rows that follow each other in a list name few different points (the
 /// points of a few cells), so most additions meet here and only one sum per point and workgroup goes to memory,
 /// where an atomic on a line shared by all compute dies costs far more than one in LDS.
+///
+/// The table is open addressing in groups of eight slots: the eight points 8k ... 8k + 7 share a group, each at its own
+/// place in it. Points of neighbouring indices are then neighbours in the table, and the workgroup's atomics to
+/// memory, one lane per component, come as stretches of up to 192 consecutive bytes. (Measured with 512 threads, 89 M
+/// rows, gradient of the distances, points spread by a hash of the whole index and added one point per lane -> like
+/// this: 1358 -> 1057 us, sorted 1785 -> 1101 us, atoms in no order 1333 -> 1195 us: 4.7 TB/s of rows read, where a
+/// plain copy on this GPU moves 4.8.)
 constexpr uint32_t BACKWARD_SLOTS = 2048;
+constexpr uint32_t BACKWARD_GROUP = 8;
 constexpr uint32_t BACKWARD_PROBES = 8;
 constexpr uint32_t BACKWARD_EMPTY = 0xFFFFFFFFu;
-constexpr size_t BACKWARD_ROWS_PER_BLOCK = 8192;
+
+/// Rows that one workgroup takes. Many rows let more additions meet in the table (1,000,000 atoms of diamond, 89 M rows,
+/// gradient of the distances: 1190 / 1098 / 1064 us with 2048 / 4096 / 8192 rows, 1101 with 16384); lists of fewer rows
+/// go for two workgroups on every one of the 256 compute units (50,000 atoms, 2.1 M rows, everything asked for: 55.6 /
+/// 47.7 / 46.1 / 57.4 us with 1024 / 2048 / 4096 / 8192 rows; sorted, of atoms in no order: 147 / 157 / 211 / 250 us).
+inline size_t backward_rows_per_block(size_t n_pairs) {
+    size_t rows = 8192;
+    while (rows > static_cast<size_t>(BACKWARD_THREADS) && n_pairs / rows < 512) {
+        rows /= 2;
+    }
+    return rows;
+}
 
 struct BackwardShared {
     uint32_t keys[BACKWARD_SLOTS];
     double sums[BACKWARD_SLOTS][3];
+    double box[BACKWARD_THREADS / WAVE][9];
 };
 
 __device__ inline void add_to_point(BackwardShared& shared, double* points_grad, size_t point, double gx, double gy, double gz) {
     const uint32_t key = static_cast<uint32_t>(point);
-    uint32_t slot = (key * 2654435761u) >> (32 - 11);
-    static_assert(BACKWARD_SLOTS == (1u << 11), "the hash keeps 11 bits");
+    uint32_t slot = (((key / BACKWARD_GROUP) * 2654435761u) >> (32 - 8)) * BACKWARD_GROUP + key % BACKWARD_GROUP;
+    static_assert(BACKWARD_SLOTS == (1u << 8) * BACKWARD_GROUP, "the hash keeps 8 bits");
     for (uint32_t probe = 0; probe < BACKWARD_PROBES; probe++) {
-        const uint32_t found = atomicCAS(&shared.keys[slot], BACKWARD_EMPTY, key);
+        // most points are in the table already: a read, which all lanes with the same point share, comes before the
+        // compare-and-swap, which goes through them one by one
+        uint32_t found = __atomic_load_n(&shared.keys[slot], __ATOMIC_RELAXED);
+        if (found == BACKWARD_EMPTY) {
+            found = atomicCAS(&shared.keys[slot], BACKWARD_EMPTY, key);
+        }
         if (found == BACKWARD_EMPTY || found == key) {
             unsafeAtomicAdd(&shared.sums[slot][0], gx);
             unsafeAtomicAdd(&shared.sums[slot][1], gy);
             unsafeAtomicAdd(&shared.sums[slot][2], gz);
             return;
         }
-        slot = (slot + 1) & (BACKWARD_SLOTS - 1);
+        slot = (slot + BACKWARD_GROUP) & (BACKWARD_SLOTS - 1);
     }
     // the neighbourhood of the slot is taken by other points
     unsafeAtomicAdd(points_grad + 3 * point + 0, gx);
@@ -111,8 +141,8 @@ __global__ __launch_bounds__(BACKWARD_THREADS) void pairs_backward_kernel(Backwa
 
     // a workgroup takes rows that follow each other; every lane of a wave runs the same number of rounds (the sums
     // over runs use the whole wave)
-    const size_t block_first = static_cast<size_t>(blockIdx.x) * BACKWARD_ROWS_PER_BLOCK;
-    const size_t block_end = min(block_first + BACKWARD_ROWS_PER_BLOCK, args.n_pairs);
+    const size_t block_first = static_cast<size_t>(blockIdx.x) * args.rows_per_block;
+    const size_t block_end = min(block_first + args.rows_per_block, args.n_pairs);
     for (size_t base = block_first + (threadIdx.x & ~(WAVE - 1)); base < block_end; base += BACKWARD_THREADS) {
         const size_t row = base + lane;
         bool active = row < block_end;
@@ -185,23 +215,35 @@ __global__ __launch_bounds__(BACKWARD_THREADS) void pairs_backward_kernel(Backwa
 
     if (args.points_grad != nullptr) {
         __syncthreads();
-        for (uint32_t slot = threadIdx.x; slot < BACKWARD_SLOTS; slot += BACKWARD_THREADS) {
+        for (uint32_t at = threadIdx.x; at < 3 * BACKWARD_SLOTS; at += BACKWARD_THREADS) {
+            const uint32_t slot = at / 3;
             const uint32_t key = shared.keys[slot];
             if (key != BACKWARD_EMPTY) {
-                double* target = args.points_grad + 3 * static_cast<size_t>(key);
-                unsafeAtomicAdd(target + 0, shared.sums[slot][0]);
-                unsafeAtomicAdd(target + 1, shared.sums[slot][1]);
-                unsafeAtomicAdd(target + 2, shared.sums[slot][2]);
+                unsafeAtomicAdd(args.points_grad + 3 * static_cast<size_t>(key) + (at - 3 * slot), shared.sums[slot][at - 3 * slot]);
             }
         }
     }
 
-    if (args.box_grad != nullptr && __ballot(any_shift) != 0) {
+    if (args.box_grad != nullptr) {
+        // one atomic per workgroup and component: they all go to the same 72 bytes, one after the other (with one per
+        // wave a list of 2.1 M rows took 150 us instead of 57, one of 89 M rows 1864 us instead of 1576)
+        const uint32_t wave = threadIdx.x / WAVE;
+        const bool wave_has_shift = __ballot(any_shift) != 0;
 #pragma unroll
         for (int k = 0; k < 9; k++) {
-            const double total = wave_sum(box_sum[k]);
-            if (lane == 0 && total != 0.0) {
-                unsafeAtomicAdd(args.box_grad + k, total);
+            const double total = wave_has_shift ? wave_sum(box_sum[k]) : 0.0;
+            if (lane == 0) {
+                shared.box[wave][k] = total;
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x < 9) {
+            double total = 0.0;
+            for (int w = 0; w < BACKWARD_THREADS / WAVE; w++) {
+                total += shared.box[w][threadIdx.x];
+            }
+            if (total != 0.0) {
+                unsafeAtomicAdd(args.box_grad + threadIdx.x, total);
             }
         }
     }

@@ -4586,7 +4586,8 @@ void pairs_backward(
     if (n_points > 0xFFFFFFF0ull) {
         throw std::runtime_error("too many points: the GPU path indexes points with 32 bits");
     }
-    const size_t wanted = (n_pairs + BACKWARD_ROWS_PER_BLOCK - 1) / BACKWARD_ROWS_PER_BLOCK;
+    args.rows_per_block = backward_rows_per_block(n_pairs);
+    const size_t wanted = (n_pairs + args.rows_per_block - 1) / args.rows_per_block;
     if (wanted > 0x7FFFFFFFull) {
         throw std::runtime_error("too many pairs for one launch");
     }

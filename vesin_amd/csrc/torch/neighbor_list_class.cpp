@@ -107,6 +107,9 @@ public:
         context->saved_data["points_grad"] = points.requires_grad();
         context->saved_data["box_grad"] = box.requires_grad() && any_periodic;
         context->saved_data["n_points"] = points.size(0);
+        // an output the caller did not use arrives as an undefined gradient, which the kernel skips: filled in with
+        // zeros, the vectors of a list of 89 M rows are 2.1 GB written (0.30 ms) and read again (0.4 ms) for nothing
+        context->set_materialize_grads(false);
         return {distances, vectors};
     }
 
