@@ -1,0 +1,158 @@
+"""sorted=True on crowded cells: the in-order search without fixed sizes (forced with VESIN_HIP_SORT=crowded) gives the
+list of the oracle, in the order (i, j, S), bit for bit; and the systems that the usual in-order search does not cover
+come to it by themselves."""
+
+import numpy as np
+import pytest
+
+import oracle
+from vesin_amd import NeighborList, configs
+
+pytestmark = pytest.mark.gpu
+
+NAMES = {"P": "pairs", "S": "shifts", "d": "distances", "D": "vectors"}
+
+
+def _expected(points, box, periodic, cutoff, full):
+    flags = [bool(periodic)] * 3 if isinstance(periodic, bool) else list(periodic)
+    return oracle.canonicalize(oracle.neighbors(points, box, flags, cutoff, full, False, "ijSdD"))
+
+
+def _compute(calculator, points, box, periodic, quantities="PSdD"):
+    import torch
+
+    outputs = calculator.compute(
+        torch.tensor(np.ascontiguousarray(points), device="cuda:0"), torch.tensor(np.ascontiguousarray(box), device="cuda:0"),
+        periodic, quantities,
+    )
+    return {NAMES[q]: out.cpu().numpy() for q, out in zip(quantities, outputs)}
+
+
+def _check(points, box, periodic, cutoff, full, capfd, monkeypatch, covered=True, calls=2):
+    expected = _expected(points, box, periodic, cutoff, full)
+    monkeypatch.setenv("VESIN_HIP_SORT", "crowded")
+    monkeypatch.setenv("VESIN_HIP_DEBUG", "1")
+    calculator = NeighborList(cutoff=cutoff, full_list=full, sorted=True)
+    for call in range(calls):
+        capfd.readouterr()
+        result = _compute(calculator, points, box, periodic)
+        lines = [line for line in capfd.readouterr().err.splitlines() if line.startswith("crowded search:")]
+        # (after a system it does not cover, a list leaves that search alone for a while)
+        assert len(lines) > 0 or (not covered and call > 0)
+        assert result["pairs"].shape == expected["pairs"].shape
+        for key in result:
+            assert np.array_equal(result[key], expected[key]), (call, key)
+
+
+def _liquid(n, edge, seed, outside=0.0, skew=0.0):
+    rng = np.random.default_rng(seed)
+    box = edge * np.array([[1.0, 0.0, 0.0], [0.6 * skew, 1.05, 0.0], [skew, 0.4 * skew, 1.1]])
+    return (rng.uniform(-outside, 1.0 + outside, size=(n, 3))) @ box, box
+
+
+@pytest.mark.parametrize("full", [True, False])
+@pytest.mark.parametrize("periodic", [(True, True, True), (True, False, True), (False, False, False)])
+@pytest.mark.parametrize(
+    "n,edge,cutoff,outside,skew",
+    [
+        (1, 5.0, 2.0, 0.0, 0.0),
+        (33, 4.0, 3.0, 0.3, 0.2),       # one cell, a tile of 32 points would leave one over; images of the same points
+        (700, 9.0, 3.0, 0.0, 0.3),      # 27 cells
+        (2500, 12.0, 3.0, 0.6, 0.2),    # cells of 39 points (two tiles), points up to half a box outside
+        (300, 30.0, 3.0, 0.0, 0.0),     # a third of a point per cell
+        (4000, 9.0, 3.0, 0.0, 0.0),     # 148 points per cell, 4000 candidates: the sort of the most crowded cells
+    ],
+)
+def test_liquids(n, edge, cutoff, outside, skew, periodic, full, capfd, monkeypatch):
+    points, box = _liquid(n, edge, n, outside, skew)
+    _check(points, box, periodic, cutoff, full, capfd, monkeypatch)
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 255, 257, 767, 768, 769, 1535, 1537, 2047, 2048, 2049])
+def test_numbers_of_candidates(n, capfd, monkeypatch):
+    """One cell: n candidates for every point, around a unit, a chunk of the writing pass and the two sorts; most of
+    them neighbours, more rows of a point than are lined up at a time."""
+    rng = np.random.default_rng(n)
+    _check(rng.random((n, 3)), np.eye(3), False, 1.3, n % 2 == 0, capfd, monkeypatch)
+
+
+@pytest.mark.parametrize("n,covered", [(8192, True), (8193, False)])
+def test_the_most_candidates(n, covered, capfd, monkeypatch):
+    """27 cells in a periodic box: every point of the system is a candidate of every cell."""
+    points, box = _liquid(n, 3.0, 5)
+    _check(points, box, True, 0.999, False, capfd, monkeypatch, covered)
+
+
+@pytest.mark.parametrize("order", ["lattice", "shuffled", "reversed"])
+@pytest.mark.parametrize("full", [True, False])
+def test_orders_of_the_points(order, full, capfd, monkeypatch):
+    points, box, _ = configs.diamond(7, seed=3)
+    if order == "shuffled":
+        points = points[np.random.default_rng(1).permutation(len(points))]
+    if order == "reversed":
+        points = points[::-1]
+    _check(points, box, True, 5.0, full, capfd, monkeypatch)
+
+
+def test_coincident_points_and_shifts_beyond_the_key(capfd, monkeypatch):
+    points, box = _liquid(900, 9.0, 8)
+    points[100:200] = points[0:100]
+    _check(points, box, True, 3.0, True, capfd, monkeypatch)
+    points[::2] += 300.0 * box[0]
+    _check(points, box, True, 3.0, True, capfd, monkeypatch, covered=False)
+
+
+def test_a_list_that_meets_other_systems(capfd, monkeypatch):
+    """More points, more candidates around as many points, fewer rows: the room of the call before is too small, the
+    arrays too."""
+    monkeypatch.setenv("VESIN_HIP_SORT", "crowded")
+    calculator = NeighborList(cutoff=3.0, full_list=True, sorted=True)
+    for n, edge in [(500, 12.0), (2000, 12.0), (2000, 9.0), (2000, 20.0), (1000, 8.0), (1000, 8.0)]:
+        points, box = _liquid(n, edge, n)
+        expected = _expected(points, box, True, 3.0, True)
+        result = _compute(calculator, points, box, True)
+        for key in result:
+            assert np.array_equal(result[key], expected[key]), (n, edge, key)
+
+
+@pytest.mark.parametrize("quantities", ["P", "PS", "Pd", "PD", "PSd"])
+def test_quantities(quantities, monkeypatch):
+    monkeypatch.setenv("VESIN_HIP_SORT", "crowded")
+    points, box = _liquid(1200, 9.0, 4, 0.2, 0.2)
+    expected = _expected(points, box, True, 3.0, False)
+    calculator = NeighborList(cutoff=3.0, full_list=False, sorted=True)
+    for _ in range(2):
+        result = _compute(calculator, points, box, True, quantities)
+        for key in result:
+            assert np.array_equal(result[key], expected[key]), key
+
+
+@pytest.mark.parametrize("kind", ["many candidates", "many rows", "mostly empty"])
+def test_systems_that_come_by_themselves(kind, capfd, monkeypatch):
+    """Called three times (first call, after the usual search reported that it does not cover the system, again), the
+    last time in two halves."""
+    import torch
+
+    monkeypatch.setenv("VESIN_HIP_DEBUG", "1")
+    rng = np.random.default_rng(2)
+    if kind == "many candidates":
+        (points, box), cutoff, periodic = _liquid(4000, 9.0, 1), 3.0, True
+    elif kind == "many rows":
+        points, box, cutoff, periodic = 1.5 * rng.random((600, 3)), 20.0 * np.eye(3), 3.0, True
+    else:
+        # two blobs in a box of 1.3 M cells: records of a fixed size per cell would take 3 GB
+        points = np.concatenate([rng.normal(size=(1500, 3)), 110.0 + rng.normal(size=(200_000, 3)) * 60.0])
+        box, cutoff, periodic = 220.0 * np.eye(3), 2.0, True
+    expected = _expected(points, box, periodic, cutoff, True)
+    calculator = NeighborList(cutoff=cutoff, full_list=True, sorted=True)
+    for call in range(3):
+        capfd.readouterr()
+        if call < 2:
+            result = _compute(calculator, points, box, periodic)
+        else:
+            device_points, device_box = torch.tensor(points, device="cuda:0"), torch.tensor(box, device="cuda:0")
+            calculator.enqueue(device_points, device_box, torch.tensor([True] * 3, device="cuda:0"), "PSdD")
+            result = {NAMES[q]: out.cpu().numpy() for q, out in zip("PSdD", calculator.collect())}
+        assert "crowded search:" in capfd.readouterr().err
+        for key in result:
+            assert np.array_equal(result[key], expected[key]), (call, key)

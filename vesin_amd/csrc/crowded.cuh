@@ -1,0 +1,736 @@
+// In-order search of systems that ordered.cuh does not cover because their cells are crowded (more than 1024 candidates
+// around a tile, or more than 256 rows of a point: dense clusters, cutoffs of several interatomic distances) or because
+// there are too many cells for its records of a fixed size (clusters in a wide, mostly empty box).
+//
+// The scheme is the same: every tile tests its points against the whole stencil, so every row is found by the tile of
+// its first point; candidates in the order of (original index, shift) make the hits of a point, taken in that order,
+// its rows in final order. What differs is how the work is laid out, so that nothing is of a fixed size:
+//   MEASURE  every cell that holds points counts its candidates and takes room for them, and for one word per
+//            candidate and tile, from a running total (where the room lies in memory does not enter the result);
+//   SORT     one workgroup per cell, not per tile: the tiles of a cell share their candidates. Candidates are grouped in
+//            LDS by ranges of the original index (buckets), then ranked inside their bucket, and go to memory as
+//            (position in the cell-sorted arrays, biased shift less the wrap of the first point) in final order;
+//   COUNT    one workgroup per tile, the candidates dealt to its four waves: hit columns in the order of the candidates,
+//            rows of every point;
+//   a scan over the points gives every point its first row;
+//   WRITE    one workgroup per tile, which brings CROWDED_CHUNK candidates at a time to LDS (coordinates, index, shift,
+//            hit column); its waves share the points. A wave walks the columns for a point, lines up the hits, and
+//            stores 64 consecutive rows at a time, which need nothing from memory but LDS.
+// A point may have any number of rows; a cell at most CROWDED_LARGE candidates (their sort takes the LDS of a compute
+// unit then). Beyond that, and for shifts or wraps beyond +-255, the host falls back to the radix sort.
+//
+// Measured per call, radix sort -> this: 500,000 points in 50 clusters (82 M rows, P d) 12.7 -> 1.67 ms, (P S d D) 17.9 ->
+// 2.27 ms; 200,000 atoms of diamond, cutoff 6.5 (1480 candidates per tile, P S d) 6.04 -> 1.04 ms; 13,824 atoms, cutoff 5.5
+// 358 -> 167 us; a liquid of 20,000 points, cutoff 7, 649 -> 208 us; 2,000 points, cutoff 7, 180 -> 147 us. On systems that
+// the usual in-order search covers it is the slower one, its passes follow each other where that one sorts beside its
+// counting (1,000,000 atoms of diamond 1.81 against 2.30 ms, 100,000 points of a liquid 274 against 430 us).
+//
+// Arithmetic and order as in ordered.cuh (vesin/src/cpu_cell_list.cpp:135-138, vesin/src/types.hpp:232-243).
+#ifndef VESIN_HIP_CROWDED_CUH
+#define VESIN_HIP_CROWDED_CUH
+
+#include "ordered.cuh"
+
+namespace vesin_hip {
+
+constexpr int CROWDED_WAVES = 4;
+constexpr int CROWDED_BLOCK = CROWDED_WAVES * WAVE;
+constexpr uint32_t CROWDED_SMALL = 2048;   // candidates that the usual sorting kernel takes (29 KB of LDS)
+constexpr uint32_t CROWDED_LARGE = 8192;   // and the one for the most crowded cells (103 KB)
+constexpr int CROWDED_SORT_BLOCK = 512;    // threads of the latter
+constexpr uint32_t CROWDED_CHUNK = 768;    // candidates that a workgroup of WRITE holds in LDS: four workgroups per unit
+constexpr uint32_t CROWDED_STEP = 4;       // units of candidates between two looks at how many rows are lined up
+constexpr uint32_t CROWDED_STAGED = (CROWDED_STEP + 1) * WAVE;
+
+/// A candidate, in the order of (original index, shift).
+struct CrowdedCandidate {
+    uint32_t at;     // position in the cell-sorted arrays
+    uint32_t biased; // cell shift less the wrap of the candidate, biased (see biased_shift)
+};
+
+/// What a cell was given, at the number of its first tile.
+struct CrowdedCell {
+    uint32_t candidates;      // 0: no room (see CrowdedStatus::overflow), or too many
+    uint32_t first_candidate; // in units of 64
+    uint32_t first_column;    // in units of 64, of the cell's first tile; the next tiles follow
+    uint32_t padding;
+};
+
+/// Device memory, cleared before MEASURE.
+struct CrowdedStatus {
+    unsigned long long used; // units of 64 candidates taken | units of 64 hit columns taken << 32
+    unsigned int max_candidates;
+    unsigned int unsuitable; // a shift or wrap outside of the key's range
+    unsigned int overflow;   // cells that found no room left
+    unsigned int padding;
+};
+
+/// What the host reads after COUNT and the scan (pinned host memory).
+struct CrowdedHostStatus {
+    CrowdedStatus found;
+    unsigned long long total_rows;
+    unsigned int first_bad_coordinate;
+    unsigned int n_tiles;
+};
+
+struct CrowdedArgs {
+    SortedPoints sorted;
+    const uint64_t* cell_scan;
+    const Tile* tiles;
+    CrowdedCell* cells;           // [tile slots]
+    CrowdedCandidate* candidates; // [candidate_units * 64]
+    uint32_t* columns;            // [column_units * 64]
+    uint32_t candidate_units;
+    uint32_t column_units;
+    CrowdedStatus* status;
+    uint32_t* rows_of_point;      // COUNT: [n_points], by original index
+    const uint64_t* first_row;    // WRITE: [n_points + 1], their exclusive scan
+    uint64_t capacity;            // WRITE: rows that the output arrays hold; nothing is written when there are more
+    SearchOutputs out;
+};
+
+/// Number `turn` of the tiles that a workgroup takes (n_tiles or beyond: none): every XCD walks a contiguous range of
+/// tiles, so that its L2 sees the same cells again and again (workgroups are dealt to the XCDs round-robin).
+__device__ __forceinline__ uint32_t crowded_tile(uint32_t turn, uint32_t n_tiles) {
+    const uint32_t per_xcd = (n_tiles + N_XCD - 1) / N_XCD;
+    const uint32_t within = blockIdx.x / N_XCD + turn * (gridDim.x / N_XCD);
+    const uint32_t tile = (blockIdx.x % N_XCD) * per_xcd + within;
+    return within < per_xcd && tile < n_tiles ? tile : 0xFFFFFFFFu;
+}
+
+__device__ __forceinline__ uint32_t crowded_first_tile(const CrowdedArgs& args, const Tile& tile) {
+    return static_cast<uint32_t>(args.cell_scan[tile.cell] >> 32);
+}
+
+__device__ __forceinline__ uint32_t fill_crowded_tables(
+    SearchTables& sh, int lane, uint32_t cell, const GridParams& g, const uint64_t* __restrict__ cell_scan
+) {
+    const int32_t span_y = 2 * g.s[1] + 1;
+    const int32_t span_z = 2 * g.s[2] + 1;
+    const uint32_t n_stencil = static_cast<uint32_t>(2 * g.s[0] + 1) * span_y * span_z; // (at most MAX_ENTRIES: the host)
+    fill_stencil_tables(
+        sh, lane, 0, n_stencil, static_cast<int32_t>(cell % g.n[0]), static_cast<int32_t>((cell / g.n[0]) % g.n[1]),
+        static_cast<int32_t>(cell / (g.n[0] * g.n[1])), span_y, span_z, g, cell_scan
+    );
+    return n_stencil;
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// MEASURE: one thread per tile, of which the first of every cell counts. The threads of a workgroup take room together:
+// one atomic each on the running total, which all compute dies share, took 1.5 ms for 44,000 cells.
+
+__global__ __launch_bounds__(CROWDED_BLOCK) void crowded_measure_kernel(CrowdedArgs args, GridParams g) {
+    __shared__ unsigned long long wave_total[CROWDED_WAVES];
+    __shared__ unsigned long long taken;
+    const int lane = lane_id();
+    const uint32_t wave = uniform(threadIdx.x / WAVE);
+    const uint32_t n_tiles = static_cast<uint32_t>(args.cell_scan[g.n_cells] >> 32);
+    for (uint32_t t0 = blockIdx.x * CROWDED_BLOCK; t0 < n_tiles; t0 += gridDim.x * CROWDED_BLOCK) {
+        const uint32_t t = t0 + threadIdx.x;
+        uint32_t n = 0;
+        uint32_t tiles_here = 0;
+        if (t < n_tiles) {
+            const uint32_t cell = args.tiles[t].cell;
+            if (static_cast<uint32_t>(args.cell_scan[cell] >> 32) == t) {
+                tiles_here = static_cast<uint32_t>(args.cell_scan[cell + 1] >> 32) - t;
+                const int32_t cx = static_cast<int32_t>(cell % g.n[0]);
+                const int32_t cy = static_cast<int32_t>((cell / g.n[0]) % g.n[1]);
+                const int32_t cz = static_cast<int32_t>(cell / (g.n[0] * g.n[1]));
+                for (int32_t dx = -g.s[0]; dx <= g.s[0]; dx++) {
+                    for (int32_t dy = -g.s[1]; dy <= g.s[1]; dy++) {
+                        for (int32_t dz = -g.s[2]; dz <= g.s[2]; dz++) {
+                            uint32_t neighbour;
+                            int32_t q[3];
+                            if (stencil_neighbour(g, cx, cy, cz, dx, dy, dz, neighbour, q)) {
+                                n += static_cast<uint32_t>(args.cell_scan[neighbour + 1]) -
+                                     static_cast<uint32_t>(args.cell_scan[neighbour]);
+                            }
+                        }
+                    }
+                }
+            }
+        }
+        const uint32_t n_units = n > CROWDED_LARGE ? 0u : (n + WAVE - 1) / WAVE;
+        const unsigned long long wanted =
+            static_cast<unsigned long long>(n_units) | (static_cast<unsigned long long>(n_units) * tiles_here << 32);
+        const unsigned long long through = wave_inclusive_scan(static_cast<uint64_t>(wanted));
+        __syncthreads(); // (the round before has read the totals)
+        if (lane == WAVE - 1) {
+            wave_total[wave] = through;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            unsigned long long all = 0;
+            for (int w = 0; w < CROWDED_WAVES; w++) {
+                all += wave_total[w];
+            }
+            taken = all != 0 ? atomicAdd(&args.status->used, all) : 0;
+        }
+        __syncthreads();
+        unsigned long long mine = taken + through - wanted;
+        for (uint32_t w = 0; w < wave; w++) {
+            mine += wave_total[w];
+        }
+        if (tiles_here != 0) {
+            CrowdedCell cell = {n, static_cast<uint32_t>(mine), static_cast<uint32_t>(mine >> 32), 0u};
+            if (n > CROWDED_LARGE) {
+                cell.candidates = 0;
+            } else if (static_cast<uint64_t>(cell.first_candidate) + n_units > args.candidate_units ||
+                       static_cast<uint64_t>(cell.first_column) + static_cast<uint64_t>(n_units) * tiles_here > args.column_units) {
+                cell.candidates = 0;
+                args.status->overflow = 1u;
+            }
+            args.cells[t] = cell;
+        }
+        uint32_t most = n;
+#pragma unroll
+        for (int offset = 32; offset > 0; offset >>= 1) {
+            most = max(most, static_cast<uint32_t>(__shfl_xor(static_cast<int>(most), offset, WAVE)));
+        }
+        if (lane == 0 && most > __atomic_load_n(&args.status->max_candidates, __ATOMIC_RELAXED)) {
+            atomicMax(&args.status->max_candidates, most);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// SORT: bound by LDS latency and atomics. Buckets of about two candidates' indices, so that a key meets few others; the
+// kernel for most cells and the one for the most crowded are apart because the latter's LDS leaves room for one workgroup
+// per compute unit (clusters of 500,000 points: 209 + 119 us).
+
+template <uint32_t CAPACITY, int THREADS>
+struct CrowdedSortShared {
+    static constexpr uint32_t BUCKETS = CAPACITY / 2;
+    SearchTables tables;
+    uint32_t index[CAPACITY];  // grouped by bucket
+    uint32_t at[CAPACITY];
+    uint32_t biased[CAPACITY];
+    uint32_t first[BUCKETS + 1]; // candidates per bucket, then the first of every bucket
+    uint32_t lowest, highest;
+    uint32_t wave_total[THREADS / WAVE];
+};
+
+/// Cells of more than `MORE_THAN` and at most `CAPACITY` candidates.
+template <uint32_t MORE_THAN, uint32_t CAPACITY, int THREADS>
+__global__ __launch_bounds__(THREADS) void crowded_sort_kernel(CrowdedArgs args, GridParams g) {
+    using Shared = CrowdedSortShared<CAPACITY, THREADS>;
+    constexpr uint32_t OWN = CAPACITY / THREADS; // candidates of a thread
+    constexpr uint32_t BUCKETS = Shared::BUCKETS;
+    constexpr uint32_t OWN_BUCKETS = BUCKETS / THREADS;
+    static_assert(OWN * THREADS == CAPACITY && OWN_BUCKETS * THREADS == BUCKETS, "the threads share everything evenly");
+    __shared__ Shared sh;
+    const int lane = lane_id();
+    const uint32_t wave = uniform(threadIdx.x / WAVE);
+    const uint32_t n_tiles = static_cast<uint32_t>(args.cell_scan[g.n_cells] >> 32);
+    if (CAPACITY == CROWDED_LARGE && args.status->max_candidates <= MORE_THAN) {
+        return;
+    }
+    for (uint32_t turn = 0;; turn++) {
+        if (turn * (gridDim.x / N_XCD) + blockIdx.x / N_XCD >= (n_tiles + N_XCD - 1) / N_XCD) {
+            return;
+        }
+        const uint32_t t = crowded_tile(turn, n_tiles);
+        if (t == 0xFFFFFFFFu) {
+            continue;
+        }
+        const Tile tile = args.tiles[t];
+        if (crowded_first_tile(args, tile) != t) {
+            continue;
+        }
+        const CrowdedCell cell = args.cells[t];
+        const uint32_t n = uniform(cell.candidates);
+        if (n == 0 || n <= MORE_THAN || n > CAPACITY) {
+            continue;
+        }
+        __syncthreads(); // (the cell before is done with the LDS)
+        const uint32_t n_stencil = static_cast<uint32_t>(2 * g.s[0] + 1) * (2 * g.s[1] + 1) * (2 * g.s[2] + 1);
+        if (wave == 0) {
+            (void)fill_crowded_tables(sh.tables, lane, tile.cell, g, args.cell_scan);
+        }
+        if (threadIdx.x == 0) {
+            sh.lowest = 0xFFFFFFFFu;
+            sh.highest = 0;
+        }
+        for (uint32_t b = threadIdx.x; b <= BUCKETS; b += THREADS) {
+            sh.first[b] = 0;
+        }
+        __syncthreads();
+
+        uint32_t index[OWN], at[OWN], biased[OWN];
+        uint32_t lowest = 0xFFFFFFFFu;
+        uint32_t highest = 0;
+        bool out_of_range = false;
+#pragma unroll
+        for (uint32_t u = 0; u < OWN; u++) {
+            const uint32_t k = u * THREADS + threadIdx.x;
+            index[u] = at[u] = biased[u] = 0;
+            if (k < n) {
+                int32_t packed;
+                locate_candidate(sh.tables, n_stencil, k, at[u], packed);
+                int32_t qx, qy, qz;
+                unpack_shift(packed, qx, qy, qz);
+                index[u] = args.sorted.p[at[u]].index;
+                qx -= args.sorted.wx[at[u]];
+                qy -= args.sorted.wy[at[u]];
+                qz -= args.sorted.wz[at[u]];
+                biased[u] = biased_shift(qx, qy, qz);
+                out_of_range = out_of_range || beyond(qx, qy, qz, ORDERED_SHIFT_LIMIT);
+                lowest = min(lowest, index[u]);
+                highest = max(highest, index[u]);
+            }
+        }
+        if (__ballot(out_of_range) != 0 && lane == 0) {
+            atomicOr(&args.status->unsuitable, 1u);
+        }
+#pragma unroll
+        for (int offset = 32; offset > 0; offset >>= 1) {
+            lowest = min(lowest, static_cast<uint32_t>(__shfl_xor(static_cast<int>(lowest), offset, WAVE)));
+            highest = max(highest, static_cast<uint32_t>(__shfl_xor(static_cast<int>(highest), offset, WAVE)));
+        }
+        if (lane == 0) {
+            atomicMin(&sh.lowest, lowest);
+            atomicMax(&sh.highest, highest);
+        }
+        __syncthreads();
+        lowest = uniform(sh.lowest);
+        highest = uniform(sh.highest);
+        // monotonic in the index: products of exact and rounded numbers with one factor, rounded again
+        const float per_index = static_cast<float>(BUCKETS) / (static_cast<float>(highest - lowest) + 1.0f);
+        auto bucket_of = [&](uint32_t i) {
+            return min(BUCKETS - 1, static_cast<uint32_t>(static_cast<float>(i - lowest) * per_index));
+        };
+        uint32_t arrival[OWN];
+#pragma unroll
+        for (uint32_t u = 0; u < OWN; u++) {
+            const uint32_t k = u * THREADS + threadIdx.x;
+            arrival[u] = k < n ? atomicAdd(&sh.first[bucket_of(index[u])], 1u) : 0u;
+        }
+        __syncthreads();
+        uint32_t in_bucket[OWN_BUCKETS];
+        uint32_t mine = 0;
+#pragma unroll
+        for (uint32_t b = 0; b < OWN_BUCKETS; b++) {
+            in_bucket[b] = sh.first[OWN_BUCKETS * threadIdx.x + b];
+            mine += in_bucket[b];
+        }
+        const uint32_t through = wave_inclusive_scan(mine);
+        if (lane == WAVE - 1) {
+            sh.wave_total[wave] = through;
+        }
+        __syncthreads();
+        uint32_t before = through - mine;
+        for (uint32_t w = 0; w < wave; w++) {
+            before += sh.wave_total[w];
+        }
+#pragma unroll
+        for (uint32_t b = 0; b < OWN_BUCKETS; b++) {
+            sh.first[OWN_BUCKETS * threadIdx.x + b] = before;
+            before += in_bucket[b];
+        }
+        if (threadIdx.x == THREADS - 1) {
+            sh.first[BUCKETS] = before; // = n
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t u = 0; u < OWN; u++) {
+            const uint32_t k = u * THREADS + threadIdx.x;
+            if (k < n) {
+                const uint32_t slot = sh.first[bucket_of(index[u])] + arrival[u];
+                sh.index[slot] = index[u];
+                sh.at[slot] = at[u];
+                sh.biased[slot] = biased[u];
+            }
+        }
+        __syncthreads();
+        CrowdedCandidate* target = args.candidates + static_cast<size_t>(cell.first_candidate) * WAVE;
+        for (uint32_t slot = threadIdx.x; slot < n; slot += THREADS) {
+            const uint32_t own = sh.index[slot];
+            const uint32_t own_biased = sh.biased[slot];
+            const uint32_t bucket = bucket_of(own);
+            const uint32_t end = sh.first[bucket + 1];
+            uint32_t place = sh.first[bucket];
+            for (uint32_t other = sh.first[bucket]; other < end; other++) {
+                const uint32_t theirs = sh.index[other];
+                // (the images of one point differ in their shifts)
+                place += theirs < own || (theirs == own && sh.biased[other] < own_biased) ? 1u : 0u;
+            }
+            target[place] = CrowdedCandidate{sh.at[slot], own_biased};
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// COUNT: bound by the fp64 distance tests (clusters of 500,000 points, 282 us). The candidates of a tile are dealt to four
+// waves, pairs of units in turn: the most crowded tiles would otherwise run long after all others are done.
+
+struct CrowdedCountShared {
+    uint32_t tile_index[TILE_POINTS];
+    double tile_x[TILE_POINTS], tile_y[TILE_POINTS], tile_z[TILE_POINTS];
+    int32_t tile_wx[TILE_POINTS], tile_wy[TILE_POINTS], tile_wz[TILE_POINTS];
+    uint32_t rows[TILE_POINTS];
+};
+
+template <bool FULL>
+__global__ __launch_bounds__(CROWDED_BLOCK) void crowded_count_kernel(CrowdedArgs args, GridParams g) {
+    constexpr int R = ORDERED_R;
+    __shared__ CrowdedCountShared sh;
+    const int lane = lane_id();
+    const uint32_t wave = uniform(threadIdx.x / WAVE);
+    const uint32_t n_tiles = static_cast<uint32_t>(args.cell_scan[g.n_cells] >> 32);
+    for (uint32_t turn = 0;; turn++) {
+        if (turn * (gridDim.x / N_XCD) + blockIdx.x / N_XCD >= (n_tiles + N_XCD - 1) / N_XCD) {
+            return;
+        }
+        const uint32_t t = crowded_tile(turn, n_tiles);
+        if (t == 0xFFFFFFFFu) {
+            continue;
+        }
+        const Tile tile = args.tiles[t];
+        const uint32_t first_tile = crowded_first_tile(args, tile);
+        const CrowdedCell cell = args.cells[first_tile];
+        const uint32_t n = uniform(cell.candidates);
+        const uint32_t n_i = tile.count;
+        const uint32_t n_units = (n + WAVE - 1) / WAVE;
+        const bool tile_wrapped = (tile.wrapped & 1u) != 0;
+        __syncthreads(); // (the tile before is done with the LDS)
+        bool out_of_range = false;
+        if (threadIdx.x < n_i) {
+            const uint32_t at = tile.first + threadIdx.x;
+            const SortedPoint point = args.sorted.p[at];
+            sh.tile_index[threadIdx.x] = point.index;
+            sh.tile_x[threadIdx.x] = point.x;
+            sh.tile_y[threadIdx.x] = point.y;
+            sh.tile_z[threadIdx.x] = point.z;
+            const int32_t wx = args.sorted.wx[at];
+            const int32_t wy = args.sorted.wy[at];
+            const int32_t wz = args.sorted.wz[at];
+            sh.tile_wx[threadIdx.x] = wx;
+            sh.tile_wy[threadIdx.x] = wy;
+            sh.tile_wz[threadIdx.x] = wz;
+            out_of_range = beyond(wx, wy, wz, ORDERED_SHIFT_LIMIT);
+            sh.rows[threadIdx.x] = 0;
+        }
+        if (__ballot(out_of_range) != 0 && lane == 0) {
+            atomicOr(&args.status->unsuitable, 1u);
+        }
+        __syncthreads();
+
+        const CrowdedCandidate* candidates = args.candidates + static_cast<size_t>(cell.first_candidate) * WAVE;
+        uint32_t* columns = args.columns + (static_cast<size_t>(cell.first_column) + static_cast<size_t>(t - first_tile) * n_units) * WAVE;
+        uint32_t own_rows = 0;
+        for (uint32_t unit0 = wave * R; unit0 < n_units; unit0 += CROWDED_WAVES * R) {
+            SweepCandidates<R> c;
+            uint32_t original[R], column[R];
+            int32_t bx[R], by[R], bz[R];
+            bool any_shift = false;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const uint32_t k = (unit0 + r) * WAVE + lane;
+                c.x[r] = c.y[r] = c.z[r] = __builtin_nan("");
+                c.tx[r] = c.ty[r] = c.tz[r] = 0.0;
+                c.shift[r] = 0;
+                c.position[r] = 0xFFFFFFFFu;
+                column[r] = 0;
+                original[r] = 0xFFFFFFFFu;
+                bx[r] = by[r] = bz[r] = 0;
+                if (k < n) {
+                    const CrowdedCandidate candidate = candidates[k];
+                    const SortedPoint point = args.sorted.p[candidate.at];
+                    c.x[r] = point.x;
+                    c.y[r] = point.y;
+                    c.z[r] = point.z;
+                    original[r] = point.index;
+                    bx[r] = static_cast<int32_t>((candidate.biased >> 20) & 0x3ffu) - 512;
+                    by[r] = static_cast<int32_t>((candidate.biased >> 10) & 0x3ffu) - 512;
+                    bz[r] = static_cast<int32_t>(candidate.biased & 0x3ffu) - 512;
+                    // a point is no neighbour of itself; a half list keeps a point with its own image under the rule of
+                    // the reference (in a tile without wrapped points the shift of such a pair is the cell shift)
+                    const bool never_with_itself =
+                        (bx[r] | by[r] | bz[r]) == 0 || (!FULL && !half_keeps_self_image(bx[r], by[r], bz[r]));
+                    c.position[r] = never_with_itself ? candidate.at : 0xFFFFFFFFu;
+                }
+                any_shift = any_shift || __ballot((bx[r] | by[r] | bz[r]) != 0) != 0;
+            }
+            if (!tile_wrapped) {
+                if (any_shift) {
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        shift_vector(g, bx[r], by[r], bz[r], c.tx[r], c.ty[r], c.tz[r]);
+                    }
+                    sweep_and_count<R, true, FULL>(sh, tile.first, n_i, c, g.cutoff2, original, lane, column, own_rows);
+                } else {
+                    sweep_and_count<R, false, FULL>(sh, tile.first, n_i, c, g.cutoff2, original, lane, column, own_rows);
+                }
+            } else {
+                // some points of the tile were moved into the box: the shift differs from point to point
+                for (uint32_t p = 0; p < n_i; p++) {
+                    const double xi = sh.tile_x[p];
+                    const double yi = sh.tile_y[p];
+                    const double zi = sh.tile_z[p];
+                    const uint32_t index_i = sh.tile_index[p];
+                    uint32_t found = 0;
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        const int32_t sx = bx[r] + sh.tile_wx[p];
+                        const int32_t sy = by[r] + sh.tile_wy[p];
+                        const int32_t sz = bz[r] + sh.tile_wz[p];
+                        double tx, ty, tz;
+                        shift_vector(g, sx, sy, sz, tx, ty, tz);
+                        const double vx = (c.x[r] - xi) + tx;
+                        const double vy = (c.y[r] - yi) + ty;
+                        const double vz = (c.z[r] - zi) + tz;
+                        const double d2 = vx * vx + vy * vy + vz * vz;
+                        const bool itself = index_i == original[r];
+                        bool keep = d2 < g.cutoff2 && !(itself && (sx | sy | sz) == 0);
+                        if (!FULL) {
+                            keep = keep && (index_i < original[r] || (itself && half_keeps_self_image(sx, sy, sz)));
+                        }
+                        const uint64_t mask = __ballot(keep);
+                        found += __popcll(mask);
+                        column[r] = shift_in(column[r], mask);
+                    }
+                    if (static_cast<uint32_t>(lane) == p) {
+                        own_rows += found;
+                    }
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                if (unit0 + r < n_units) {
+                    columns[(unit0 + r) * WAVE + lane] = column[r];
+                }
+            }
+        }
+        if (static_cast<uint32_t>(lane) < n_i && own_rows != 0) {
+            atomicAdd(&sh.rows[lane], own_rows);
+        }
+        __syncthreads();
+        if (threadIdx.x < n_i) {
+            args.rows_of_point[sh.tile_index[threadIdx.x]] = sh.rows[threadIdx.x];
+        }
+    }
+}
+
+__global__ void publish_crowded_status(
+    const CrowdedStatus* found, const uint64_t* total, const DeviceStatus* status, const uint64_t* cell_scan_end,
+    CrowdedHostStatus* host
+) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) {
+        host->found = *found;
+        host->total_rows = total != nullptr ? *total : 0;
+        host->first_bad_coordinate = status->first_bad_coordinate;
+        host->n_tiles = static_cast<unsigned int>(*cell_scan_end >> 32);
+    }
+}
+
+__global__ void clear_crowded_status(CrowdedStatus* status) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) {
+        *status = CrowdedStatus{};
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// WRITE
+
+struct CrowdedWriteShared {
+    // the chunk's candidates
+    double x[CROWDED_CHUNK], y[CROWDED_CHUNK], z[CROWDED_CHUNK];
+    uint32_t index[CROWDED_CHUNK];
+    uint32_t biased[CROWDED_CHUNK];
+    uint32_t column[CROWDED_CHUNK];
+    // the vectors of 64 consecutive rows on their way to memory (store_vector_block), per wave
+    __attribute__((aligned(16))) double vector_stage[CROWDED_WAVES][3 * WAVE];
+    // rows lined up: (number of the first point in the tile << 16) | number of the candidate in the chunk
+    uint32_t staged[CROWDED_WAVES][CROWDED_STAGED];
+    double tile_x[TILE_POINTS], tile_y[TILE_POINTS], tile_z[TILE_POINTS];
+    uint64_t tile_row[TILE_POINTS];  // first output row of each point that is not written yet
+    uint32_t tile_index[TILE_POINTS];
+    uint32_t tile_wrap[TILE_POINTS]; // the three wraps in the fields of the key
+    uint32_t by_index[TILE_POINTS];  // the tile's points in the order of their original indices
+};
+
+/// Stores the first `count` rows lined up by this wave as the rows `first_row` ... of the list: 64 consecutive rows per
+/// step, each step ending on a multiple of 64 rows (whole cache lines in every output array).
+__device__ __forceinline__ void store_crowded_rows(
+    CrowdedWriteShared& sh, uint32_t wave, const GridParams& g, const SearchOutputs& out, uint32_t count, uint64_t first_row,
+    int lane
+) {
+    const uint32_t skew = static_cast<uint32_t>(first_row % WAVE);
+    for (uint32_t e0 = 0; e0 < count + skew; e0 += WAVE) {
+        const uint32_t e = e0 + lane - skew;
+        const bool active = e < count; // (not before the first row either: unsigned)
+        const uint32_t entry = sh.staged[wave][active ? e : 0];
+        const uint32_t point = entry >> 16;
+        const uint32_t candidate = entry & 0xffffu;
+        const uint32_t biased = sh.biased[candidate] + sh.tile_wrap[point];
+        const int32_t sx = static_cast<int32_t>((biased >> 20) & 0x3ffu) - 512;
+        const int32_t sy = static_cast<int32_t>((biased >> 10) & 0x3ffu) - 512;
+        const int32_t sz = static_cast<int32_t>(biased & 0x3ffu) - 512;
+        double tx, ty, tz;
+        shift_vector(g, sx, sy, sz, tx, ty, tz);
+        const double vx = (sh.x[candidate] - sh.tile_x[point]) + tx;
+        const double vy = (sh.y[candidate] - sh.tile_y[point]) + ty;
+        const double vz = (sh.z[candidate] - sh.tile_z[point]) + tz;
+        const uint64_t row = first_row + e;
+        if (active) {
+            stream_store(out.pairs + 2 * row, PairRow{sh.tile_index[point], sh.index[candidate]});
+            if (out.shifts != nullptr) {
+                stream_store(out.shifts + 3 * row, ShiftRow{sx, sy, sz});
+            }
+            if (out.distances != nullptr) {
+                stream_store(out.distances + row, sqrt(vx * vx + vy * vy + vz * vz));
+            }
+        }
+        if (out.vectors != nullptr) {
+            const uint32_t lo = e0 == 0 ? skew : 0;
+            const uint32_t hi = min(count + skew - e0, static_cast<uint32_t>(WAVE));
+            store_vector_block(
+                sh.vector_stage[wave], reinterpret_cast<char*>(out.vectors + 3 * (first_row - skew + e0)), lo, hi, active,
+                static_cast<uint32_t>(lane), vx, vy, vz
+            );
+        }
+    }
+}
+
+__global__ __launch_bounds__(CROWDED_BLOCK) void crowded_write_kernel(CrowdedArgs args, GridParams g) {
+    __shared__ CrowdedWriteShared sh;
+    const int lane = lane_id();
+    const uint32_t wave = uniform(threadIdx.x / WAVE);
+    const CrowdedStatus found = *args.status;
+    if (found.overflow != 0 || found.unsuitable != 0 || found.max_candidates > CROWDED_LARGE ||
+        args.first_row[g.n_points] > args.capacity) {
+        return;
+    }
+    const uint32_t n_tiles = static_cast<uint32_t>(args.cell_scan[g.n_cells] >> 32);
+    for (uint32_t turn = 0;; turn++) {
+        if (turn * (gridDim.x / N_XCD) + blockIdx.x / N_XCD >= (n_tiles + N_XCD - 1) / N_XCD) {
+            return;
+        }
+        const uint32_t t = crowded_tile(turn, n_tiles);
+        if (t == 0xFFFFFFFFu) {
+            continue;
+        }
+        const Tile tile = args.tiles[t];
+        const uint32_t first_tile = crowded_first_tile(args, tile);
+        const CrowdedCell cell = args.cells[first_tile];
+        const uint32_t n = uniform(cell.candidates);
+        const uint32_t n_i = uniform(tile.count);
+        const uint32_t n_units = (n + WAVE - 1) / WAVE;
+        __syncthreads(); // (the tile before is done with the LDS)
+        if (threadIdx.x < n_i) {
+            const uint32_t at = tile.first + threadIdx.x;
+            const SortedPoint point = args.sorted.p[at];
+            sh.tile_index[threadIdx.x] = point.index;
+            sh.tile_x[threadIdx.x] = point.x;
+            sh.tile_y[threadIdx.x] = point.y;
+            sh.tile_z[threadIdx.x] = point.z;
+            // every field of biased shift and wrap together stays inside its ten bits (operands within +-255)
+            sh.tile_wrap[threadIdx.x] = (static_cast<uint32_t>(args.sorted.wx[at]) << 20) +
+                                        (static_cast<uint32_t>(args.sorted.wy[at]) << 10) +
+                                        static_cast<uint32_t>(args.sorted.wz[at]);
+            sh.tile_row[threadIdx.x] = args.first_row[point.index];
+        }
+        __syncthreads();
+        if (threadIdx.x < n_i) {
+            const uint32_t own = sh.tile_index[threadIdx.x];
+            uint32_t smaller = 0;
+            for (uint32_t other = 0; other < n_i; other++) {
+                smaller += sh.tile_index[other] < own ? 1u : 0u;
+            }
+            sh.by_index[smaller] = threadIdx.x;
+        }
+        const CrowdedCandidate* candidates = args.candidates + static_cast<size_t>(cell.first_candidate) * WAVE;
+        const uint32_t* columns =
+            args.columns + (static_cast<size_t>(cell.first_column) + static_cast<size_t>(t - first_tile) * n_units) * WAVE;
+        // this wave's share of the points
+        const uint32_t per_wave = (n_i + CROWDED_WAVES - 1) / CROWDED_WAVES;
+        const uint32_t turn_begin = wave * per_wave;
+        const uint32_t turn_end = min(n_i, turn_begin + per_wave);
+
+        for (uint32_t first = 0; first < n; first += CROWDED_CHUNK) {
+            const uint32_t in_chunk = min(n - first, CROWDED_CHUNK);
+            const uint32_t units_here = (in_chunk + WAVE - 1) / WAVE;
+            if (first != 0) {
+                __syncthreads();
+            }
+            for (uint32_t k = threadIdx.x; k < units_here * WAVE; k += CROWDED_BLOCK) {
+                uint32_t column = 0;
+                if (k < in_chunk) {
+                    column = columns[first + k];
+                    const CrowdedCandidate candidate = candidates[first + k];
+                    const SortedPoint point = args.sorted.p[candidate.at];
+                    sh.x[k] = point.x;
+                    sh.y[k] = point.y;
+                    sh.z[k] = point.z;
+                    sh.index[k] = point.index;
+                    sh.biased[k] = candidate.biased;
+                }
+                sh.column[k] = column;
+            }
+            __syncthreads();
+            uint32_t staged = 0;
+            uint64_t staged_row = 0; // row of the first one lined up
+            for (uint32_t at = turn_begin; at < turn_end; at++) {
+                const uint32_t p = uniform(sh.by_index[at]);
+                const uint64_t row_p = uniform(sh.tile_row[p]);
+                // (the rows of points with consecutive indices are consecutive rows of the list, as long as the
+                // candidates of the cell come in one chunk)
+                if (staged != 0 && row_p != staged_row + staged) {
+                    store_crowded_rows(sh, wave, g, args.out, staged, staged_row, lane);
+                    staged = 0;
+                    wave_sync();
+                }
+                if (staged == 0) {
+                    staged_row = row_p;
+                }
+                const uint32_t bit = n_i - 1 - p;
+                uint32_t rows_here = 0;
+                for (uint32_t unit0 = 0; unit0 < units_here; unit0 += CROWDED_STEP) {
+#pragma unroll
+                    for (uint32_t u = 0; u < CROWDED_STEP; u++) {
+                        const uint32_t k = (unit0 + u) * WAVE + lane;
+                        const bool hit = unit0 + u < units_here && ((sh.column[min(k, CROWDED_CHUNK - 1)] >> bit) & 1u) != 0;
+                        const uint64_t mask = __ballot(hit);
+                        if (hit) {
+                            sh.staged[wave][staged + rank_in_mask(mask)] = (p << 16) | k;
+                        }
+                        const uint32_t hits = __popcll(mask);
+                        staged += hits;
+                        rows_here += hits;
+                    }
+                    const uint64_t whole = (staged_row + staged) & ~static_cast<uint64_t>(WAVE - 1);
+                    if (whole > staged_row) {
+                        // everything up to the last multiple of 64 rows; what is left moves to the front
+                        wave_sync();
+                        const uint32_t count = static_cast<uint32_t>(whole - staged_row);
+                        store_crowded_rows(sh, wave, g, args.out, count, staged_row, lane);
+                        const uint32_t left = staged - count; // < 64
+                        const uint32_t entry = sh.staged[wave][min(count + lane, CROWDED_STAGED - 1)];
+                        wave_sync();
+                        if (static_cast<uint32_t>(lane) < left) {
+                            sh.staged[wave][lane] = entry;
+                        }
+                        staged_row = whole;
+                        staged = left;
+                        wave_sync();
+                    }
+                }
+                if (n > CROWDED_CHUNK) {
+                    wave_sync();
+                    if (lane == 0) {
+                        sh.tile_row[p] = row_p + rows_here;
+                    }
+                }
+            }
+            if (staged != 0) {
+                wave_sync();
+                store_crowded_rows(sh, wave, g, args.out, staged, staged_row, lane);
+                wave_sync();
+            }
+        }
+    }
+}
+
+} // namespace vesin_hip
+
+#endif

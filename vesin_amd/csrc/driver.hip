@@ -29,6 +29,7 @@
 #include <vector>
 
 #include "backward.cuh"
+#include "crowded.cuh"
 #include "cells.cuh"
 #include "device_common.cuh"
 #include "driver.hpp"
@@ -200,6 +201,13 @@ static bool radix_sort_only() {
     return text != nullptr && std::strcmp(text, "radix") == 0;
 }
 
+/// VESIN_HIP_SORT=crowded sends every sorted list of one system to the in-order search for crowded cells (for
+/// comparisons and tests).
+static bool crowded_search_only() {
+    const char* text = std::getenv("VESIN_HIP_SORT");
+    return text != nullptr && std::strcmp(text, "crowded") == 0;
+}
+
 /// VESIN_HIP_LAUNCHES=separate keeps the passes of a small system's search in launches of their own (for comparisons
 /// and tests) instead of one launch whose workgroups wait for each other between the passes.
 static bool separate_launches() {
@@ -270,6 +278,7 @@ struct Mailbox {
     // what only some do
     BlockBounds bounds[BOUNDING_BLOCKS]; // one slot per workgroup of the bounding pass
     ShiftRange ranges[SHIFT_RANGE_BLOCKS]; // one slot per workgroup of the sort's range pass
+    CrowdedHostStatus crowded;
 };
 
 /// Makes `device` current for a scope and gives the caller's device back afterwards.
@@ -845,6 +854,10 @@ struct HipExtras {
     int single_pass_rest = 0;         // calls left before the single-pass search is tried again after it did not fit
     int direct_rest = 0;              // calls left before the one-pass cell build is tried again after a cell overflowed
     int in_order_rest = 0;            // calls left before the in-order search is tried again on a system it did not cover
+    int crowded_rest = 0;             // the same for the in-order search for crowded cells (crowded.cuh)
+    size_t crowded_points = 0;        // the last system that search covered: its number of points ...
+    size_t crowded_candidate_units = 0; // ... and the room its candidates and hit columns took, in units of 64
+    size_t crowded_column_units = 0;
     int one_launch_rest = 0;          // calls left before a small system is tried in one launch again
     WaitRest meeting_rest;            // ... after workgroups of that launch gave up waiting for the others
     WaitRest chain_rest;              // the same for the chain of the single-pass search (rows in work-item order)
@@ -1713,6 +1726,15 @@ bool compute(
         extras.in_order_rest -= 1;
         try_in_order = false;
     }
+    if (crowded_search_only()) {
+        try_in_order = false;
+    }
+    // what that search does not cover goes to the one for crowded cells (which allocates its work memory on the way)
+    bool try_crowded = options.sorted && full_stencil <= MAX_ENTRIES && !radix_sort_only() && !extras.fixed_memory;
+    if (try_crowded && extras.crowded_rest > 0) {
+        extras.crowded_rest -= try_in_order ? 0 : 1;
+        try_crowded = false;
+    }
     // Small systems with arrays from earlier calls: everything in one launch (small.cuh), as one work item per point
     // for a sorted list, as one per point and slice of its candidates otherwise (about four units of 64 candidates
     // per item, as many items as the smallest shape of that launch takes).
@@ -1793,8 +1815,9 @@ bool compute(
     }
     const size_t scratch_elements = std::max(
         std::max(scan_scratch_elements(n_cells), scan_scratch_elements(n_slots)),
-        try_in_order ? scan_scratch_elements(n_points) : 0
+        try_in_order || try_crowded ? scan_scratch_elements(n_points) : 0
     );
+    CrowdedStatus* crowded_status = nullptr;
 
     auto carve = [&](Carver& carver) {
         // adjacent, so that one fill clears the histogram, the tiles' flags and the state of the single-pass search
@@ -1805,12 +1828,13 @@ bool compute(
         chain.bases = carver.take<uint64_t>(chain_groups);
         direct_wrapped = carver.take<uint32_t>(direct_slots);
         fused_status = carver.take<FusedStatus>(1);
+        crowded_status = carver.take<CrowdedStatus>(1);
         ordered_status = carver.take<OrderedStatus>(1);
         // (behind the state that every call clears: place_points wants them cleared too)
         sorted.wx = carver.take<int32_t>(sorted_slots + SORTED_PADDING);
         sorted.wy = carver.take<int32_t>(sorted_slots + SORTED_PADDING);
         sorted.wz = carver.take<int32_t>(sorted_slots + SORTED_PADDING);
-        if (try_in_order) {
+        if (try_in_order || try_crowded) {
             rows_of_point = carver.take<uint32_t>(n_points); // (cleared as well: its counting pass may add to it)
         }
 
@@ -1832,8 +1856,10 @@ bool compute(
         offsets = carver.take<uint64_t>(std::max(n_slots, direct_slots * n_slices) + 1);
         scan_scratch = carver.take<uint64_t>(scratch_elements);
         rows_of_item = carver.take<uint32_t>(small_items);
-        if (try_in_order) {
+        if (try_in_order || try_crowded) {
             first_row_of_point = carver.take<uint64_t>(n_points + 1);
+        }
+        if (try_in_order) {
             candidate_records = carver.take<CandidateRecord>(static_cast<size_t>(ordered_blocks) * ORDERED_WAVES * ORDERED_UNITS * WAVE);
             candidates_of_item = carver.take<uint32_t>(static_cast<size_t>(ordered_blocks) * ORDERED_WAVES);
             if (ordered_items_per_tile == 1) {
@@ -2411,9 +2437,151 @@ bool compute(
             }
             return true;
         }
-        // rows per point, candidates per tile or shifts beyond what that search handles: the general way below,
-        // and for a while without asking again
+        // rows per point, candidates per tile or shifts beyond what that search handles: the ways below, and for a
+        // while without asking again
         extras.in_order_rest = SINGLE_PASS_REST;
+        try_crowded = try_crowded && found.found.unsuitable == 0;
+    }
+
+    // ---- the same for crowded cells, and for systems whose cells are too many for records of a fixed size
+    if (try_crowded && n_points > 0) {
+        CrowdedArgs cargs = {};
+        cargs.sorted = sorted;
+        cargs.cell_scan = cell_scan;
+        cargs.tiles = tiles;
+        cargs.status = crowded_status;
+        cargs.rows_of_point = rows_of_point;
+        cargs.first_row = first_row_of_point;
+        // workgroups of the passes, a multiple of the XCDs: each goes through as many tiles as there are for it (the
+        // number of tiles, known on the device, may be far below its bound where most cells are empty)
+        const uint32_t tile_blocks = static_cast<uint32_t>(std::min<size_t>((tiles_bound + N_XCD - 1) / N_XCD * N_XCD, 16384));
+        const uint32_t measure_blocks = static_cast<uint32_t>(std::min<size_t>((tiles_bound + CROWDED_BLOCK - 1) / CROWDED_BLOCK, 4096));
+        // The room that candidates and hit columns take is what the call before on as many points found, and an eighth
+        // more; a first call (and one that finds too little room) has it counted first.
+        size_t candidate_units = extras.crowded_points == n_points ? extras.crowded_candidate_units : 0;
+        size_t column_units = extras.crowded_points == n_points ? extras.crowded_column_units : 0;
+        bool known = candidate_units > 0;
+        bool covered = false;
+        for (int attempt = 0; attempt < 3; attempt++) {
+            const size_t record_bytes = candidate_units * WAVE * sizeof(CrowdedCandidate) + column_units * WAVE * sizeof(uint32_t);
+            if (candidate_units > 0xFFFFFFF0ull || column_units > 0xFFFFFFF0ull || !ordered_records_fit(n_points, record_bytes)) {
+                break;
+            }
+            auto carve_crowded = [&](Carver& c) {
+                cargs.cells = c.take<CrowdedCell>(tiles_bound);
+                cargs.candidates = c.take<CrowdedCandidate>(candidate_units * WAVE);
+                cargs.columns = c.take<uint32_t>(column_units * WAVE);
+            };
+            Carver crowded_measure(nullptr);
+            carve_crowded(crowded_measure);
+            extras.sort_work.reserve(crowded_measure.used);
+            Carver crowded_carver(extras.sort_work.ptr);
+            carve_crowded(crowded_carver);
+            cargs.candidate_units = static_cast<uint32_t>(candidate_units);
+            cargs.column_units = static_cast<uint32_t>(column_units);
+            const bool early_write = known && extras.capacity > 0;
+            if (attempt > 0) {
+                hipLaunchKernelGGL(clear_crowded_status, dim3(1), dim3(1), 0, stream, crowded_status);
+            }
+            hipLaunchKernelGGL(crowded_measure_kernel, dim3(measure_blocks), dim3(CROWDED_BLOCK), 0, stream, cargs, g);
+            if (known) {
+                hipLaunchKernelGGL(
+                    (crowded_sort_kernel<0, CROWDED_SMALL, CROWDED_BLOCK>), dim3(tile_blocks), dim3(CROWDED_BLOCK), 0, stream, cargs, g
+                );
+                hipLaunchKernelGGL(
+                    (crowded_sort_kernel<CROWDED_SMALL, CROWDED_LARGE, CROWDED_SORT_BLOCK>), dim3(std::min(tile_blocks, 2048u)),
+                    dim3(CROWDED_SORT_BLOCK), 0, stream, cargs, g
+                );
+                auto count = options.full ? crowded_count_kernel<true> : crowded_count_kernel<false>;
+                hipLaunchKernelGGL(count, dim3(tile_blocks), dim3(CROWDED_BLOCK), 0, stream, cargs, g);
+                mark(T_COUNT);
+                exclusive_scan<SCAN_U32>(rows_of_point, n_points, first_row_of_point, scan_scratch, stream);
+                mark(T_SCAN);
+            }
+            hipLaunchKernelGGL(
+                publish_crowded_status, dim3(1), dim3(1), 0, stream, crowded_status,
+                known ? first_row_of_point + n_points : static_cast<const uint64_t*>(nullptr), extras.d_status, cell_scan + n_cells,
+                &extras.mail_device->crowded
+            );
+            // (as in the in-order search: into the arrays of earlier calls without waiting for the host; the launch
+            // checks on the device that nothing stands against it)
+            size_t early_capacity = 0;
+            if (early_write) {
+                size_outputs(neighbors, extras, 0, options);
+                early_capacity = extras.capacity;
+                cargs.out = outputs_of();
+                cargs.capacity = early_capacity;
+                mark(T_WRITE_BEGIN);
+                hipLaunchKernelGGL(crowded_write_kernel, dim3(tile_blocks), dim3(CROWDED_BLOCK), 0, stream, cargs, g);
+                mark(T_WRITE);
+            }
+            extras.wait(stream);
+            if (!box_was_right()) {
+                return false;
+            }
+            const CrowdedHostStatus found = extras.mail->crowded;
+            if (found.first_bad_coordinate != 0xFFFFFFFFu) {
+                non_finite_error(points, found.first_bad_coordinate);
+            }
+            const size_t candidate_units_found = static_cast<size_t>(found.found.used & 0xFFFFFFFFull);
+            const size_t column_units_found = static_cast<size_t>(found.found.used >> 32);
+            if (std::getenv("VESIN_HIP_DEBUG") != nullptr) {
+                std::fprintf(
+                    stderr, "crowded search: rows %llu, most candidates of a cell %u, unsuitable %u, %zu + %zu units of candidates and columns, room for %zu + %zu\n",
+                    found.total_rows, found.found.max_candidates, found.found.unsuitable, candidate_units_found, column_units_found,
+                    candidate_units, column_units
+                );
+            }
+            if (found.found.unsuitable != 0 || found.found.max_candidates > CROWDED_LARGE) {
+                break;
+            }
+            if (!known || found.found.overflow != 0) {
+                candidate_units = candidate_units_found + candidate_units_found / 8 + 64;
+                column_units = column_units_found + column_units_found / 8 + 64;
+                known = true;
+                continue;
+            }
+            extras.crowded_points = n_points;
+            extras.crowded_candidate_units = std::max(candidate_units, candidate_units_found + candidate_units_found / 8 + 64);
+            extras.crowded_column_units = std::max(column_units, column_units_found + column_units_found / 8 + 64);
+            const size_t total = found.total_rows;
+            check_pair_limit(total);
+            if (!(early_write && total <= early_capacity)) {
+                // first call of the list, or more rows than its arrays hold
+                size_outputs(neighbors, extras, total, options);
+                cargs.out = outputs_of();
+                cargs.capacity = extras.capacity;
+                mark(T_WRITE_BEGIN);
+                if (total > 0) {
+                    hipLaunchKernelGGL(crowded_write_kernel, dim3(tile_blocks), dim3(CROWDED_BLOCK), 0, stream, cargs, g);
+                }
+                mark(T_WRITE);
+                mark(T_SORT);
+                HIP_CHECK(hipStreamSynchronize(stream));
+            } else {
+                mark(T_SORT);
+                if (timed) {
+                    HIP_CHECK(hipStreamSynchronize(stream));
+                }
+            }
+            HIP_CHECK(hipGetLastError());
+            neighbors.length = total;
+            if (timed) {
+                extras.timings = {};
+                extras.timings.total = elapsed(T_START, T_SORT);
+                extras.timings.cell_build = elapsed(T_START, T_CELLS);
+                extras.timings.count = elapsed(T_CELLS, T_COUNT);
+                extras.timings.scan = elapsed(T_COUNT, T_SCAN);
+                extras.timings.write = elapsed(T_WRITE_BEGIN, T_WRITE);
+                extras.timings_valid = true;
+            }
+            covered = true;
+            break;
+        }
+        if (covered) {
+            return true;
+        }
+        extras.crowded_rest = SINGLE_PASS_REST;
     }
 
     // ---- pass 1: count

@@ -174,6 +174,50 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
+/// The cell (dx, dy, dz) away from cell (cx, cy, cz): its number and cell shift. False when there is none, or none that
+/// can hold a neighbour.
+__device__ __forceinline__ bool stencil_neighbour(
+    const GridParams& g, int32_t cx, int32_t cy, int32_t cz, int32_t dx, int32_t dy, int32_t dz, uint32_t& neighbour,
+    int32_t (&q)[3]
+) {
+    int32_t cell[3] = {cx + dx, cy + dy, cz + dz};
+    q[0] = q[1] = q[2] = 0;
+    bool valid = true;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const int32_t n = g.n[d];
+        if (g.periodic[d]) {
+            if (g.s[d] <= n) {
+                // the neighbour is at most one box away: no division needed
+                if (cell[d] < 0) {
+                    cell[d] += n;
+                    q[d] = -1;
+                } else if (cell[d] >= n) {
+                    cell[d] -= n;
+                    q[d] = 1;
+                }
+            } else {
+                int32_t quotient = cell[d] / n;
+                int32_t rest = cell[d] - quotient * n;
+                if (rest < 0) {
+                    rest += n;
+                    quotient -= 1;
+                }
+                q[d] = quotient;
+                cell[d] = rest;
+            }
+        } else if (cell[d] < 0 || cell[d] >= n) {
+            valid = false;
+        }
+    }
+    if (stencil_entry_too_far(g, dx, dy, dz)) {
+        // points lie inside their cells: no pair between these two cells is within the cutoff
+        valid = false;
+    }
+    neighbour = (static_cast<uint32_t>(cell[2]) * g.n[1] + cell[1]) * g.n[0] + cell[0];
+    return valid;
+}
+
 /// Stencil entries [first_linear, first_linear + n_batch) around cell (cx, cy, cz) go to the wave's LDS tables:
 /// neighbour cell start, packed cell shift, and the running number of candidates (scanned in place). Linear stencil
 /// offsets run dx major, dz minor. `cell_scan`: exclusive scan of the points per cell in the low 32 bits of its words.
@@ -198,45 +242,13 @@ __device__ __forceinline__ void fill_stencil_tables(
             dy = static_cast<int32_t>((linear / span_z) % span_y) - g.s[1];
             dx = static_cast<int32_t>(linear / (span_z * span_y)) - g.s[0];
         }
-        int32_t cell[3] = {cx + dx, cy + dy, cz + dz};
-        int32_t q[3] = {0, 0, 0};
-        bool valid = true;
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            const int32_t n = g.n[d];
-            if (g.periodic[d]) {
-                if (g.s[d] <= n) {
-                    // the neighbour is at most one box away: no division needed
-                    if (cell[d] < 0) {
-                        cell[d] += n;
-                        q[d] = -1;
-                    } else if (cell[d] >= n) {
-                        cell[d] -= n;
-                        q[d] = 1;
-                    }
-                } else {
-                    int32_t quotient = cell[d] / n;
-                    int32_t rest = cell[d] - quotient * n;
-                    if (rest < 0) {
-                        rest += n;
-                        quotient -= 1;
-                    }
-                    q[d] = quotient;
-                    cell[d] = rest;
-                }
-            } else if (cell[d] < 0 || cell[d] >= n) {
-                valid = false;
-            }
-        }
-        if (stencil_entry_too_far(g, dx, dy, dz)) {
-            // points lie inside their cells: no pair between these two cells is within the cutoff
-            valid = false;
-        }
+        uint32_t neighbour;
+        int32_t q[3];
+        const bool valid = stencil_neighbour(g, cx, cy, cz, dx, dy, dz, neighbour, q);
         uint32_t start = 0;
         uint32_t count = 0;
         int32_t packed = 0;
         if (valid) {
-            uint32_t neighbour = (static_cast<uint32_t>(cell[2]) * g.n[1] + cell[1]) * g.n[0] + cell[0];
             if (direct_capacity != 0) {
                 start = neighbour * direct_capacity;
                 count = min(direct_counts[neighbour], direct_capacity);
