@@ -13,13 +13,11 @@
 //   COUNT    one workgroup per tile, the candidates dealt to its four waves: hit columns in the order of the candidates,
 //            rows of every point;
 //   a scan over the points gives every point its first row;
-//   WRITE    one workgroup per tile, which brings CROWDED_CHUNK candidates at a time to LDS (coordinates, index, shift,
-//            hit column); its waves share the points. A wave walks the columns for a point, lines up the hits, and
-//            stores 64 consecutive rows at a time, which need nothing from memory but LDS.
+//   WRITE    one workgroup per tile: write_tile.cuh.
 // A point may have any number of rows; a cell at most CROWDED_LARGE candidates (their sort takes the LDS of a compute
 // unit then). Beyond that, and for shifts or wraps beyond +-255, the host falls back to the radix sort.
 //
-// Measured per call, radix sort -> this: 500,000 points in 50 clusters (82 M rows, P d) 12.7 -> 1.67 ms, (P S d D) 17.9 ->
+// Measured per call, radix sort -> this: 500,000 points in 50 clusters (82 M rows, P d) 12.7 -> 1.42 ms, (P S d D) 17.9 ->
 // 2.27 ms; 200,000 atoms of diamond, cutoff 6.5 (1480 candidates per tile, P S d) 6.04 -> 1.04 ms; 13,824 atoms, cutoff 5.5
 // 358 -> 167 us; a liquid of 20,000 points, cutoff 7, 649 -> 208 us; 2,000 points, cutoff 7, 180 -> 147 us. On systems that
 // the usual in-order search covers it is the slower one, its passes follow each other where that one sorts beside its
@@ -30,6 +28,7 @@
 #define VESIN_HIP_CROWDED_CUH
 
 #include "ordered.cuh"
+#include "write_tile.cuh"
 
 namespace vesin_hip {
 
@@ -38,9 +37,6 @@ constexpr int CROWDED_BLOCK = CROWDED_WAVES * WAVE;
 constexpr uint32_t CROWDED_SMALL = 2048;   // candidates that the usual sorting kernel takes (29 KB of LDS)
 constexpr uint32_t CROWDED_LARGE = 8192;   // and the one for the most crowded cells (103 KB)
 constexpr int CROWDED_SORT_BLOCK = 512;    // threads of the latter
-constexpr uint32_t CROWDED_CHUNK = 768;    // candidates that a workgroup of WRITE holds in LDS: four workgroups per unit
-constexpr uint32_t CROWDED_STEP = 4;       // units of candidates between two looks at how many rows are lined up
-constexpr uint32_t CROWDED_STAGED = (CROWDED_STEP + 1) * WAVE;
 
 /// A candidate, in the order of (original index, shift).
 struct CrowdedCandidate {
@@ -532,69 +528,10 @@ __global__ void clear_crowded_status(CrowdedStatus* status) {
 // ---------------------------------------------------------------------------------------------------------------
 // WRITE
 
-struct CrowdedWriteShared {
-    // the chunk's candidates
-    double x[CROWDED_CHUNK], y[CROWDED_CHUNK], z[CROWDED_CHUNK];
-    uint32_t index[CROWDED_CHUNK];
-    uint32_t biased[CROWDED_CHUNK];
-    uint32_t column[CROWDED_CHUNK];
-    // the vectors of 64 consecutive rows on their way to memory (store_vector_block), per wave
-    __attribute__((aligned(16))) double vector_stage[CROWDED_WAVES][3 * WAVE];
-    // rows lined up: (number of the first point in the tile << 16) | number of the candidate in the chunk
-    uint32_t staged[CROWDED_WAVES][CROWDED_STAGED];
-    double tile_x[TILE_POINTS], tile_y[TILE_POINTS], tile_z[TILE_POINTS];
-    uint64_t tile_row[TILE_POINTS];  // first output row of each point that is not written yet
-    uint32_t tile_index[TILE_POINTS];
-    uint32_t tile_wrap[TILE_POINTS]; // the three wraps in the fields of the key
-    uint32_t by_index[TILE_POINTS];  // the tile's points in the order of their original indices
-};
-
-/// Stores the first `count` rows lined up by this wave as the rows `first_row` ... of the list: 64 consecutive rows per
-/// step, each step ending on a multiple of 64 rows (whole cache lines in every output array).
-__device__ __forceinline__ void store_crowded_rows(
-    CrowdedWriteShared& sh, uint32_t wave, const GridParams& g, const SearchOutputs& out, uint32_t count, uint64_t first_row,
-    int lane
-) {
-    const uint32_t skew = static_cast<uint32_t>(first_row % WAVE);
-    for (uint32_t e0 = 0; e0 < count + skew; e0 += WAVE) {
-        const uint32_t e = e0 + lane - skew;
-        const bool active = e < count; // (not before the first row either: unsigned)
-        const uint32_t entry = sh.staged[wave][active ? e : 0];
-        const uint32_t point = entry >> 16;
-        const uint32_t candidate = entry & 0xffffu;
-        const uint32_t biased = sh.biased[candidate] + sh.tile_wrap[point];
-        const int32_t sx = static_cast<int32_t>((biased >> 20) & 0x3ffu) - 512;
-        const int32_t sy = static_cast<int32_t>((biased >> 10) & 0x3ffu) - 512;
-        const int32_t sz = static_cast<int32_t>(biased & 0x3ffu) - 512;
-        double tx, ty, tz;
-        shift_vector(g, sx, sy, sz, tx, ty, tz);
-        const double vx = (sh.x[candidate] - sh.tile_x[point]) + tx;
-        const double vy = (sh.y[candidate] - sh.tile_y[point]) + ty;
-        const double vz = (sh.z[candidate] - sh.tile_z[point]) + tz;
-        const uint64_t row = first_row + e;
-        if (active) {
-            stream_store(out.pairs + 2 * row, PairRow{sh.tile_index[point], sh.index[candidate]});
-            if (out.shifts != nullptr) {
-                stream_store(out.shifts + 3 * row, ShiftRow{sx, sy, sz});
-            }
-            if (out.distances != nullptr) {
-                stream_store(out.distances + row, sqrt(vx * vx + vy * vy + vz * vz));
-            }
-        }
-        if (out.vectors != nullptr) {
-            const uint32_t lo = e0 == 0 ? skew : 0;
-            const uint32_t hi = min(count + skew - e0, static_cast<uint32_t>(WAVE));
-            store_vector_block(
-                sh.vector_stage[wave], reinterpret_cast<char*>(out.vectors + 3 * (first_row - skew + e0)), lo, hi, active,
-                static_cast<uint32_t>(lane), vx, vy, vz
-            );
-        }
-    }
-}
-
-__global__ __launch_bounds__(CROWDED_BLOCK) void crowded_write_kernel(CrowdedArgs args, GridParams g) {
-    __shared__ CrowdedWriteShared sh;
-    const int lane = lane_id();
+template <bool STAGED>
+__global__ __launch_bounds__(TILE_BLOCK, STAGED ? 4 : 5) void crowded_write_kernel(CrowdedArgs args, GridParams g) {
+    __shared__ TileWriteShared<STAGED> sh;
+    const uint32_t lane = static_cast<uint32_t>(lane_id());
     const uint32_t wave = uniform(threadIdx.x / WAVE);
     const CrowdedStatus found = *args.status;
     if (found.overflow != 0 || found.unsuitable != 0 || found.max_candidates > CROWDED_LARGE ||
@@ -617,43 +554,18 @@ __global__ __launch_bounds__(CROWDED_BLOCK) void crowded_write_kernel(CrowdedArg
         const uint32_t n_i = uniform(tile.count);
         const uint32_t n_units = (n + WAVE - 1) / WAVE;
         __syncthreads(); // (the tile before is done with the LDS)
-        if (threadIdx.x < n_i) {
-            const uint32_t at = tile.first + threadIdx.x;
-            const SortedPoint point = args.sorted.p[at];
-            sh.tile_index[threadIdx.x] = point.index;
-            sh.tile_x[threadIdx.x] = point.x;
-            sh.tile_y[threadIdx.x] = point.y;
-            sh.tile_z[threadIdx.x] = point.z;
-            // every field of biased shift and wrap together stays inside its ten bits (operands within +-255)
-            sh.tile_wrap[threadIdx.x] = (static_cast<uint32_t>(args.sorted.wx[at]) << 20) +
-                                        (static_cast<uint32_t>(args.sorted.wy[at]) << 10) +
-                                        static_cast<uint32_t>(args.sorted.wz[at]);
-            sh.tile_row[threadIdx.x] = args.first_row[point.index];
-        }
-        __syncthreads();
-        if (threadIdx.x < n_i) {
-            const uint32_t own = sh.tile_index[threadIdx.x];
-            uint32_t smaller = 0;
-            for (uint32_t other = 0; other < n_i; other++) {
-                smaller += sh.tile_index[other] < own ? 1u : 0u;
-            }
-            sh.by_index[smaller] = threadIdx.x;
-        }
+        const bool moved = load_tile(sh, args.sorted, tile.first, n_i, args.first_row);
         const CrowdedCandidate* candidates = args.candidates + static_cast<size_t>(cell.first_candidate) * WAVE;
         const uint32_t* columns =
             args.columns + (static_cast<size_t>(cell.first_column) + static_cast<size_t>(t - first_tile) * n_units) * WAVE;
-        // this wave's share of the points
-        const uint32_t per_wave = (n_i + CROWDED_WAVES - 1) / CROWDED_WAVES;
-        const uint32_t turn_begin = wave * per_wave;
-        const uint32_t turn_end = min(n_i, turn_begin + per_wave);
-
-        for (uint32_t first = 0; first < n; first += CROWDED_CHUNK) {
-            const uint32_t in_chunk = min(n - first, CROWDED_CHUNK);
+        for (uint32_t first = 0; first < n; first += TILE_CHUNK) {
+            const uint32_t in_chunk = min(n - first, TILE_CHUNK);
             const uint32_t units_here = (in_chunk + WAVE - 1) / WAVE;
             if (first != 0) {
                 __syncthreads();
             }
-            for (uint32_t k = threadIdx.x; k < units_here * WAVE; k += CROWDED_BLOCK) {
+            bool shifted = moved;
+            for (uint32_t k = threadIdx.x; k < units_here * WAVE; k += TILE_BLOCK) {
                 uint32_t column = 0;
                 if (k < in_chunk) {
                     column = columns[first + k];
@@ -664,68 +576,14 @@ __global__ __launch_bounds__(CROWDED_BLOCK) void crowded_write_kernel(CrowdedArg
                     sh.z[k] = point.z;
                     sh.index[k] = point.index;
                     sh.biased[k] = candidate.biased;
+                    shifted = shifted || candidate.biased != NO_SHIFT;
                 }
                 sh.column[k] = column;
             }
-            __syncthreads();
-            uint32_t staged = 0;
-            uint64_t staged_row = 0; // row of the first one lined up
-            for (uint32_t at = turn_begin; at < turn_end; at++) {
-                const uint32_t p = uniform(sh.by_index[at]);
-                const uint64_t row_p = uniform(sh.tile_row[p]);
-                // (the rows of points with consecutive indices are consecutive rows of the list, as long as the
-                // candidates of the cell come in one chunk)
-                if (staged != 0 && row_p != staged_row + staged) {
-                    store_crowded_rows(sh, wave, g, args.out, staged, staged_row, lane);
-                    staged = 0;
-                    wave_sync();
-                }
-                if (staged == 0) {
-                    staged_row = row_p;
-                }
-                const uint32_t bit = n_i - 1 - p;
-                uint32_t rows_here = 0;
-                for (uint32_t unit0 = 0; unit0 < units_here; unit0 += CROWDED_STEP) {
-#pragma unroll
-                    for (uint32_t u = 0; u < CROWDED_STEP; u++) {
-                        const uint32_t k = (unit0 + u) * WAVE + lane;
-                        const bool hit = unit0 + u < units_here && ((sh.column[min(k, CROWDED_CHUNK - 1)] >> bit) & 1u) != 0;
-                        const uint64_t mask = __ballot(hit);
-                        if (hit) {
-                            sh.staged[wave][staged + rank_in_mask(mask)] = (p << 16) | k;
-                        }
-                        const uint32_t hits = __popcll(mask);
-                        staged += hits;
-                        rows_here += hits;
-                    }
-                    const uint64_t whole = (staged_row + staged) & ~static_cast<uint64_t>(WAVE - 1);
-                    if (whole > staged_row) {
-                        // everything up to the last multiple of 64 rows; what is left moves to the front
-                        wave_sync();
-                        const uint32_t count = static_cast<uint32_t>(whole - staged_row);
-                        store_crowded_rows(sh, wave, g, args.out, count, staged_row, lane);
-                        const uint32_t left = staged - count; // < 64
-                        const uint32_t entry = sh.staged[wave][min(count + lane, CROWDED_STAGED - 1)];
-                        wave_sync();
-                        if (static_cast<uint32_t>(lane) < left) {
-                            sh.staged[wave][lane] = entry;
-                        }
-                        staged_row = whole;
-                        staged = left;
-                        wave_sync();
-                    }
-                }
-                if (n > CROWDED_CHUNK) {
-                    wave_sync();
-                    if (lane == 0) {
-                        sh.tile_row[p] = row_p + rows_here;
-                    }
-                }
-            }
-            if (staged != 0) {
-                wave_sync();
-                store_crowded_rows(sh, wave, g, args.out, staged, staged_row, lane);
-                wave_sync();
+            if (__syncthreads_or(shifted) != 0) {
+                write_tile_chunk<true, STAGED>(sh, wave, g, args.out, n_i, units_here, n > TILE_CHUNK, lane);
+            } else {
+                write_tile_chunk<false, STAGED>(sh, wave, g, args.out, n_i, units_here, n > TILE_CHUNK, lane);
             }
         }
     }

@@ -2286,8 +2286,16 @@ bool compute(
         oargs.candidates_of_item = candidates_of_item;
         // How many waves share a tile in either pass follows the number of tiles the call before had on the same
         // number of points (policy.hpp); a list's first call on a system keeps one wave per tile.
-        const size_t tiles_before = ordered_items_per_tile == 1 && extras.ordered_tiles_points == n_points ? extras.ordered_tiles : 0;
+        const bool presorted = ordered_items_per_tile == 1;
+        const size_t tiles_before = presorted && extras.ordered_tiles_points == n_points ? extras.ordered_tiles : 0;
         oargs.write_split = ordered_write_split(n_points, tiles_before);
+        // well-filled tiles whose candidates come in one chunk: a workgroup per tile (write_tile.cuh)
+        const bool tile_writer =
+            presorted && std::getenv("VESIN_HIP_WRITE_SPLIT") == nullptr &&
+            ordered_write_by_tiles(n_points, n_cells, tiles_before, full_stencil, options.return_vectors);
+        if (tile_writer) {
+            oargs.write_split = TILE_WAVES;
+        }
         if (const char* text = std::getenv("VESIN_HIP_WRITE_SPLIT")) {
             oargs.write_split = static_cast<uint32_t>(std::max(1, std::min(4, std::atoi(text))));
         }
@@ -2310,7 +2318,6 @@ bool compute(
         // counting pass, and neither fills the GPU on systems of a few hundred thousand points (one wave per tile,
         // two waves per SIMD on 100,000 points): the two run side by side, the ordering on a stream of the list's
         // own that starts after the cell build and that the call's stream waits for right after the counting pass.
-        const bool presorted = ordered_items_per_tile == 1;
         auto launch_order = [&](hipStream_t where) {
             hipLaunchKernelGGL(
                 ordered_sort_kernel<false>, dim3(static_cast<uint32_t>((tiles_bound + ORDER_WAVES - 1) / ORDER_WAVES)),
@@ -2318,6 +2325,11 @@ bool compute(
             );
         };
         auto launch_write = [&]() {
+            if (tile_writer) {
+                auto kernel = oargs.out.vectors != nullptr ? ordered_write_kernel<true> : ordered_write_kernel<false>;
+                hipLaunchKernelGGL(kernel, dim3(blocks * ORDERED_WAVES), dim3(TILE_BLOCK), 0, stream, oargs, g);
+                return;
+            }
             auto kernel = presorted ? (options.full ? ordered_search_kernel<true, true, true> : ordered_search_kernel<true, false, true>)
                                     : (options.full ? ordered_search_kernel<true, true, false> : ordered_search_kernel<true, false, false>);
             hipLaunchKernelGGL(kernel, dim3(blocks * oargs.write_split), dim3(ORDERED_BLOCK), 0, stream, oargs, g);
@@ -2480,6 +2492,10 @@ bool compute(
             cargs.candidate_units = static_cast<uint32_t>(candidate_units);
             cargs.column_units = static_cast<uint32_t>(column_units);
             const bool early_write = known && extras.capacity > 0;
+            auto launch_write = [&]() {
+                auto kernel = cargs.out.vectors != nullptr ? crowded_write_kernel<true> : crowded_write_kernel<false>;
+                hipLaunchKernelGGL(kernel, dim3(tile_blocks), dim3(TILE_BLOCK), 0, stream, cargs, g);
+            };
             if (attempt > 0) {
                 hipLaunchKernelGGL(clear_crowded_status, dim3(1), dim3(1), 0, stream, crowded_status);
             }
@@ -2512,7 +2528,7 @@ bool compute(
                 cargs.out = outputs_of();
                 cargs.capacity = early_capacity;
                 mark(T_WRITE_BEGIN);
-                hipLaunchKernelGGL(crowded_write_kernel, dim3(tile_blocks), dim3(CROWDED_BLOCK), 0, stream, cargs, g);
+                launch_write();
                 mark(T_WRITE);
             }
             extras.wait(stream);
@@ -2553,7 +2569,7 @@ bool compute(
                 cargs.capacity = extras.capacity;
                 mark(T_WRITE_BEGIN);
                 if (total > 0) {
-                    hipLaunchKernelGGL(crowded_write_kernel, dim3(tile_blocks), dim3(CROWDED_BLOCK), 0, stream, cargs, g);
+                    launch_write();
                 }
                 mark(T_WRITE);
                 mark(T_SORT);

@@ -214,6 +214,23 @@ inline unsigned int ordered_write_split(size_t n_points, size_t tiles_before) {
     return tiles > 0.85 * resident && tiles <= 5.0 * resident ? 4 : 1;
 }
 
+/// Whether the writing pass gives every tile a workgroup that brings the candidates' coordinates to LDS (write_tile.cuh),
+/// from the same number. Bringing them pays when enough rows are made of them: 10 points per tile, or 16 when vectors are
+/// returned (their way through LDS leaves room for fewer workgroups). Candidates beyond 704 come in a second chunk,
+/// which costs more than it gives: 665 on average at most, so that few tiles have more. Writing pass, kernel with a wave
+/// per tile -> this, cutoff 5, liquids of 300,000 points with 8 / 10 / 16 / 20 / 28 points per cell: full lists P S d 220 ->
+/// 227, 228 -> 207, 307 -> 250, 328 -> 277, 388 -> 421 us; half lists P S d D 206 -> 299, 211 -> 278, 288 -> 260, 298 ->
+/// 291, 350 -> 439 us; 60,000 points with 6 / 10 / 16 / 20: full 57 -> 56, 68 -> 50, 81 -> 60, 89 -> 70 us, half 54 -> 74,
+/// 63 -> 64, 79 -> 66, 87 -> 70 us.
+inline bool ordered_write_by_tiles(size_t n_points, size_t n_cells, size_t tiles_before, size_t stencil_cells, bool vectors) {
+    if (tiles_before == 0 || n_cells == 0) {
+        return false;
+    }
+    const double points = static_cast<double>(n_points);
+    return points >= (vectors ? 16.0 : 10.0) * static_cast<double>(tiles_before) &&
+           static_cast<double>(stencil_cells) * points <= 665.0 * static_cast<double>(n_cells);
+}
+
 /// Waves that share the candidates of a tile in the counting pass (1 or 2), decided like the other.
 ///
 /// That pass runs seven waves per SIMD (7168 at a time) and lasts as long as its slowest wave, the one of the tile
