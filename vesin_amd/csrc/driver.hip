@@ -158,7 +158,7 @@ static bool two_pass_only() {
 
 /// Cells of the upper half of the stencil (the centre cell and what follows it in the kernels' order) that can hold
 /// a neighbour: what a tile's candidates are drawn from.
-static double upper_stencil_cells(const GridParams& g) {
+__host__ __device__ static double upper_stencil_cells(const GridParams& g) {
     if (g.prune == 0) {
         return 0.5 * ((2.0 * g.s[0] + 1.0) * (2.0 * g.s[1] + 1.0) * (2.0 * g.s[2] + 1.0) + 1.0);
     }
@@ -567,8 +567,214 @@ struct BatchVerletCache {
 /// stay few: up to 256 points without images (free molecules: 20,000 molecules of 3 to 40 atoms 0.75 -> 0.29 ms per
 /// unsorted batch, 1.16 -> 0.46 ms sorted), up to 69 points with the 27 images of a box wider than the cutoff.
 constexpr uint64_t ONE_CELL_TESTS = 131072; // points x points x images
-inline bool one_cell_in_a_batch(uint64_t n_points, uint64_t n_images) {
+__host__ __device__ inline bool one_cell_in_a_batch(uint64_t n_points, uint64_t n_images) {
     return n_points <= IMAGE_MAX_POINTS && n_images <= IMAGE_MAX_ENTRIES && n_points * n_points * n_images <= ONE_CELL_TESTS;
+}
+
+/// The grid of a system of a batch (box, flags and number of points of `g` are there already). False when a stencil
+/// would be wider than choose_grid allows.
+__host__ __device__ inline bool choose_batch_grid(
+    const HostBox& box, double cutoff, size_t n_points, const double* lo, const double* hi, int algorithm, GridParams& g
+) {
+    // (fewer than 32 points under the automatic choice: one cell whatever the grid would have been)
+    const bool automatic = algorithm == static_cast<int>(VesinAutoAlgorithm);
+    const bool single_cell = algorithm == static_cast<int>(VesinBruteForce) || (automatic && n_points < 32);
+    HostGrid grid;
+    if (!choose_grid_into(box, cutoff, n_points, lo, hi, single_cell, grid)) {
+        return false;
+    }
+    if (automatic && !single_cell && (grid.n_cells == 1 || n_points <= IMAGE_MAX_POINTS)) {
+        HostGrid one_cell;
+        const bool possible = choose_grid_into(box, cutoff, n_points, lo, hi, true, one_cell);
+        const uint64_t images = possible ? static_cast<uint64_t>(2 * one_cell.s[0] + 1) * (2 * one_cell.s[1] + 1) * (2 * one_cell.s[2] + 1) : 0;
+        if (grid.n_cells == 1) {
+            if (!possible) {
+                return false;
+            }
+            grid = one_cell;
+        } else if (possible && one_cell_in_a_batch(n_points, images)) {
+            // (a radius beyond what a stencil may have is no error of a choice that is only tried)
+            grid = one_cell;
+        }
+    }
+    for (int d = 0; d < 3; d++) {
+        g.n[d] = grid.n[d];
+        g.s[d] = grid.s[d];
+        g.np_min[d] = grid.np_min[d];
+        g.np_scale[d] = grid.np_scale[d];
+    }
+    g.cutoff2 = cutoff * cutoff;
+    g.n_points = static_cast<uint32_t>(n_points);
+    g.n_cells = static_cast<uint32_t>(grid.n_cells);
+    choose_pruning(box, grid, cutoff, g);
+    return true;
+}
+
+/// What the searches of a batch want to know of a system of some points.
+struct BatchShape {
+    bool images;          // the search over images covers it
+    bool tiles;           // not that, but the in-order search over tiles
+    uint32_t image_words; // words of 64 images per pair of points
+    double units;         // candidates per tile, in units of 64 (estimate)
+};
+
+__host__ __device__ inline BatchShape shape_in_batch(const GridParams& g) {
+    BatchShape shape;
+    const double per_cell = ::fmax(1.0, static_cast<double>(g.n_points) / static_cast<double>(g.n_cells > 0 ? g.n_cells : 1u));
+    shape.units = ::ceil(upper_stencil_cells(g) * per_cell / WAVE);
+    shape.images = g.n_points > 0 && images_cover(g);
+    shape.image_words = shape.images ? image_words(g) : 1u;
+    shape.tiles = g.n_points > 0 && !shape.images &&
+                  static_cast<uint64_t>(2 * g.s[0] + 1) * (2 * g.s[1] + 1) * (2 * g.s[2] + 1) <= MAX_ENTRIES;
+    return shape;
+}
+
+/// What the host learns of grids that were picked on the device (pinned memory).
+struct PickedGrids {
+    unsigned long long total_cells;
+    unsigned int problem; // some system has a direction that is not periodic, a box that is not invertible, a stencil
+                          // that is too wide: the host picks the grids (or says what is wrong)
+    unsigned int for_images;
+    unsigned int for_tiles;
+    unsigned int image_words;
+    unsigned int most_units;
+    unsigned int padding;
+};
+
+// Batches of fewer systems: the host picks their grids. (Sorted batches of crystals of 8 to 64 points, all new, grids picked
+// on the host -> on the device: 32 systems 151 -> 137, 256 systems 206 -> 157, 1024 systems 295 -> 175, 4096 systems 589 ->
+// 311 us per batch.)
+constexpr size_t PICK_SYSTEMS = 32;
+constexpr uint32_t PICK_PROBLEM = 1u << 31;
+constexpr uint32_t PICK_IMAGES = 1u << 30;
+constexpr uint32_t PICK_TILES = 1u << 29;
+constexpr uint32_t PICK_WORDS_AT = 25; // four bits
+constexpr uint32_t PICK_UNITS = (1u << PICK_WORDS_AT) - 1;
+
+/// The grids of a batch of systems that are periodic in all directions, one thread per system, by the functions the
+/// host picks them with. Bound by the chains of divisions and roots of a thread, which thousands of systems go through
+/// at once: 2000 crystals of 8 to 64 points take 19 us here, and took the host 0.2 ms, behind a copy of the
+/// boxes to it and before a copy of the grids back (a sorted batch of them, all new: 434 -> 233 us).
+__global__ __launch_bounds__(WAVE) void pick_grids_kernel(
+    const double* __restrict__ boxes, const bool* __restrict__ periodic, const uint32_t* __restrict__ first_point,
+    uint32_t n_systems, double cutoff, int algorithm, int full_stencil, GridParams* __restrict__ grids,
+    uint32_t* __restrict__ cells_of_system, uint32_t* __restrict__ shapes, double* __restrict__ kept_boxes,
+    unsigned char* __restrict__ kept_periodic
+) {
+    const uint32_t system = blockIdx.x * WAVE + threadIdx.x;
+    if (system >= n_systems) {
+        return;
+    }
+    double matrix[9];
+    bool flags[3];
+    for (int k = 0; k < 9; k++) {
+        matrix[k] = boxes[9 * static_cast<size_t>(system) + k];
+        kept_boxes[9 * static_cast<size_t>(system) + k] = matrix[k];
+    }
+    bool problem = false;
+    for (int d = 0; d < 3; d++) {
+        flags[d] = periodic[3 * static_cast<size_t>(system) + d];
+        kept_periodic[3 * static_cast<size_t>(system) + d] = flags[d] ? 1 : 0;
+        problem = problem || !flags[d];
+    }
+    const uint32_t n_here = first_point[system + 1] - first_point[system];
+    const double zeros[3] = {0.0, 0.0, 0.0};
+    HostBox box;
+    GridParams g = {};
+    uint32_t shape_word = PICK_PROBLEM;
+    uint32_t cells = 0;
+    if (!problem && normalise_box_into(matrix, flags, box)) {
+        for (int d = 0; d < 3; d++) {
+            for (int e = 0; e < 3; e++) {
+                g.H[3 * d + e] = box.H[d][e];
+                g.Hinv[3 * d + e] = box.Hinv[d][e];
+            }
+            g.periodic[d] = 1;
+        }
+        if (choose_batch_grid(box, cutoff, n_here, zeros, zeros, algorithm, g)) {
+            if (full_stencil != 0) {
+                g.prune = 0;
+            }
+            const BatchShape shape = shape_in_batch(g);
+            shape_word = (shape.images ? PICK_IMAGES : 0u) | (shape.tiles ? PICK_TILES : 0u) | (shape.image_words << PICK_WORDS_AT) |
+                         static_cast<uint32_t>(::fmin(shape.units, static_cast<double>(PICK_UNITS)));
+            cells = g.n_cells;
+        }
+    }
+    grids[system] = g;
+    cells_of_system[system] = cells;
+    shapes[system] = shape_word;
+}
+
+/// First cell of every system (exclusive scan of the cells per system, one workgroup), and what the host wants to know.
+__global__ __launch_bounds__(1024) void picked_bases_kernel(
+    const uint32_t* __restrict__ cells_of_system, const uint32_t* __restrict__ shapes, uint32_t n_systems,
+    uint32_t* __restrict__ cell_base, PickedGrids* report
+) {
+    __shared__ uint64_t wave_sums[16];
+    __shared__ unsigned int found[5]; // problem, images, tiles, words, units
+    const int lane = lane_id();
+    const int wave = threadIdx.x / WAVE;
+    if (threadIdx.x < 5) {
+        found[threadIdx.x] = 0;
+    }
+    __syncthreads();
+    uint32_t problem = 0, images = 0, tiles = 0, words = 1, units = 1;
+    uint64_t carried = 0;
+    for (uint32_t chunk = 0; chunk < n_systems; chunk += 1024) {
+        const uint32_t system = chunk + threadIdx.x;
+        const uint64_t own = system < n_systems ? cells_of_system[system] : 0;
+        if (system < n_systems) {
+            const uint32_t shape = shapes[system];
+            if ((shape & PICK_PROBLEM) != 0) {
+                problem = 1;
+            } else {
+                images += (shape & PICK_IMAGES) != 0 ? 1 : 0;
+                tiles += (shape & PICK_TILES) != 0 ? 1 : 0;
+                words = max(words, (shape >> PICK_WORDS_AT) & 15u);
+                units = max(units, shape & PICK_UNITS);
+            }
+        }
+        const uint64_t inclusive = wave_inclusive_scan(own);
+        if (lane == WAVE - 1) {
+            wave_sums[wave] = inclusive;
+        }
+        __syncthreads();
+        uint64_t before = 0;
+        uint64_t all = 0;
+        for (int w = 0; w < 16; w++) {
+            before += w < wave ? wave_sums[w] : 0;
+            all += wave_sums[w];
+        }
+        __syncthreads();
+        if (system < n_systems) {
+            cell_base[system] = static_cast<uint32_t>(carried + before + inclusive - own);
+        }
+        carried += all;
+    }
+    // (one atomic per wave: 1024 threads on one word go one after the other)
+    images = wave_inclusive_scan(images);
+    tiles = wave_inclusive_scan(tiles);
+#pragma unroll
+    for (int offset = WAVE / 2; offset > 0; offset >>= 1) {
+        words = max(words, static_cast<uint32_t>(__shfl_xor(static_cast<int>(words), offset, WAVE)));
+        units = max(units, static_cast<uint32_t>(__shfl_xor(static_cast<int>(units), offset, WAVE)));
+    }
+    const bool any_problem = __ballot(problem != 0) != 0;
+    if (lane == WAVE - 1) {
+        if (any_problem) {
+            atomicOr(&found[0], 1u);
+        }
+        atomicAdd(&found[1], images);
+        atomicAdd(&found[2], tiles);
+        atomicMax(&found[3], words);
+        atomicMax(&found[4], units);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        cell_base[n_systems] = static_cast<uint32_t>(carried);
+        *report = PickedGrids{carried, found[0], found[1], found[2], found[3], found[4], 0u};
+    }
 }
 
 struct BatchSetup {
@@ -604,6 +810,16 @@ struct BatchSetup {
     // bringing 75 bytes per system to the host and waiting for them before anything can be launched.
     DeviceBuffer kept_boxes;
     bool kept_on_device = false;
+    // grids picked on the device (pick_grids_kernel): they live in a buffer of their own, with the first points and first
+    // cells of the systems, and the host has neither grids nor boxes
+    bool picked = false;
+    DeviceBuffer picked_work;
+    GridParams* picked_grids = nullptr;
+    uint32_t* picked_first_point = nullptr;
+    uint32_t* picked_cell_base = nullptr;
+    PickedGrids* picked_report = nullptr;   // pinned
+    int pick_rest = 0;                      // calls left before that is tried again after a batch it is not for
+    size_t boxes_of = 0;                    // number of systems whose boxes are kept
     BoxGuess guess;
     // The single-pass search of a batch places its rows through the chain of workgroups: after a launch whose waves
     // gave up waiting, reused lists go straight to the two passes for a while.
@@ -965,6 +1181,11 @@ struct HipExtras {
         work.release();
         sort_work.release();
         batch.kept_boxes.release();
+        batch.picked_work.release();
+        if (batch.picked_report != nullptr) {
+            (void)hipHostFree(batch.picked_report);
+            batch.picked_report = nullptr;
+        }
         batch.molecule_work.release();
         if (batch.molecule_report != nullptr) {
             (void)hipHostFree(batch.molecule_report);
@@ -3134,7 +3355,7 @@ void direct_batch(
         setup.cutoff == options.cutoff && setup.algorithm == static_cast<int>(options.algorithm) &&
         setup.full_stencil == full_stencil_only() && setup.first_point.size() == n_systems + 1 &&
         std::memcmp(setup.first_point.data(), first_point, (n_systems + 1) * sizeof(size_t)) == 0 &&
-        setup.boxes.size() == 9 * n_systems && extras.mail == extras.mail_device;
+        setup.boxes_of == n_systems && extras.mail == extras.mail_device;
     if (may_guess && rest_is_the_same) {
         bool right = false;
         std::exception_ptr failure;
@@ -3654,6 +3875,105 @@ void verlet_batch(
 
 namespace {
 
+/// The grids of a batch picked on the device: what the host keeps of them, its work buffers apart. False when that is
+/// not for this batch (nothing has changed then but what an earlier call left).
+bool pick_grids(
+    const size_t* first_point, size_t n_systems, const double (*boxes)[3][3], const bool (*periodic)[3],
+    const VesinOptions& options, HipExtras& extras, hipStream_t stream
+) {
+    BatchSetup& setup = extras.batch;
+    const size_t n_points = first_point[n_systems];
+    if (n_points == 0 || n_systems < PICK_SYSTEMS || extras.mail != extras.mail_device || std::getenv("VESIN_HIP_GRIDS") != nullptr) {
+        return false;
+    }
+    if (setup.pick_rest > 0) {
+        setup.pick_rest -= 1;
+        return false;
+    }
+    if (setup.picked_report == nullptr) {
+        HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&setup.picked_report), sizeof(PickedGrids), hipHostMallocDefault));
+    }
+    // the set-up of the call before is gone from here on
+    setup.valid = false;
+    setup.picked = false;
+    setup.on_device = false;
+    setup.kept_on_device = false;
+    setup.boxes.clear();
+    setup.boxes_of = 0;
+    setup.first_point.assign(first_point, first_point + n_systems + 1);
+    setup.first_point32.resize(n_systems + 1);
+    setup.pair_base.resize(n_systems + 1);
+    setup.systems_with_points = 0;
+    setup.most_points = 0;
+    uint64_t pairs_so_far = 0;
+    for (size_t s = 0; s < n_systems; s++) {
+        const size_t n_here = first_point[s + 1] - first_point[s];
+        setup.first_point32[s] = static_cast<uint32_t>(first_point[s]);
+        setup.pair_base[s] = pairs_so_far;
+        pairs_so_far += n_here <= IMAGE_MAX_POINTS ? n_here * n_here : 0;
+        setup.systems_with_points += n_here > 0 ? 1 : 0;
+        setup.most_points = std::max(setup.most_points, n_here);
+    }
+    setup.first_point32[n_systems] = static_cast<uint32_t>(n_points);
+    setup.pair_base[n_systems] = pairs_so_far;
+
+    uint32_t* cells_of_system = nullptr;
+    uint32_t* shapes = nullptr;
+    auto carve = [&](Carver& c) {
+        setup.picked_grids = c.take<GridParams>(n_systems);
+        setup.picked_first_point = c.take<uint32_t>(n_systems + 1);
+        setup.picked_cell_base = c.take<uint32_t>(n_systems + 1);
+        cells_of_system = c.take<uint32_t>(n_systems);
+        shapes = c.take<uint32_t>(n_systems);
+    };
+    Carver measure(nullptr);
+    carve(measure);
+    setup.picked_work.reserve(measure.used);
+    Carver carver(setup.picked_work.ptr);
+    carve(carver);
+    setup.kept_boxes.reserve(75 * n_systems);
+    auto* kept = static_cast<unsigned char*>(setup.kept_boxes.ptr);
+    HIP_CHECK(hipMemcpyAsync(
+        setup.picked_first_point, setup.first_point32.data(), (n_systems + 1) * sizeof(uint32_t), hipMemcpyHostToDevice, stream
+    ));
+    hipLaunchKernelGGL(
+        pick_grids_kernel, dim3(static_cast<uint32_t>((n_systems + WAVE - 1) / WAVE)), dim3(WAVE), 0, stream,
+        reinterpret_cast<const double*>(boxes), reinterpret_cast<const bool*>(periodic), setup.picked_first_point,
+        static_cast<uint32_t>(n_systems), options.cutoff, static_cast<int>(options.algorithm), full_stencil_only() ? 1 : 0,
+        setup.picked_grids, cells_of_system, shapes, reinterpret_cast<double*>(kept), kept + 72 * n_systems
+    );
+    hipLaunchKernelGGL(
+        picked_bases_kernel, dim3(1), dim3(1024), 0, stream, cells_of_system, shapes, static_cast<uint32_t>(n_systems),
+        setup.picked_cell_base, setup.picked_report
+    );
+    HIP_CHECK(hipGetLastError());
+    extras.sync(stream);
+    const PickedGrids found = *setup.picked_report;
+    if (found.problem != 0) {
+        setup.pick_rest = SINGLE_PASS_REST;
+        return false;
+    }
+    if (found.total_cells >= 0xFFFFFFF0ull) {
+        throw std::runtime_error("too many cells in this batch");
+    }
+    setup.cutoff = options.cutoff;
+    setup.algorithm = static_cast<int>(options.algorithm);
+    setup.full_stencil = full_stencil_only();
+    setup.any_open_direction = false;
+    setup.all_open = false;
+    setup.cells_bound = 0;
+    setup.systems_for_images = found.for_images;
+    setup.systems_for_tiles = found.for_tiles;
+    setup.image_words = found.image_words;
+    setup.most_units = static_cast<double>(found.most_units);
+    setup.total_cells = found.total_cells;
+    setup.kept_on_device = true;
+    setup.boxes_of = n_systems;
+    setup.picked = true;
+    setup.valid = true;
+    return true;
+}
+
 /// The batch itself. `speculate`: from the grids of the call before, with the boxes compared on the device; false is
 /// returned when they turned out to be others (nothing of the result is to be used then).
 bool batch_attempt(
@@ -3678,6 +3998,8 @@ bool batch_attempt(
             setup.all_open ? size_t(0) : 9 * n_systems, 3 * n_systems, &extras.mail_device->batch_changed
         );
         same_setup = true;
+    } else if (pick_grids(first_point, n_systems, boxes, periodic, options, extras, stream)) {
+        same_setup = true;
     } else {
         // ---- every system's box comes to the host: the grids are picked there
         setup.incoming_boxes.resize(9 * n_systems);
@@ -3690,7 +4012,7 @@ bool batch_attempt(
         ));
         extras.sync(stream);
         same_setup =
-            setup.valid && !setup.any_open_direction && setup.cutoff == options.cutoff &&
+            setup.valid && !setup.picked && !setup.any_open_direction && setup.cutoff == options.cutoff &&
             setup.algorithm == static_cast<int>(options.algorithm) && setup.full_stencil == full_stencil_only() &&
             setup.first_point.size() == n_systems + 1 &&
             std::memcmp(setup.first_point.data(), first_point, (n_systems + 1) * sizeof(size_t)) == 0 &&
@@ -3704,8 +4026,10 @@ bool batch_attempt(
     PinnedVector<uint32_t>& first_point_host = setup.first_point32;
     if (!same_setup) {
         setup.valid = false;
+        setup.picked = false;
         setup.on_device = false;
         setup.kept_on_device = false;
+        setup.boxes_of = n_systems;
         setup.boxes.swap(setup.incoming_boxes);
         setup.periodic.swap(setup.incoming_periodic);
         setup.first_point.assign(first_point, first_point + n_systems + 1);
@@ -3837,47 +4161,22 @@ bool batch_attempt(
             const size_t n_here = first_point[s + 1] - first_point[s];
             const double* lo = bounds.empty() ? zeros : bounds[s].lo;
             const double* hi = bounds.empty() ? zeros : bounds[s].hi;
-            // (fewer than 32 points under the automatic choice: one cell whatever the grid would have been)
-            bool single_cell = options.algorithm == VesinBruteForce || (options.algorithm == VesinAutoAlgorithm && n_here < 32);
-            HostGrid grid = choose_grid(hbox, options.cutoff, n_here, lo, hi, single_cell);
-            if (options.algorithm == VesinAutoAlgorithm && !single_cell && grid.n_cells == 1) {
-                grid = choose_grid(hbox, options.cutoff, n_here, lo, hi, true);
-            } else if (options.algorithm == VesinAutoAlgorithm && !single_cell && n_here <= IMAGE_MAX_POINTS) {
-                // (a radius beyond what a stencil may have is an error of choose_grid: not for a choice that is only
-                // tried)
-                try {
-                    const HostGrid one_cell = choose_grid(hbox, options.cutoff, n_here, lo, hi, true);
-                    const uint64_t images = static_cast<uint64_t>(2 * one_cell.s[0] + 1) * (2 * one_cell.s[1] + 1) * (2 * one_cell.s[2] + 1);
-                    if (one_cell_in_a_batch(n_here, images)) {
-                        grid = one_cell;
-                    }
-                } catch (const std::runtime_error&) {
-                }
-            }
             GridParams& g = grids[s];
-            for (int d = 0; d < 3; d++) {
-                g.n[d] = grid.n[d];
-                g.s[d] = grid.s[d];
-                g.np_min[d] = grid.np_min[d];
-                g.np_scale[d] = grid.np_scale[d];
+            if (!choose_batch_grid(hbox, options.cutoff, n_here, lo, hi, static_cast<int>(options.algorithm), g)) {
+                throw std::runtime_error(
+                    "cutoff is too large for this box: more than 500 periodic images would be needed in one direction"
+                );
             }
-            g.cutoff2 = options.cutoff * options.cutoff;
-            g.n_points = static_cast<uint32_t>(n_here);
-            g.n_cells = static_cast<uint32_t>(grid.n_cells);
-            choose_pruning(hbox, grid, options.cutoff, g);
             if (full_stencil_only()) {
                 g.prune = 0;
             }
-            const double per_cell = std::max(1.0, static_cast<double>(g.n_points) / std::max(1u, g.n_cells));
-            mine.most_units = std::max(mine.most_units, std::ceil(upper_stencil_cells(g) * per_cell / WAVE));
+            const BatchShape shape = shape_in_batch(g);
+            mine.most_units = std::max(mine.most_units, shape.units);
             mine.systems_with_points += n_here > 0 ? 1 : 0;
             mine.most_points = std::max(mine.most_points, n_here);
-            if (n_here > 0 && images_cover(g)) {
-                mine.systems_for_images += 1;
-                mine.image_words = std::max(mine.image_words, image_words(g));
-            } else if (n_here > 0 && static_cast<uint64_t>(2 * g.s[0] + 1) * (2 * g.s[1] + 1) * (2 * g.s[2] + 1) <= MAX_ENTRIES) {
-                mine.systems_for_tiles += 1;
-            }
+            mine.systems_for_images += shape.images ? 1 : 0;
+            mine.systems_for_tiles += shape.tiles ? 1 : 0;
+            mine.image_words = std::max(mine.image_words, shape.image_words);
             setup.pair_base[s] = n_here <= IMAGE_MAX_POINTS ? n_here * n_here : 0;
             cell_base_host[s] = g.n_cells;
         }
@@ -4087,7 +4386,12 @@ bool batch_attempt(
     const bool already_there = same_setup && setup.on_device && setup.work_generation == extras.work.generation &&
                                setup.d_grids == d_grids &&
                                setup.d_first_point == d_first_point && setup.d_cell_base == d_cell_base;
-    if (device_grids) {
+    if (setup.picked) {
+        setup.on_device = false;
+        d_grids = setup.picked_grids;
+        d_first_point = setup.picked_first_point;
+        d_cell_base = setup.picked_cell_base;
+    } else if (device_grids) {
         setup.on_device = false; // (grids and first cells of this call are the device's own)
         HIP_CHECK(hipMemcpyAsync(
             d_first_point, first_point_host.data(), (n_systems + 1) * sizeof(uint32_t), hipMemcpyHostToDevice, stream

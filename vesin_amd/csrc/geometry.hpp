@@ -18,6 +18,13 @@
 #include <cstdint>
 #include <stdexcept>
 
+// this header is read by the host compiler alone (tests) and by hipcc, where some of its functions also run in kernels
+#ifdef __HIPCC__
+#define VESIN_HOST_DEVICE __host__ __device__
+#else
+#define VESIN_HOST_DEVICE
+#endif
+
 namespace vesin_hip {
 
 struct HostBox {
@@ -32,35 +39,33 @@ namespace detail {
         double x, y, z;
     };
 
-    inline double dot(V3 a, V3 b) {
+    VESIN_HOST_DEVICE inline double dot(V3 a, V3 b) {
         return a.x * b.x + a.y * b.y + a.z * b.z;
     }
 
-    inline V3 cross(V3 a, V3 b) {
+    VESIN_HOST_DEVICE inline V3 cross(V3 a, V3 b) {
         return V3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
     }
 
-    inline V3 unit(V3 a) {
-        double s = 1.0 / std::sqrt(dot(a, a));
+    VESIN_HOST_DEVICE inline V3 unit(V3 a) {
+        double s = 1.0 / ::sqrt(dot(a, a));
         return V3{s * a.x, s * a.y, s * a.z};
     }
 
-    inline V3 get_row(const double m[3][3], int i) {
+    VESIN_HOST_DEVICE inline V3 get_row(const double m[3][3], int i) {
         return V3{m[i][0], m[i][1], m[i][2]};
     }
 
-    inline void put_row(double m[3][3], int i, V3 v) {
+    VESIN_HOST_DEVICE inline void put_row(double m[3][3], int i, V3 v) {
         m[i][0] = v.x;
         m[i][1] = v.y;
         m[i][2] = v.z;
     }
 } // namespace detail
 
-/// Build the normalised box. Throws std::runtime_error("the box matrix is not invertible") like the reference
-/// (types.hpp:75-78).
-inline HostBox normalise_box(const double box[9], const bool periodic[3]) {
+/// Build the normalised box; false when it is not invertible.
+VESIN_HOST_DEVICE inline bool normalise_box_into(const double box[9], const bool periodic[3], HostBox& out) {
     using namespace detail;
-    HostBox out;
     int n_periodic = 0;
     int first = -1;
     int second = -1;
@@ -88,7 +93,7 @@ inline HostBox normalise_box(const double box[9], const bool periodic[3]) {
     } else if (n_periodic == 1) {
         V3 a = get_row(out.H, first);
         V3 helper{0.0, 1.0, 0.0};
-        if (std::abs(dot(unit(a), helper)) > 0.9) {
+        if (::fabs(dot(unit(a), helper)) > 0.9) {
             helper = V3{0.0, 0.0, 1.0};
         }
         V3 c = unit(cross(a, helper));
@@ -104,8 +109,8 @@ inline HostBox normalise_box(const double box[9], const bool periodic[3]) {
     double det = m[0][0] * (m[1][1] * m[2][2] - m[2][1] * m[1][2])
                - m[0][1] * (m[1][0] * m[2][2] - m[1][2] * m[2][0])
                + m[0][2] * (m[1][0] * m[2][1] - m[1][1] * m[2][0]);
-    if (!(std::abs(det) >= 1e-30)) {
-        throw std::runtime_error("the box matrix is not invertible");
+    if (!(::fabs(det) >= 1e-30)) {
+        return false;
     }
 
     out.Hinv[0][0] = (m[1][1] * m[2][2] - m[2][1] * m[1][2]) / det;
@@ -121,9 +126,18 @@ inline HostBox normalise_box(const double box[9], const bool periodic[3]) {
     V3 a = get_row(out.H, 0);
     V3 b = get_row(out.H, 1);
     V3 c = get_row(out.H, 2);
-    out.face[0] = std::abs(dot(unit(cross(b, c)), a));
-    out.face[1] = std::abs(dot(unit(cross(c, a)), b));
-    out.face[2] = std::abs(dot(unit(cross(a, b)), c));
+    out.face[0] = ::fabs(dot(unit(cross(b, c)), a));
+    out.face[1] = ::fabs(dot(unit(cross(c, a)), b));
+    out.face[2] = ::fabs(dot(unit(cross(a, b)), c));
+    return true;
+}
+
+/// The same, throwing std::runtime_error("the box matrix is not invertible") like the reference (types.hpp:75-78).
+inline HostBox normalise_box(const double box[9], const bool periodic[3]) {
+    HostBox out;
+    if (!normalise_box_into(box, periodic, out)) {
+        throw std::runtime_error("the box matrix is not invertible");
+    }
     return out;
 }
 
@@ -137,13 +151,6 @@ struct HostGrid {
 
 constexpr double CELL_MARGIN = 1.0 + 1e-9;
 constexpr int32_t MAX_STENCIL_RADIUS = 500;
-
-// this header is read by the host compiler alone (tests) and by hipcc, where some of its functions also run in kernels
-#ifdef __HIPCC__
-#define VESIN_HOST_DEVICE __host__ __device__
-#else
-#define VESIN_HOST_DEVICE
-#endif
 
 /// Shrinks a grid of cells[0] x cells[1] x cells[2] cells (whole numbers, 1 at least) until it holds at most `most`
 /// cells (1 at least), all directions that have more than one cell by the same factor. A direction that the factor
@@ -180,11 +187,12 @@ VESIN_HOST_DEVICE inline void limit_cells(double cells[3], double most) {
 
 /// Choose the cell grid. `lo`/`hi` are the extrema of the fractional (projected) coordinates; they are only read
 /// for non-periodic directions. With `single_cell` every point goes to one cell and the stencil enumerates the
-/// periodic images directly (the brute-force and multi-image path).
-inline HostGrid choose_grid(
-    const HostBox& box, double cutoff, size_t n_points, const double lo[3], const double hi[3], bool single_cell
+/// periodic images directly (the brute-force and multi-image path). False when a direction would need more than
+/// MAX_STENCIL_RADIUS images.
+VESIN_HOST_DEVICE inline bool choose_grid_into(
+    const HostBox& box, double cutoff, size_t n_points, const double lo[3], const double hi[3], bool single_cell,
+    HostGrid& grid
 ) {
-    HostGrid grid;
     double extent[3];
     double cells[3];
     const double padded = cutoff * CELL_MARGIN;
@@ -209,7 +217,7 @@ inline HostGrid choose_grid(
             grid.np_scale[d] = 1.0 / extent[d];
         }
 
-        cells[d] = std::floor(extent[d] / padded);
+        cells[d] = ::floor(extent[d] / padded);
         if (!(cells[d] >= 1.0)) {
             cells[d] = 1.0;
         }
@@ -236,7 +244,7 @@ inline HostGrid choose_grid(
         grid.n[d] = static_cast<int32_t>(cells[d]);
         grid.n_cells *= static_cast<uint64_t>(grid.n[d]);
 
-        double radius = std::ceil(padded * cells[d] / extent[d]);
+        double radius = ::ceil(padded * cells[d] / extent[d]);
         if (!(radius >= 1.0)) {
             radius = 1.0;
         }
@@ -247,11 +255,22 @@ inline HostGrid choose_grid(
             }
         }
         if (radius > static_cast<double>(MAX_STENCIL_RADIUS)) {
-            throw std::runtime_error(
-                "cutoff is too large for this box: more than 500 periodic images would be needed in one direction"
-            );
+            return false;
         }
         grid.s[d] = static_cast<int32_t>(radius);
+    }
+    return true;
+}
+
+/// The same, throwing std::runtime_error instead.
+inline HostGrid choose_grid(
+    const HostBox& box, double cutoff, size_t n_points, const double lo[3], const double hi[3], bool single_cell
+) {
+    HostGrid grid;
+    if (!choose_grid_into(box, cutoff, n_points, lo, hi, single_cell, grid)) {
+        throw std::runtime_error(
+            "cutoff is too large for this box: more than 500 periodic images would be needed in one direction"
+        );
     }
     return grid;
 }
@@ -277,7 +296,7 @@ VESIN_HOST_DEVICE inline bool stencil_entry_too_far(const Grid& g, int32_t dx, i
 /// of two or more: with radius one every cell of the stencil touches the centre cell. The slack carries a millionth
 /// of a cell for the rounding of the fractional coordinates that put the points into their cells.
 template <typename Grid>
-inline void choose_pruning(const HostBox& box, const HostGrid& grid, double cutoff, Grid& g) {
+VESIN_HOST_DEVICE inline void choose_pruning(const HostBox& box, const HostGrid& grid, double cutoff, Grid& g) {
     using namespace detail;
     g.prune = 0;
     g.prune_limit = cutoff * cutoff * CELL_MARGIN * CELL_MARGIN;
@@ -299,15 +318,15 @@ inline void choose_pruning(const HostBox& box, const HostGrid& grid, double cuto
         edge[d] = V3{row.x * scale, row.y * scale, row.z * scale};
     }
     // orthonormal frame by Gram-Schmidt: q0 along edge 0, q1 in the plane of edges 0 and 1
-    const double l00 = std::sqrt(dot(edge[0], edge[0]));
-    if (!(l00 > 0.0) || !std::isfinite(l00)) {
+    const double l00 = ::sqrt(dot(edge[0], edge[0]));
+    if (!(l00 > 0.0) || !(l00 < INFINITY)) {
         return;
     }
     const V3 q0 = V3{edge[0].x / l00, edge[0].y / l00, edge[0].z / l00};
     const double l10 = dot(edge[1], q0);
     const V3 rest1 = V3{edge[1].x - l10 * q0.x, edge[1].y - l10 * q0.y, edge[1].z - l10 * q0.z};
-    const double l11 = std::sqrt(dot(rest1, rest1));
-    if (!(l11 > 1e-9 * l00) || !std::isfinite(l11)) {
+    const double l11 = ::sqrt(dot(rest1, rest1));
+    if (!(l11 > 1e-9 * l00) || !(l11 < INFINITY)) {
         return;
     }
     const V3 q1 = V3{rest1.x / l11, rest1.y / l11, rest1.z / l11};
@@ -315,7 +334,7 @@ inline void choose_pruning(const HostBox& box, const HostGrid& grid, double cuto
     const double l21 = dot(edge[2], q1);
     const V3 q2 = cross(q0, q1);
     const double l22 = dot(edge[2], q2);
-    if (!(std::abs(l22) > 1e-9 * l00) || !std::isfinite(l22)) {
+    if (!(::fabs(l22) > 1e-9 * l00) || !(::fabs(l22) < INFINITY)) {
         return;
     }
     const double margin = 1.0 + 1e-6;
@@ -325,9 +344,9 @@ inline void choose_pruning(const HostBox& box, const HostGrid& grid, double cuto
     g.prune_edges[3] = l11;
     g.prune_edges[4] = l21;
     g.prune_edges[5] = l22;
-    g.prune_slack[0] = (std::abs(l00) + std::abs(l10) + std::abs(l20)) * margin;
-    g.prune_slack[1] = (std::abs(l11) + std::abs(l21)) * margin;
-    g.prune_slack[2] = std::abs(l22) * margin;
+    g.prune_slack[0] = (::fabs(l00) + ::fabs(l10) + ::fabs(l20)) * margin;
+    g.prune_slack[1] = (::fabs(l11) + ::fabs(l21)) * margin;
+    g.prune_slack[2] = ::fabs(l22) * margin;
     g.prune = 1;
 }
 
