@@ -217,3 +217,14 @@ def test_other_molecules_with_every_call_and_a_list_that_starts_with_crystals(ca
         lists = batch(another, crystals, flags=flags, boxes=boxes)
         assert ("free molecules no more" in capfd.readouterr().err) == (call == 0)
         check_in_order(lists, crystals, 2.5, True, f"crystals, call {call}", flags=flags, boxes=boxes)
+
+
+@pytest.mark.parametrize("full", [True, False], ids=["full", "half"])
+def test_every_number_of_points_of_a_wave(full):
+    """Systems of 0, 1, ..., 64 points, a wave each whose lanes share the pairs: the step from one pair of a lane to its
+    next is another one for every number of points."""
+    rng = np.random.default_rng(64)
+    molecules = [rng.normal(scale=1.5, size=(n, 3)) for n in range(65)]
+    calculator = NeighborList(cutoff=2.5, full_list=full, sorted=True)
+    for call in range(2):
+        check_in_order(batch(calculator, molecules), molecules, 2.5, full, f"call {call}")

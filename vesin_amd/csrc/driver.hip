@@ -3461,7 +3461,7 @@ bool molecules_batch(
 
     args.total_points = static_cast<uint32_t>(n_points);
     args.first_row = d_first_row;
-    const size_t per_block = wide ? 1 : static_cast<size_t>(MOLECULE_BLOCK / WAVE) * (WAVE / lanes);
+    const size_t per_block = wide ? 1 : static_cast<size_t>(MOLECULE_BLOCK / WAVE) * (lanes >= 32 ? 1 : WAVE / lanes);
     const unsigned blocks = static_cast<unsigned>((n_systems + per_block - 1) / per_block);
     auto launch = [&](bool write) {
         const dim3 grid(blocks), block(MOLECULE_BLOCK);
@@ -3472,10 +3472,9 @@ bool molecules_batch(
         case 17: hipLaunchKernelGGL((molecules_kernel<8, true>), grid, block, 0, stream, args); break;
         case 32: hipLaunchKernelGGL((molecules_kernel<16, false>), grid, block, 0, stream, args); break;
         case 33: hipLaunchKernelGGL((molecules_kernel<16, true>), grid, block, 0, stream, args); break;
-        case 64: hipLaunchKernelGGL((molecules_kernel<32, false>), grid, block, 0, stream, args); break;
-        case 65: hipLaunchKernelGGL((molecules_kernel<32, true>), grid, block, 0, stream, args); break;
-        case 128: hipLaunchKernelGGL((molecules_kernel<64, false>), grid, block, 0, stream, args); break;
-        default: hipLaunchKernelGGL((molecules_kernel<64, true>), grid, block, 0, stream, args); break;
+        case 64:
+        case 128: hipLaunchKernelGGL((molecules_pairs_kernel<false>), grid, block, 0, stream, args); break;
+        default: hipLaunchKernelGGL((molecules_pairs_kernel<true>), grid, block, 0, stream, args); break;
         }
     };
 

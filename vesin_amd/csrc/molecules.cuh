@@ -1,11 +1,12 @@
 // Batches of free molecules: systems without any periodic direction and with at most 256 points each. Such a system has
 // no images and no use for a cell list: every point is tested against every other, v = r_j - r_i, |v|^2 < cutoff^2
 // (the rows of the reference's CPU engine for such a system, vesin/src/cpu_cell_list.cpp:634-730 with all shifts
-// zero). A group of 8, 16, 32 or 64 lanes takes one system, so a wave takes up to eight: lane j of the group holds
+// zero). A group of 8 or 16 lanes takes one system, so a wave takes up to eight: lane j of the group holds
 // point j, the group goes over i = 0, 1, ..., every lane tests (i, j), and the kept lanes of the group are consecutive
 // rows. The rows of a system therefore come out ordered by (i, j), which is the sorted order, and a call is a counting
 // pass (rows per system), a scan over the systems (which is `first_pair`), and a writing pass. Batches with a system
-// of more than 64 points give every system a workgroup of four waves instead (molecules_wide_kernel), each wave taking
+// of more than 16 points give every system a wave, whose lanes take the pairs (i, j) in the same order
+// (molecules_pairs_kernel). Batches with a system of more than 64 points give every system a workgroup of four waves instead (molecules_wide_kernel), each wave taking
 // every fourth i with the j in rounds of 64: rows are counted per point then, and scanned over the points.
 #ifndef VESIN_HIP_MOLECULES_CUH
 #define VESIN_HIP_MOLECULES_CUH
@@ -148,6 +149,109 @@ __global__ __launch_bounds__(MOLECULE_BLOCK) void molecules_kernel(MoleculeArgs 
         }
     }
     if (!WRITE && exists && j == 0) {
+        a.rows_of_system[system] = rows;
+    }
+}
+
+/// One wave per system, for systems of 17 to 64 points (by the largest of the batch): lane l takes the pairs l, l + 64, ...
+/// of the n x n pairs (i, j) in the order of the list, the points in LDS. COUNT is bound by the arithmetic and the latency
+/// of a round: a lane per second point (molecules_kernel) goes through n rounds with n of its lanes at work, this through
+/// n^2 / 64 with all of them. WRITE is bound by its stores: rows follow each other without regard to cache lines, which
+/// the caches put together (non-temporal stores, which go past them, took twice as long).
+/// 20,000 molecules of 3 to 40 points, cutoff 5, rows P d D, 64 lanes per system -> this: COUNT 38 -> 23 us, WRITE 81 -> 74 us
+/// (4.2 TB/s); two such batches 438 -> 395 us.
+template <bool WRITE>
+__global__ __launch_bounds__(MOLECULE_BLOCK) void molecules_pairs_kernel(MoleculeArgs a) {
+    constexpr uint32_t WAVES = MOLECULE_BLOCK / WAVE;
+    __shared__ double px[WAVES][MOLECULE_GROUP_POINTS], py[WAVES][MOLECULE_GROUP_POINTS], pz[WAVES][MOLECULE_GROUP_POINTS];
+    const uint32_t lane = static_cast<uint32_t>(lane_id());
+    const uint32_t wave = uniform(threadIdx.x / WAVE);
+    const uint32_t system = blockIdx.x * WAVES + wave;
+
+    if (WRITE) {
+        const unsigned long long total = a.first_pair[a.n_systems];
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            a.report->periodic = a.status->periodic;
+            a.report->first_bad = a.status->first_bad;
+            a.report->total_rows = total;
+        }
+        if (total > a.capacity || a.status->periodic != 0) {
+            return;
+        }
+    }
+    if (system >= a.n_systems) {
+        return;
+    }
+    const uint32_t begin = uniform(a.first_point[system]);
+    const uint32_t n = uniform(a.first_point[system + 1]) - begin; // (at most MOLECULE_GROUP_POINTS: the host)
+    if (lane < n) {
+        const size_t at = 3 * static_cast<size_t>(begin + lane);
+        const double x = a.points[at + 0];
+        const double y = a.points[at + 1];
+        const double z = a.points[at + 2];
+        px[wave][lane] = x;
+        py[wave][lane] = y;
+        pz[wave][lane] = z;
+        if (!WRITE) {
+            unsigned int axis;
+            if (!all_finite(x, y, z, axis)) {
+                atomicMin(&a.status->first_bad, 3u * (begin + lane) + axis);
+            }
+        }
+    }
+    if (!WRITE && lane < 3 && a.periodic[3 * static_cast<size_t>(system) + lane]) {
+        a.status->periodic = 1;
+    }
+    wave_sync();
+
+    uint64_t row = WRITE ? uniform(a.first_pair[system]) : 0;
+    uint32_t rows = 0;
+    const uint32_t divisor = n > 0 ? n : 1u;
+    uint32_t i = lane / divisor;
+    uint32_t j = lane % divisor;
+    const uint32_t step_i = WAVE / divisor;
+    const uint32_t step_j = WAVE % divisor;
+    for (uint32_t pair = 0; pair < n * n; pair += WAVE) {
+        const bool there = i < n;
+        const uint32_t from = there ? i : 0u;
+        // (the shift of every pair is zero: adding it is what the general search does, and what turns a -0 into 0)
+        const double vx = (px[wave][j] - px[wave][from]) + 0.0;
+        const double vy = (py[wave][j] - py[wave][from]) + 0.0;
+        const double vz = (pz[wave][j] - pz[wave][from]) + 0.0;
+        const double dd = vx * vx + vy * vy + vz * vz;
+        const bool keep = there && (a.full ? j != i : j > i) && dd < a.cutoff2;
+        const uint64_t mask = __ballot(keep);
+        if (WRITE) {
+            if (keep) {
+                const uint64_t at = row + rank_in_mask(mask);
+                a.out.pairs[2 * at + 0] = i;
+                a.out.pairs[2 * at + 1] = j;
+                if (a.out.shifts != nullptr) {
+                    a.out.shifts[3 * at + 0] = 0;
+                    a.out.shifts[3 * at + 1] = 0;
+                    a.out.shifts[3 * at + 2] = 0;
+                }
+                if (a.out.distances != nullptr) {
+                    a.out.distances[at] = sqrt(dd);
+                }
+                if (a.out.vectors != nullptr) {
+                    a.out.vectors[3 * at + 0] = vx;
+                    a.out.vectors[3 * at + 1] = vy;
+                    a.out.vectors[3 * at + 2] = vz;
+                }
+            }
+            row += static_cast<uint64_t>(__popcll(mask));
+        } else {
+            rows += static_cast<uint32_t>(__popcll(mask));
+        }
+        i += step_i;
+        j += step_j;
+        if (j >= n) {
+            j -= n;
+            i += 1;
+        }
+    }
+    if (!WRITE && lane == 0) {
         a.rows_of_system[system] = rows;
     }
 }
