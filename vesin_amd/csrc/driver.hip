@@ -2729,6 +2729,7 @@ bool compute(
                     (crowded_sort_kernel<CROWDED_SMALL, CROWDED_LARGE, CROWDED_SORT_BLOCK>), dim3(std::min(tile_blocks, 2048u)),
                     dim3(CROWDED_SORT_BLOCK), 0, stream, cargs, g
                 );
+                mark(T_SORT);
                 auto count = options.full ? crowded_count_kernel<true> : crowded_count_kernel<false>;
                 hipLaunchKernelGGL(count, dim3(tile_blocks), dim3(CROWDED_BLOCK), 0, stream, cargs, g);
                 mark(T_COUNT);
@@ -2793,21 +2794,18 @@ bool compute(
                     launch_write();
                 }
                 mark(T_WRITE);
-                mark(T_SORT);
                 HIP_CHECK(hipStreamSynchronize(stream));
-            } else {
-                mark(T_SORT);
-                if (timed) {
-                    HIP_CHECK(hipStreamSynchronize(stream));
-                }
+            } else if (timed) {
+                HIP_CHECK(hipStreamSynchronize(stream));
             }
             HIP_CHECK(hipGetLastError());
             neighbors.length = total;
             if (timed) {
                 extras.timings = {};
-                extras.timings.total = elapsed(T_START, T_SORT);
+                extras.timings.total = elapsed(T_START, T_WRITE);
                 extras.timings.cell_build = elapsed(T_START, T_CELLS);
-                extras.timings.count = elapsed(T_CELLS, T_COUNT);
+                extras.timings.sort = elapsed(T_CELLS, T_SORT); // (of the candidates: MEASURE and SORT)
+                extras.timings.count = elapsed(T_SORT, T_COUNT);
                 extras.timings.scan = elapsed(T_COUNT, T_SCAN);
                 extras.timings.write = elapsed(T_WRITE_BEGIN, T_WRITE);
                 extras.timings_valid = true;
