@@ -2773,13 +2773,17 @@ bool compute(
             if (found.found.unsuitable != 0 || found.found.max_candidates > CROWDED_LARGE) {
                 break;
             }
+            const bool pays = crowded_search_only() || crowded_search_pays(n_points, found.n_tiles);
+            if (!known && !pays) {
+                break;
+            }
             if (!known || found.found.overflow != 0) {
                 candidate_units = candidate_units_found + candidate_units_found / 8 + 64;
                 column_units = column_units_found + column_units_found / 8 + 64;
                 known = true;
                 continue;
             }
-            extras.crowded_points = n_points;
+            extras.crowded_points = pays ? n_points : 0; // (0: the next call counts, and decides, before it does anything else)
             extras.crowded_candidate_units = std::max(candidate_units, candidate_units_found + candidate_units_found / 8 + 64);
             extras.crowded_column_units = std::max(column_units, column_units_found + column_units_found / 8 + 64);
             const size_t total = found.total_rows;

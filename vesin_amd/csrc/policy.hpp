@@ -190,6 +190,15 @@ inline bool ordered_records_fit(size_t n_points, size_t record_bytes) {
     return static_cast<double>(record_bytes) <= allowed;
 }
 
+/// Whether the in-order search for crowded cells (crowded.cuh) is the faster way to a sorted list than the radix sort. It
+/// gives every tile workgroups of its own, whatever the tile holds; the radix sort's time follows the rows and has a floor
+/// of 0.2 ms. Per call, radix sort -> that search, cutoff 5, liquids of 300,000 points with 2 / 3 / 4 / 6 / 8 points per cell:
+/// full lists i j S d 793 -> 1118, 869 -> 920, 1007 -> 762, 1279 -> 622, 1587 -> 545 us, half lists i j S d D 676 -> 1242,
+/// 707 -> 1032, 764 -> 859, 909 -> 710, 1101 -> 628 us; 20,000 points with 0.3 / 1 / 4: 203 -> 202, 218 -> 182, 215 -> 126 us.
+inline bool crowded_search_pays(size_t n_points, size_t n_tiles) {
+    return n_tiles <= 16384 || n_points >= 5 * n_tiles;
+}
+
 /// Waves that share the points of a tile in the writing pass (1 or 4), from the number of tiles the call before had
 /// on the same points (0: not known, one wave).
 ///
