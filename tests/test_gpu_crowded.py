@@ -107,7 +107,11 @@ def test_a_list_that_meets_other_systems(capfd, monkeypatch):
     arrays too."""
     monkeypatch.setenv("VESIN_HIP_SORT", "crowded")
     calculator = NeighborList(cutoff=3.0, full_list=True, sorted=True)
-    for n, edge in [(500, 12.0), (2000, 12.0), (2000, 9.0), (2000, 20.0), (1000, 8.0), (1000, 8.0)]:
+    # (2600 points: as many candidates around a cell of the smaller box, few in the larger one: the sort for the most
+    # crowded cells is not launched where the call before had none)
+    systems = [(500, 12.0), (2000, 12.0), (2000, 9.0), (2000, 20.0), (1000, 8.0), (1000, 8.0)]
+    systems += [(2600, 20.0), (2600, 20.0), (2600, 9.0), (2600, 9.0), (2600, 20.0), (2600, 20.0)]
+    for n, edge in systems:
         points, box = _liquid(n, edge, n)
         expected = _expected(points, box, True, 3.0, True)
         result = _compute(calculator, points, box, True)

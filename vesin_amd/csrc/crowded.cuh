@@ -35,7 +35,7 @@ namespace vesin_hip {
 constexpr int CROWDED_WAVES = 4;
 constexpr int CROWDED_BLOCK = CROWDED_WAVES * WAVE;
 constexpr uint32_t CROWDED_SMALL = 2048;   // candidates that the usual sorting kernel takes (29 KB of LDS)
-constexpr uint32_t CROWDED_LARGE = 8192;   // and the one for the most crowded cells (103 KB)
+constexpr uint32_t CROWDED_LARGE = 8192;   // and the one for the most crowded cells (115 KB)
 constexpr int CROWDED_SORT_BLOCK = 512;    // threads of the latter
 
 /// A candidate, in the order of (original index, shift).

@@ -653,8 +653,8 @@ constexpr uint32_t PICK_UNITS = (1u << PICK_WORDS_AT) - 1;
 
 /// The grids of a batch of systems that are periodic in all directions, one thread per system, by the functions the
 /// host picks them with. Bound by the chains of divisions and roots of a thread, which thousands of systems go through
-/// at once: 2000 crystals of 8 to 64 points take 19 us here, and took the host 0.2 ms, behind a copy of the
-/// boxes to it and before a copy of the grids back (a sorted batch of them, all new: 434 -> 233 us).
+/// at once: 2000 crystals of 8 to 64 points take 13 us here, and took the host 0.2 ms, behind a copy of the
+/// boxes to it and before a copy of the grids back (a sorted batch of them, all new: 433 -> 211 us).
 __global__ __launch_bounds__(WAVE) void pick_grids_kernel(
     const double* __restrict__ boxes, const bool* __restrict__ periodic, const uint32_t* __restrict__ first_point,
     uint32_t n_systems, double cutoff, int algorithm, int full_stencil, GridParams* __restrict__ grids,

@@ -18,7 +18,8 @@
 // Small systems (several waves per tile) skip SORT: their WRITE takes the candidates in table order and ranks the
 // rows of every point by comparing all its keys (at most 256, read as LDS broadcasts).
 // Rows per point beyond 256, candidates per tile beyond 1024, stencils beyond 64 cells or shifts and wraps beyond
-// +-255 are reported in the status and the host falls back to the unsorted search followed by the radix sort.
+// +-255 are reported in the status and the host goes on with the search for crowded cells (crowded.cuh) where that covers the
+// system, or with the unsorted search followed by the radix sort.
 //
 // Arithmetic as everywhere (vesin/src/cpu_cell_list.cpp:135-138, vesin/src/types.hpp:232-243):
 // S = cell shift - wrap_j + wrap_i, T = S . H left to right, v = (r_j - r_i) + T, d2 = vx*vx + vy*vy + vz*vz,
