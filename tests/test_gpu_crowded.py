@@ -163,3 +163,29 @@ def test_systems_that_come_by_themselves(kind, capfd, monkeypatch):
         assert ("crowded search:" in capfd.readouterr().err) == (kind != "sparse" or call == 0)
         for key in result:
             assert np.array_equal(result[key], expected[key]), (call, key)
+
+
+def test_the_rest_after_a_refused_system_ends(capfd, monkeypatch):
+    """A list that met a system this search refuses leaves it alone for 64 calls, also where the usual in-order search is
+    not tried either (records of a fixed size for so many cells would not fit), and takes it up again then."""
+    import torch
+
+    monkeypatch.setenv("VESIN_HIP_DEBUG", "1")
+    rng = np.random.default_rng(4)
+    box, cutoff = 220.0 * np.eye(3), 2.0
+    sparse = 220.0 * rng.random((200_000, 3))
+    blobs = (220.0 * rng.random((50, 1, 3)) + 3.2 * rng.normal(size=(50, 4000, 3))).reshape(-1, 3)
+    expected = _expected(blobs, box, True, cutoff, False)
+    calculator = NeighborList(cutoff=cutoff, full_list=False, sorted=True)
+    _compute(calculator, sparse, box, True)
+    device_points, device_box = torch.tensor(blobs, device="cuda:0"), torch.tensor(box, device="cuda:0")
+    tried = []
+    for _ in range(66):
+        capfd.readouterr()
+        outputs = calculator.compute(device_points, device_box, True, "PSdD")
+        err = capfd.readouterr().err
+        assert "in-order search:" not in err
+        tried.append("crowded search:" in err)
+    assert tried == [False] * 64 + [True] * 2
+    for q, out in zip("PSdD", outputs):
+        assert np.array_equal(out.cpu().numpy(), expected[NAMES[q]]), q

@@ -1950,12 +1950,6 @@ bool compute(
     if (crowded_search_only()) {
         try_in_order = false;
     }
-    // what that search does not cover goes to the one for crowded cells (which allocates its work memory on the way)
-    bool try_crowded = options.sorted && full_stencil <= MAX_ENTRIES && !radix_sort_only() && !extras.fixed_memory;
-    if (try_crowded && extras.crowded_rest > 0) {
-        extras.crowded_rest -= try_in_order ? 0 : 1;
-        try_crowded = false;
-    }
     // Small systems with arrays from earlier calls: everything in one launch (small.cuh), as one work item per point
     // for a sorted list, as one per point and slice of its candidates otherwise (about four units of 64 candidates
     // per item, as many items as the smallest shape of that launch takes).
@@ -2033,6 +2027,13 @@ bool compute(
         static_cast<size_t>(ordered_blocks) * ORDERED_WAVES * ORDERED_UNITS * WAVE * sizeof(CandidateRecord);
     if (try_in_order && !extras.fixed_memory && !ordered_records_fit(n_points, ordered_record_bytes)) {
         try_in_order = false; // a sparse system of many cells: see ordered_records_fit
+    }
+    // what that search does not cover goes to the one for crowded cells (which allocates its work memory on the way);
+    // its rest is over after as many calls that would have come to it, whatever keeps the usual search from them
+    bool try_crowded = options.sorted && full_stencil <= MAX_ENTRIES && !radix_sort_only() && !extras.fixed_memory;
+    if (try_crowded && extras.crowded_rest > 0) {
+        extras.crowded_rest -= try_in_order ? 0 : 1;
+        try_crowded = false;
     }
     const size_t scratch_elements = std::max(
         std::max(scan_scratch_elements(n_cells), scan_scratch_elements(n_slots)),
