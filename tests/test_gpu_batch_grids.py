@@ -98,3 +98,20 @@ def test_open_directions_and_boxes_without_an_inverse(monkeypatch):
         with pytest.raises(RuntimeError, match=message):
             _rows(calculator, (batch[0], batch[1], boxes))
         _same(_rows(calculator, batch), all_periodic)
+
+
+@pytest.mark.parametrize("n_systems", [32, 300])
+def test_a_repeated_batch_sends_nothing_again(n_systems, capfd, monkeypatch):
+    """What the sorted search needs of the division into systems goes to the device once for a batch that is called
+    again, and again for another batch."""
+    monkeypatch.setenv("VESIN_HIP_DEBUG", "1")
+    calculator = NeighborList(cutoff=3.5, full_list=True, sorted=True)
+    for batch in (_batch(n_systems, 9, 12), _batch(n_systems, 10, 12)):
+        expected = _rows(NeighborList(cutoff=3.5, full_list=True, sorted=True), batch)
+        sent = []
+        for _ in range(4):
+            capfd.readouterr()
+            rows = _rows(calculator, batch)
+            sent.append("first pairs of" in capfd.readouterr().err)
+            _same(rows, expected)
+        assert sent == [True, False, False, False]

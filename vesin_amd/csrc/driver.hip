@@ -810,13 +810,15 @@ struct BatchSetup {
     // bringing 75 bytes per system to the host and waiting for them before anything can be launched.
     DeviceBuffer kept_boxes;
     bool kept_on_device = false;
-    // grids picked on the device (pick_grids_kernel): they live in a buffer of their own, with the first points and first
-    // cells of the systems, and the host has neither grids nor boxes
+    // grids picked on the device (pick_grids_kernel): they live in a buffer of their own, with the first points, first
+    // cells and first pairs of the systems, and the host has neither grids nor boxes
     bool picked = false;
     DeviceBuffer picked_work;
     GridParams* picked_grids = nullptr;
     uint32_t* picked_first_point = nullptr;
     uint32_t* picked_cell_base = nullptr;
+    uint64_t* picked_pair_base = nullptr;
+    bool picked_pairs_there = false;        // the first pairs have been sent (only sorted batches need them)
     PickedGrids* picked_report = nullptr;   // pinned
     int pick_rest = 0;                      // calls left before that is tried again after a batch it is not for
     size_t boxes_of = 0;                    // number of systems whose boxes are kept
@@ -3898,6 +3900,7 @@ bool pick_grids(
     // the set-up of the call before is gone from here on
     setup.valid = false;
     setup.picked = false;
+    setup.picked_pairs_there = false;
     setup.on_device = false;
     setup.kept_on_device = false;
     setup.boxes.clear();
@@ -3925,6 +3928,7 @@ bool pick_grids(
         setup.picked_grids = c.take<GridParams>(n_systems);
         setup.picked_first_point = c.take<uint32_t>(n_systems + 1);
         setup.picked_cell_base = c.take<uint32_t>(n_systems + 1);
+        setup.picked_pair_base = c.take<uint64_t>(n_systems + 1);
         cells_of_system = c.take<uint32_t>(n_systems);
         shapes = c.take<uint32_t>(n_systems);
     };
@@ -4365,7 +4369,7 @@ bool batch_attempt(
         d_cell_base = carver.take<uint32_t>(n_systems + 1);
         d_first_pair = carver.take<unsigned long long>(n_systems + 1);
         d_cells_of_system = carver.take<uint32_t>(n_systems);
-        d_pair_base = carver.take<uint64_t>(try_in_order ? n_systems + 1 : 0);
+        d_pair_base = carver.take<uint64_t>(try_in_order && !setup.picked ? n_systems + 1 : 0);
         image_hits = carver.take<uint64_t>(try_in_order ? hit_words : 0);
         candidate_records = carver.take<CandidateRecord>(try_in_order ? record_slots * ORDERED_CANDIDATES : 0);
         candidates_of_item = carver.take<uint32_t>(try_in_order ? record_slots : 0);
@@ -4378,12 +4382,24 @@ bool batch_attempt(
     carve(carver);
     extras.batch_first_pair_device = d_first_pair;
 
-    if (try_in_order && !(same_setup && setup.on_device && setup.work_generation == extras.work.generation &&
-                          setup.d_pair_base == d_pair_base)) {
+    bool pairs_there = same_setup && setup.on_device && setup.work_generation == extras.work.generation &&
+                       setup.d_pair_base == d_pair_base;
+    if (setup.picked) {
+        d_pair_base = setup.picked_pair_base;
+        pairs_there = setup.picked_pairs_there;
+    }
+    if (try_in_order && !pairs_there) {
+        if (std::getenv("VESIN_HIP_DEBUG") != nullptr) {
+            std::fprintf(stderr, "sorted batch: first pairs of %zu systems go to the device\n", n_systems);
+        }
         HIP_CHECK(hipMemcpyAsync(
             d_pair_base, setup.pair_base.data(), (n_systems + 1) * sizeof(uint64_t), hipMemcpyHostToDevice, stream
         ));
-        setup.d_pair_base = d_pair_base;
+        if (setup.picked) {
+            setup.picked_pairs_there = true;
+        } else {
+            setup.d_pair_base = d_pair_base;
+        }
     }
     const bool already_there = same_setup && setup.on_device && setup.work_generation == extras.work.generation &&
                                setup.d_grids == d_grids &&
