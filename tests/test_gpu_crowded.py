@@ -94,6 +94,39 @@ def test_orders_of_the_points(order, full, capfd, monkeypatch):
     _check(points, box, True, 5.0, full, capfd, monkeypatch)
 
 
+@pytest.mark.parametrize(
+    "labels,n_dense",
+    [
+        ("a run and far ones", 1300), ("a run and far ones", 4500), ("runs near each other and a far one", 1300),
+        ("runs near each other and a far one", 4500), ("powers", 1300), ("powers", 4500), ("images and far ones", 700),
+    ],
+)
+def test_labels_that_clump(labels, n_dense, capfd, monkeypatch):
+    """Original indices of a cell's candidates that are no even spread: nearly all in a small part of the range between
+    the lowest and the highest, which is shared out again, once or several times; the order is the oracle's every time. The
+    other points lie apart, on a lattice. In a long box, two cells wide, points come with their images."""
+    rng = np.random.default_rng(n_dense)
+    images = labels == "images and far ones"
+    # (a bucket of the first sharing covers 98 indices or more; 68 in the long box, of which each comes twice on average)
+    n, cutoff = 70_000 if images else 400_000, 3.0
+    if labels in ("a run and far ones", "images and far ones"):
+        dense = np.concatenate([np.arange(n_dense - 3), [n // 2, n - 2, n - 1]])
+    elif labels == "powers":
+        dense = np.unique(np.exp(np.linspace(0.0, np.log(n - 1.0), 4 * n_dense)).astype(int))
+        dense = rng.permutation(dense)[:n_dense]
+    else:
+        dense = np.concatenate([np.arange(n_dense // 2), 5 + n_dense // 2 + np.arange(n_dense - n_dense // 2 - 1), [n - 1]])
+    others = np.setdiff1d(np.arange(n), dense)
+    side = 2 if images else int(np.ceil(len(others) ** (1 / 3)))
+    grid = np.arange(len(others))
+    lattice = 3.5 * np.stack([grid // side // side, grid // side % side, grid % side], axis=1)
+    box = np.diag([15.0 + lattice[:, 0].max() + 5.0, *([7.0] * 2 if images else [15.0 + 3.5 * side + 5.0] * 2)])
+    points = np.empty((n, 3))
+    points[others] = lattice + ([15.0, 0.5, 0.5] if images else 15.0)
+    points[dense] = np.array([8.9, 7.0, 7.0] if images else [8.9] * 3) * rng.random((len(dense), 3))
+    _check(points, box, images, cutoff, False, capfd, monkeypatch)
+
+
 def test_coincident_points_and_shifts_beyond_the_key(capfd, monkeypatch):
     points, box = _liquid(900, 9.0, 8)
     points[100:200] = points[0:100]

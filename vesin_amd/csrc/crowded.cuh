@@ -37,6 +37,9 @@ constexpr int CROWDED_BLOCK = CROWDED_WAVES * WAVE;
 constexpr uint32_t CROWDED_SMALL = 2048;   // candidates that the usual sorting kernel takes (29 KB of LDS)
 constexpr uint32_t CROWDED_LARGE = 8192;   // and the one for the most crowded cells (115 KB)
 constexpr int CROWDED_SORT_BLOCK = 512;    // threads of the latter
+constexpr uint32_t CROWDED_BUCKET = 64;    // keys of a bucket that is left as it is
+constexpr uint32_t CROWDED_LEVELS = 6;     // times that the buckets are shared out again at most
+static_assert(CROWDED_BUCKET >= MAX_ENTRIES, "the images of one point share a bucket, whatever it is shared out into");
 
 /// A candidate, in the order of (original index, shift).
 struct CrowdedCandidate {
@@ -190,9 +193,13 @@ __global__ __launch_bounds__(CROWDED_BLOCK) void crowded_measure_kernel(CrowdedA
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// SORT: bound by LDS latency and atomics. Buckets of about two candidates' indices, so that a key meets few others; the
-// kernel for most cells and the one for the most crowded are apart because the latter's LDS leaves room for one workgroup
-// per compute unit (clusters of 500,000 points: 209 + 119 us).
+// SORT: bound by LDS latency and atomics. Buckets of about two candidates' indices, so that a key meets few others, where
+// the indices are spread evenly; where they clump (a blob numbered in one go and some points of another, a solute numbered
+// before its solvent) nearly all would share a few buckets and be compared one by one, and the range of every bucket is
+// shared out again until none holds more than 64. The kernel for most cells and the one for the most crowded are apart
+// because the latter's LDS leaves room for one workgroup per compute unit (clusters of 500,000 points without and with sharing
+// out again: in no order 209 + 121 and 211 + 126 us, blobs numbered one after the other, each along x, 0.2 % of the points
+// before them all 645 + 158 and 346 + 163 us; per call of 2,000,000 points 5.65 and 5.66 ms, 9.41 and 6.06 ms).
 
 template <uint32_t CAPACITY, int THREADS>
 struct CrowdedSortShared {
@@ -203,6 +210,7 @@ struct CrowdedSortShared {
     uint32_t biased[CAPACITY];
     uint32_t first[BUCKETS + 1]; // candidates per bucket, then the first of every bucket
     uint32_t lowest, highest;
+    uint32_t wide_bucket; // some bucket holds more than CROWDED_BUCKET
     uint32_t wave_total[THREADS / WAVE];
 };
 
@@ -246,6 +254,7 @@ __global__ __launch_bounds__(THREADS) void crowded_sort_kernel(CrowdedArgs args,
         if (threadIdx.x == 0) {
             sh.lowest = 0xFFFFFFFFu;
             sh.highest = 0;
+            sh.wide_bucket = 0;
         }
         for (uint32_t b = threadIdx.x; b <= BUCKETS; b += THREADS) {
             sh.first[b] = 0;
@@ -295,43 +304,93 @@ __global__ __launch_bounds__(THREADS) void crowded_sort_kernel(CrowdedArgs args,
         auto bucket_of = [&](uint32_t i) {
             return min(BUCKETS - 1, static_cast<uint32_t>(static_cast<float>(i - lowest) * per_index));
         };
-        uint32_t arrival[OWN];
+        uint32_t bucket[OWN], arrival[OWN];
 #pragma unroll
         for (uint32_t u = 0; u < OWN; u++) {
-            const uint32_t k = u * THREADS + threadIdx.x;
-            arrival[u] = k < n ? atomicAdd(&sh.first[bucket_of(index[u])], 1u) : 0u;
+            bucket[u] = bucket_of(index[u]);
         }
-        __syncthreads();
-        uint32_t in_bucket[OWN_BUCKETS];
-        uint32_t mine = 0;
+        uint32_t level = 0;
+        for (;; level++) {
 #pragma unroll
-        for (uint32_t b = 0; b < OWN_BUCKETS; b++) {
-            in_bucket[b] = sh.first[OWN_BUCKETS * threadIdx.x + b];
-            mine += in_bucket[b];
-        }
-        const uint32_t through = wave_inclusive_scan(mine);
-        if (lane == WAVE - 1) {
-            sh.wave_total[wave] = through;
-        }
-        __syncthreads();
-        uint32_t before = through - mine;
-        for (uint32_t w = 0; w < wave; w++) {
-            before += sh.wave_total[w];
-        }
+            for (uint32_t u = 0; u < OWN; u++) {
+                const uint32_t k = u * THREADS + threadIdx.x;
+                arrival[u] = k < n ? atomicAdd(&sh.first[bucket[u]], 1u) : 0u;
+            }
+            __syncthreads();
+            uint32_t in_bucket[OWN_BUCKETS];
+            uint32_t mine = 0;
+            uint32_t most = 0;
 #pragma unroll
-        for (uint32_t b = 0; b < OWN_BUCKETS; b++) {
-            sh.first[OWN_BUCKETS * threadIdx.x + b] = before;
-            before += in_bucket[b];
-        }
-        if (threadIdx.x == THREADS - 1) {
-            sh.first[BUCKETS] = before; // = n
+            for (uint32_t b = 0; b < OWN_BUCKETS; b++) {
+                in_bucket[b] = sh.first[OWN_BUCKETS * threadIdx.x + b];
+                mine += in_bucket[b];
+                most = max(most, in_bucket[b]);
+            }
+            const uint32_t through = wave_inclusive_scan(mine);
+            if (lane == WAVE - 1) {
+                sh.wave_total[wave] = through;
+            }
+            if (most > CROWDED_BUCKET) {
+                sh.wide_bucket = 1;
+            }
+            __syncthreads();
+            const bool share_again = uniform(sh.wide_bucket) != 0 && level < CROWDED_LEVELS;
+            uint32_t before = through - mine;
+            for (uint32_t w = 0; w < wave; w++) {
+                before += sh.wave_total[w];
+            }
+#pragma unroll
+            for (uint32_t b = 0; b < OWN_BUCKETS; b++) {
+                sh.first[OWN_BUCKETS * threadIdx.x + b] = before;
+                before += in_bucket[b];
+            }
+            if (threadIdx.x == THREADS - 1) {
+                sh.first[BUCKETS] = before; // = n
+            }
+            if (!share_again) {
+                break;
+            }
+            // Some bucket holds many: every bucket's own range of indices is shared out again among as many places as it
+            // has keys, which gives an estimate of every key's rank, and the ranks two by two are the new buckets.
+            uint32_t* const low = sh.index;
+            uint32_t* const high = sh.at;
+            for (uint32_t b = threadIdx.x; b < BUCKETS; b += THREADS) {
+                low[b] = 0xFFFFFFFFu;
+                high[b] = 0;
+            }
+            __syncthreads();
+#pragma unroll
+            for (uint32_t u = 0; u < OWN; u++) {
+                if (u * THREADS + threadIdx.x < n) {
+                    atomicMin(&low[bucket[u]], index[u]);
+                    atomicMax(&high[bucket[u]], index[u]);
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (uint32_t u = 0; u < OWN; u++) {
+                if (u * THREADS + threadIdx.x < n) {
+                    const uint32_t first = sh.first[bucket[u]];
+                    const uint32_t keys = sh.first[bucket[u] + 1] - first;
+                    const uint32_t lowest_here = low[bucket[u]];
+                    const float per_place = static_cast<float>(keys) / (static_cast<float>(high[bucket[u]] - lowest_here) + 1.0f);
+                    bucket[u] = (first + min(keys - 1, static_cast<uint32_t>(static_cast<float>(index[u] - lowest_here) * per_place))) / 2;
+                }
+            }
+            __syncthreads();
+            for (uint32_t b = threadIdx.x; b <= BUCKETS; b += THREADS) {
+                sh.first[b] = 0;
+            }
+            if (threadIdx.x == 0) {
+                sh.wide_bucket = 0;
+            }
+            __syncthreads();
         }
         __syncthreads();
 #pragma unroll
         for (uint32_t u = 0; u < OWN; u++) {
-            const uint32_t k = u * THREADS + threadIdx.x;
-            if (k < n) {
-                const uint32_t slot = sh.first[bucket_of(index[u])] + arrival[u];
+            if (u * THREADS + threadIdx.x < n) {
+                const uint32_t slot = sh.first[bucket[u]] + arrival[u];
                 sh.index[slot] = index[u];
                 sh.at[slot] = at[u];
                 sh.biased[slot] = biased[u];
@@ -342,10 +401,19 @@ __global__ __launch_bounds__(THREADS) void crowded_sort_kernel(CrowdedArgs args,
         for (uint32_t slot = threadIdx.x; slot < n; slot += THREADS) {
             const uint32_t own = sh.index[slot];
             const uint32_t own_biased = sh.biased[slot];
-            const uint32_t bucket = bucket_of(own);
-            const uint32_t end = sh.first[bucket + 1];
-            uint32_t place = sh.first[bucket];
-            for (uint32_t other = sh.first[bucket]; other < end; other++) {
+            uint32_t own_bucket = 0;
+            if (level == 0) {
+                own_bucket = bucket_of(own);
+            } else {
+                // the last bucket that starts at the slot or before it
+#pragma unroll
+                for (uint32_t step = BUCKETS / 2; step > 0; step /= 2) {
+                    own_bucket += sh.first[own_bucket + step] <= slot ? step : 0u;
+                }
+            }
+            const uint32_t end = sh.first[own_bucket + 1];
+            uint32_t place = sh.first[own_bucket];
+            for (uint32_t other = place; other < end; other++) {
                 const uint32_t theirs = sh.index[other];
                 // (the images of one point differ in their shifts)
                 place += theirs < own || (theirs == own && sh.biased[other] < own_biased) ? 1u : 0u;
