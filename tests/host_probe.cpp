@@ -170,6 +170,27 @@ extern "C" void probe_candidate_lifetime(const unsigned char* outdated, size_t n
     }
 }
 
+/// The room of the search for crowded cells over a sequence of calls on as many points: call k counts `counted[2k]` units of
+/// candidates and `counted[2k + 1]` of columns. `room[2k]`, `room[2k + 1]` receive the room it ran in (0, 0: it did not),
+/// `counts[k]` how often it counted without knowing the room. The driver's use of the functions is reproduced.
+extern "C" void probe_crowded_room(size_t n_points, const size_t* counted, size_t n_calls, size_t* room, int* counts) {
+    vesin_hip::CrowdedRoom kept;
+    for (size_t k = 0; k < n_calls; k++) {
+        const vesin_hip::CrowdedRoom found = {counted[2 * k], counted[2 * k + 1]};
+        vesin_hip::CrowdedRoom now = kept;
+        counts[k] = 0;
+        if (now.candidate_units < found.candidate_units || now.column_units < found.column_units) {
+            counts[k] = 1;
+            now = vesin_hip::crowded_room_for(n_points, found);
+        }
+        room[2 * k] = now.candidate_units;
+        room[2 * k + 1] = now.column_units;
+        if (now.candidate_units > 0) {
+            kept = vesin_hip::crowded_room_kept(n_points, now, found);
+        }
+    }
+}
+
 extern "C" int probe_ordered_records_fit(size_t n_points, size_t record_bytes) {
     return vesin_hip::ordered_records_fit(n_points, record_bytes) ? 1 : 0;
 }

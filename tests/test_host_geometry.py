@@ -35,6 +35,8 @@ def probe(tmp_path_factory):
     lib.probe_box_guess.restype = None
     lib.probe_ordered_records_fit.argtypes = [ctypes.c_size_t, ctypes.c_size_t]
     lib.probe_ordered_records_fit.restype = ctypes.c_int
+    lib.probe_crowded_room.argtypes = [ctypes.c_size_t, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_void_p]
+    lib.probe_crowded_room.restype = None
     lib.probe_prefilter.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_double, ctypes.c_size_t, ctypes.c_void_p,
                                     ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
     lib.probe_wait_rest.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
@@ -450,6 +452,38 @@ def test_work_memory_of_the_in_order_search_is_bounded(probe):
     # small systems always fit
     assert probe.probe_ordered_records_fit(216, 2048 * 12288)
     assert probe.probe_ordered_records_fit(1, 64 * 12288)
+
+
+def run_crowded_room(probe, n_points, counted):
+    counted = np.ascontiguousarray(counted, dtype=np.uint64)
+    room = np.zeros_like(counted)
+    counts = np.zeros(len(counted), dtype=np.int32)
+    probe.probe_crowded_room(n_points, counted.ctypes.data, len(counted), room.ctypes.data, counts.ctypes.data)
+    return [tuple(r) for r in room.tolist()], counts.tolist()
+
+
+def test_room_of_the_search_for_crowded_cells(probe):
+    # 2 GiB + 1536 bytes per point; 512 bytes per unit of candidates, 256 per unit of columns
+    n_points = 100_000
+    allowed = (2147483648 + 1536 * n_points) // 256
+    ample = lambda units: units + units // 8 + 64  # noqa: E731
+    # an eighth more than what was counted, kept while the system grows into it, and through a smaller one
+    first, grown = (1000, 8000), (1100, 9000)
+    assert run_crowded_room(probe, n_points, [first, first, grown, grown, (10, 10), grown]) == (
+        [(ample(1000), ample(8000)), (ample(1000), ample(8000)), (ample(1000), ample(8000))] + [(ample(1100), ample(9000))] * 3,
+        [1, 0, 0, 0, 0, 0],
+    )
+    # what was counted fits, an eighth more does not: room for just that, also the next time
+    tight = (100, allowed - 200)
+    assert run_crowded_room(probe, n_points, [tight, tight]) == ([tight, tight], [1, 0])
+    # it does not fit: not covered, and what is kept of the calls before is as good as before
+    beyond = (100, allowed - 199)
+    rooms, counts = run_crowded_room(probe, n_points, [first, beyond, first, beyond, first])
+    assert rooms == [(ample(1000), ample(8000)), (0, 0)] * 2 + [(ample(1000), ample(8000))] and counts == [1, 1, 0, 1, 0]
+    # a system that comes near the room it has, where the room of both would be too much: the room it had is kept
+    half = allowed // 4
+    rooms, counts = run_crowded_room(probe, n_points, [(half, 100), (100, half * 2 - 1000), (half, 100)])
+    assert all(2 * c + k <= allowed for c, k in rooms) and (0, 0) not in rooms
 
 
 def run_prefilter(probe, box, periodic, cutoff, n_points, lo, hi, single_cell=False):

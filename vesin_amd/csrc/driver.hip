@@ -1074,8 +1074,7 @@ struct HipExtras {
     int in_order_rest = 0;            // calls left before the in-order search is tried again on a system it did not cover
     int crowded_rest = 0;             // the same for the in-order search for crowded cells (crowded.cuh)
     size_t crowded_points = 0;        // the last system that search covered: its number of points ...
-    size_t crowded_candidate_units = 0; // ... and the room its candidates and hit columns took, in units of 64
-    size_t crowded_column_units = 0;
+    CrowdedRoom crowded_room;         // ... and the room for its candidates and hit columns
     int one_launch_rest = 0;          // calls left before a small system is tried in one launch again
     WaitRest meeting_rest;            // ... after workgroups of that launch gave up waiting for the others
     WaitRest chain_rest;              // the same for the chain of the single-pass search (rows in work-item order)
@@ -2692,29 +2691,25 @@ bool compute(
         // number of tiles, known on the device, may be far below its bound where most cells are empty)
         const uint32_t tile_blocks = static_cast<uint32_t>(std::min<size_t>((tiles_bound + N_XCD - 1) / N_XCD * N_XCD, 16384));
         const uint32_t measure_blocks = static_cast<uint32_t>(std::min<size_t>((tiles_bound + CROWDED_BLOCK - 1) / CROWDED_BLOCK, 4096));
-        // The room that candidates and hit columns take is what the call before on as many points found, and an eighth
-        // more; a first call (and one that finds too little room) has it counted first.
-        size_t candidate_units = extras.crowded_points == n_points ? extras.crowded_candidate_units : 0;
-        size_t column_units = extras.crowded_points == n_points ? extras.crowded_column_units : 0;
-        bool known = candidate_units > 0;
+        // The room that candidates and hit columns take is what the call before on as many points left (policy.hpp); a
+        // first call (and one that finds too little room) has it counted first.
+        static_assert(WAVE == 64 && sizeof(CrowdedCandidate) == 8, "policy.hpp and the kernels agree on the bytes of the records");
+        CrowdedRoom room = extras.crowded_points == n_points ? extras.crowded_room : CrowdedRoom{};
+        bool known = room.candidate_units > 0;
         bool covered = false;
         for (int attempt = 0; attempt < 3; attempt++) {
-            const size_t record_bytes = candidate_units * WAVE * sizeof(CrowdedCandidate) + column_units * WAVE * sizeof(uint32_t);
-            if (candidate_units > 0xFFFFFFF0ull || column_units > 0xFFFFFFF0ull || !ordered_records_fit(n_points, record_bytes)) {
-                break;
-            }
             auto carve_crowded = [&](Carver& c) {
                 cargs.cells = c.take<CrowdedCell>(tiles_bound);
-                cargs.candidates = c.take<CrowdedCandidate>(candidate_units * WAVE);
-                cargs.columns = c.take<uint32_t>(column_units * WAVE);
+                cargs.candidates = c.take<CrowdedCandidate>(room.candidate_units * WAVE);
+                cargs.columns = c.take<uint32_t>(room.column_units * WAVE);
             };
             Carver crowded_measure(nullptr);
             carve_crowded(crowded_measure);
             extras.sort_work.reserve(crowded_measure.used);
             Carver crowded_carver(extras.sort_work.ptr);
             carve_crowded(crowded_carver);
-            cargs.candidate_units = static_cast<uint32_t>(candidate_units);
-            cargs.column_units = static_cast<uint32_t>(column_units);
+            cargs.candidate_units = static_cast<uint32_t>(room.candidate_units);
+            cargs.column_units = static_cast<uint32_t>(room.column_units);
             const bool early_write = known && extras.capacity > 0;
             auto launch_write = [&]() {
                 auto kernel = cargs.out.vectors != nullptr ? crowded_write_kernel<true> : crowded_write_kernel<false>;
@@ -2764,13 +2759,14 @@ bool compute(
             if (found.first_bad_coordinate != 0xFFFFFFFFu) {
                 non_finite_error(points, found.first_bad_coordinate);
             }
-            const size_t candidate_units_found = static_cast<size_t>(found.found.used & 0xFFFFFFFFull);
-            const size_t column_units_found = static_cast<size_t>(found.found.used >> 32);
+            const CrowdedRoom counted = {
+                static_cast<size_t>(found.found.used & 0xFFFFFFFFull), static_cast<size_t>(found.found.used >> 32)
+            };
             if (std::getenv("VESIN_HIP_DEBUG") != nullptr) {
                 std::fprintf(
                     stderr, "crowded search: rows %llu, most candidates of a cell %u, unsuitable %u, %zu + %zu units of candidates and columns, room for %zu + %zu\n",
-                    found.total_rows, found.found.max_candidates, found.found.unsuitable, candidate_units_found, column_units_found,
-                    candidate_units, column_units
+                    found.total_rows, found.found.max_candidates, found.found.unsuitable, counted.candidate_units, counted.column_units,
+                    room.candidate_units, room.column_units
                 );
             }
             if (found.found.unsuitable != 0 || found.found.max_candidates > CROWDED_LARGE) {
@@ -2781,14 +2777,15 @@ bool compute(
                 break;
             }
             if (!known || found.found.overflow != 0) {
-                candidate_units = candidate_units_found + candidate_units_found / 8 + 64;
-                column_units = column_units_found + column_units_found / 8 + 64;
+                room = crowded_room_for(n_points, counted);
+                if (room.candidate_units == 0) {
+                    break;
+                }
                 known = true;
                 continue;
             }
             extras.crowded_points = pays ? n_points : 0; // (0: the next call counts, and decides, before it does anything else)
-            extras.crowded_candidate_units = std::max(candidate_units, candidate_units_found + candidate_units_found / 8 + 64);
-            extras.crowded_column_units = std::max(column_units, column_units_found + column_units_found / 8 + 64);
+            extras.crowded_room = crowded_room_kept(n_points, room, counted);
             const size_t total = found.total_rows;
             check_pair_limit(total);
             if (!(early_write && total <= early_capacity)) {

@@ -190,6 +190,38 @@ inline bool ordered_records_fit(size_t n_points, size_t record_bytes) {
     return static_cast<double>(record_bytes) <= allowed;
 }
 
+/// Room for what the search for crowded cells leaves between its passes, in units of 64: candidates of every cell (8 bytes
+/// each), hit columns of every tile (4 bytes per candidate).
+struct CrowdedRoom {
+    size_t candidate_units = 0; // 0: not known, or none
+    size_t column_units = 0;
+};
+
+inline bool crowded_room_fits(size_t n_points, const CrowdedRoom& room) {
+    return room.candidate_units <= 0xFFFFFFF0ull && room.column_units <= 0xFFFFFFF0ull &&
+           ordered_records_fit(n_points, 64 * (8 * room.candidate_units + 4 * room.column_units));
+}
+
+/// The room for a system whose candidates and columns were counted: an eighth more than that, so that the next frame finds
+/// room too, or just that where the rule allows no more. None when not even that fits.
+inline CrowdedRoom crowded_room_for(size_t n_points, const CrowdedRoom& counted) {
+    const CrowdedRoom ample = {
+        counted.candidate_units + counted.candidate_units / 8 + 64, counted.column_units + counted.column_units / 8 + 64
+    };
+    return crowded_room_fits(n_points, ample) ? ample : crowded_room_fits(n_points, counted) ? counted : CrowdedRoom{};
+}
+
+/// The room that the next call on as many points starts from: what this call had, and more where its system comes near
+/// that, as long as the two together fit.
+inline CrowdedRoom crowded_room_kept(size_t n_points, const CrowdedRoom& had, const CrowdedRoom& counted) {
+    const CrowdedRoom wanted = crowded_room_for(n_points, counted);
+    const CrowdedRoom both = {
+        had.candidate_units > wanted.candidate_units ? had.candidate_units : wanted.candidate_units,
+        had.column_units > wanted.column_units ? had.column_units : wanted.column_units
+    };
+    return crowded_room_fits(n_points, both) ? both : had;
+}
+
 /// Whether the in-order search for crowded cells (crowded.cuh) is the faster way to a sorted list than the radix sort. It
 /// gives every tile workgroups of its own, whatever the tile holds; the radix sort's time follows the rows and has a floor
 /// of 0.2 ms. Per call, radix sort -> that search, cutoff 5, liquids of 300,000 points with 2 / 3 / 4 / 6 / 8 points per cell:
