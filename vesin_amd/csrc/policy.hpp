@@ -258,11 +258,19 @@ inline unsigned int ordered_write_split(size_t n_points, size_t tiles_before) {
 /// Whether the writing pass gives every tile a workgroup that brings the candidates' coordinates to LDS (write_tile.cuh),
 /// from the same number. Bringing them pays when enough rows are made of them: 10 points per tile, or 16 when vectors are
 /// returned (their way through LDS leaves room for fewer workgroups). Candidates beyond 704 come in a second chunk,
-/// which costs more than it gives: 665 on average at most, so that few tiles have more. Writing pass, kernel with a wave
-/// per tile -> this, cutoff 5, liquids of 300,000 points with 8 / 10 / 16 / 20 / 28 points per cell: full lists P S d 220 ->
-/// 227, 228 -> 207, 307 -> 250, 328 -> 277, 388 -> 421 us; half lists P S d D 206 -> 299, 211 -> 278, 288 -> 260, 298 ->
-/// 291, 350 -> 439 us; 60,000 points with 6 / 10 / 16 / 20: full 57 -> 56, 68 -> 50, 81 -> 60, 89 -> 70 us, half 54 -> 74,
-/// 63 -> 64, 79 -> 66, 87 -> 70 us.
+/// which costs more than it gives: 665 on average at most, so that few tiles have more. Writing pass, the other kernel with
+/// a wave per tile -> this, cutoff 5, liquids of 300,000 points with 8 / 10 / 16 / 20 / 28 points per cell: full lists P S d
+/// 220 -> 227, 228 -> 207, 307 -> 250, 328 -> 277, 388 -> 421 us; half lists P S d D 206 -> 299, 211 -> 278, 288 -> 260,
+/// 298 -> 291, 350 -> 439 us; 60,000 points with 6 / 10 / 16 / 20: full 57 -> 56, 68 -> 50, 81 -> 60, 89 -> 70 us, half 54 ->
+/// 74, 63 -> 64, 79 -> 66, 87 -> 70 us.
+///
+/// The same against the kernel it takes the place of (ordered_write_split: four waves per tile from 3,482 to 20,480 tiles, one
+/// below), cutoff 5, 2,197 / 4,096 / 9,261 / 19,683 cells; cutoffs 4 and 6 differ by 1-2 %. Liquids with 20 points per cell:
+/// half P S d 70 -> 42, 85 -> 66, 175 -> 131, 372 -> 260 us; half P S d D 70 -> 60, 100 -> 98, 196 -> 193, 394 -> 389; full
+/// P S d D 105 -> 84, 150 -> 147, 294 -> 308, 597 -> 609. Lattices in order, 22.4 per cell: half P S d D 64 -> 56, 111 -> 104,
+/// 224 -> 211, 405 -> 393; full P S d D 99 -> 79, 191 -> 167, 380 -> 343, 711 -> 643. The one shape that loses (full lists with
+/// vectors, points in no order, 9,000 to 20,480 tiles: up to 5 % of the pass, 1 % of a call) cannot be told from the one
+/// that wins a tenth, the same list of points in order.
 inline bool ordered_write_by_tiles(size_t n_points, size_t n_cells, size_t tiles_before, size_t stencil_cells, bool vectors) {
     if (tiles_before == 0 || n_cells == 0) {
         return false;
