@@ -69,7 +69,7 @@ def test_molecules_of_every_size(most, full, is_sorted, capfd, monkeypatch):
         expected_here = most <= 64 or is_sorted
         assert ("batch of free molecules" in report) == expected_here, report
         if expected_here:
-            assert f"{most if most <= 64 else 256} lanes per system" in report
+            assert f"{most if most <= 16 else 64 if most <= 64 else 256} lanes per system" in report
             check_in_order(lists, molecules, 2.4, full, f"call {call}")
         else:
             for s, rows in enumerate(lists):

@@ -3415,9 +3415,8 @@ bool molecules_batch(
     uint32_t* d_first_point = nullptr;
     uint64_t* d_first_pair = nullptr;
     uint64_t* scan_scratch = nullptr;
-    // lanes per system: the next power of two from the largest system on, eight at least; a workgroup beyond 64
-    const int lanes = most_points <= 8 ? 8 : most_points <= 16 ? 16 : most_points <= 32 ? 32
-                    : most_points <= MOLECULE_GROUP_POINTS ? 64 : MOLECULE_BLOCK;
+    // lanes per system, by the largest one: a lane per point up to 16, a wave up to 64, a workgroup beyond
+    const int lanes = most_points <= 8 ? 8 : most_points <= 16 ? 16 : most_points <= MOLECULE_GROUP_POINTS ? WAVE : MOLECULE_BLOCK;
     const bool wide = lanes == MOLECULE_BLOCK;
     uint64_t* d_first_row = nullptr;
     auto carve = [&](Carver& c) {
@@ -3463,7 +3462,7 @@ bool molecules_batch(
 
     args.total_points = static_cast<uint32_t>(n_points);
     args.first_row = d_first_row;
-    const size_t per_block = wide ? 1 : static_cast<size_t>(MOLECULE_BLOCK / WAVE) * (lanes >= 32 ? 1 : WAVE / lanes);
+    const size_t per_block = wide ? 1 : static_cast<size_t>(MOLECULE_BLOCK / lanes);
     const unsigned blocks = static_cast<unsigned>((n_systems + per_block - 1) / per_block);
     auto launch = [&](bool write) {
         const dim3 grid(blocks), block(MOLECULE_BLOCK);
@@ -3474,8 +3473,7 @@ bool molecules_batch(
         case 17: hipLaunchKernelGGL((molecules_kernel<8, true>), grid, block, 0, stream, args); break;
         case 32: hipLaunchKernelGGL((molecules_kernel<16, false>), grid, block, 0, stream, args); break;
         case 33: hipLaunchKernelGGL((molecules_kernel<16, true>), grid, block, 0, stream, args); break;
-        case 64:
-        case 128: hipLaunchKernelGGL((molecules_pairs_kernel<false>), grid, block, 0, stream, args); break;
+        case 2 * WAVE: hipLaunchKernelGGL((molecules_pairs_kernel<false>), grid, block, 0, stream, args); break;
         default: hipLaunchKernelGGL((molecules_pairs_kernel<true>), grid, block, 0, stream, args); break;
         }
     };

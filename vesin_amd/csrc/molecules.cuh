@@ -57,6 +57,7 @@ struct MoleculeArgs {
 
 template <int G, bool WRITE>
 __global__ __launch_bounds__(MOLECULE_BLOCK) void molecules_kernel(MoleculeArgs a) {
+    static_assert(G < WAVE, "a group's lanes are a part of a wave");
     constexpr int GROUPS = WAVE / G;
     const uint32_t lane = static_cast<uint32_t>(lane_id());
     const uint32_t group = lane / G;
@@ -109,7 +110,7 @@ __global__ __launch_bounds__(MOLECULE_BLOCK) void molecules_kernel(MoleculeArgs 
     rounds = uniform(rounds);
 
     const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (WAVE - lane));              // the lanes before this one
-    const uint64_t of_group = (G == WAVE ? ~0ull : ((1ull << G) - 1ull)) << (group * G); // the lanes of this group
+    const uint64_t of_group = ((1ull << G) - 1ull) << (group * G);                       // the lanes of this group
     uint64_t row = WRITE && exists ? a.first_pair[system] : 0;
     uint32_t rows = 0;
     for (uint32_t i = 0; i < rounds; i++) {
