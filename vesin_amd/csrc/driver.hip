@@ -2631,10 +2631,10 @@ bool compute(
             std::fprintf(
                 stderr,
                 "in-order search: rows %llu, most rows of a point %u, most candidates of a tile %u, unsuitable %u, "
-                "candidates of %u tiles ordered by window and of %u by buckets, %u tiles written by %u waves each and counted by %u: %s\n",
+                "candidates of %u tiles ordered by window and of %u by buckets, %u tiles written by %u waves each%s and counted by %u: %s\n",
                 found.total_rows, found.found.max_rows, found.found.max_candidates, found.found.unsuitable,
-                found.found.windowed, found.found.bucketed, found.n_tiles, oargs.write_split, oargs.count_split,
-                suitable ? "used" : "left to the radix sort"
+                found.found.windowed, found.found.bucketed, found.n_tiles, oargs.write_split,
+                tile_writer ? " (candidates in LDS)" : "", oargs.count_split, suitable ? "used" : "not covered"
             );
         }
         if (suitable) {
