@@ -40,6 +40,13 @@ def _rows(calculator, batch, periodic=True, sort=False):
     return rows + [first_pair]
 
 
+def _rows_and_where(calculator, batch, capfd, periodic=True, sort=False):
+    """The rows, and whether their grids were picked on the device."""
+    capfd.readouterr()
+    rows = _rows(calculator, batch, periodic, sort)
+    return rows, "from grids picked on the device" in capfd.readouterr().err
+
+
 def _same(one, other):
     for a, b in zip(one, other):
         assert np.array_equal(a, b)
@@ -47,19 +54,23 @@ def _same(one, other):
 
 @pytest.mark.parametrize("full,sort", [(True, True), (False, True), (True, False), (False, False)])
 @pytest.mark.parametrize("algorithm", ["auto", "cell_list", "brute_force"])
-def test_lists(algorithm, full, sort, monkeypatch):
+def test_lists(algorithm, full, sort, capfd, monkeypatch):
     """Other systems in every call, then the same ones again (which starts from the grids of the call before), then
     other boxes around as many points."""
     batches = [_batch(32, 1), _batch(300, 2, empty=True), _batch(1030, 3, 1, 12, 0.02)]
     batches += [batches[-1], (batches[-1][0], batches[-1][1], 1.05 * batches[-1][2]), _batch(31, 4), _batch(400, 5, 30, 200)]
+    monkeypatch.setenv("VESIN_HIP_DEBUG", "1")
     results = {}
     for where in ("device", "host"):
         if where == "host":
             monkeypatch.setenv("VESIN_HIP_GRIDS", "host")
         calculator = NeighborList(cutoff=3.5, full_list=full, sorted=sort, algorithm=algorithm)
-        results[where] = [_rows(calculator, batch, sort=not sort) for batch in batches]
-    for one, other in zip(results["device"], results["host"]):
+        results[where] = [_rows_and_where(calculator, batch, capfd, sort=not sort) for batch in batches]
+    for (one, _), (other, _) in zip(results["device"], results["host"]):
         _same(one, other)
+    # (not for the batch of the call before, nor for fewer than 32 systems)
+    assert [picked for _, picked in results["device"]] == [True, True, True, False, True, False, True]
+    assert not any(picked for _, picked in results["host"])
 
 
 @pytest.mark.parametrize("sort", [True, False])
@@ -76,9 +87,11 @@ def test_a_single_system_in_between(sort):
             _same(_rows(calculator, batch, sort=not sort), expected)
 
 
-def test_open_directions_and_boxes_without_an_inverse(monkeypatch):
+def test_open_directions_and_boxes_without_an_inverse(capfd, monkeypatch):
+    """A batch with an open direction has its grids picked on the host, and so have the next 64 new ones."""
     import torch
 
+    monkeypatch.setenv("VESIN_HIP_DEBUG", "1")
     batch = _batch(300, 8)
     periodic = np.ones((300, 3), dtype=bool)
     periodic[17] = [True, False, True]
@@ -88,9 +101,12 @@ def test_open_directions_and_boxes_without_an_inverse(monkeypatch):
     expected, all_periodic = _rows(on_host, batch, torch.tensor(periodic)), _rows(on_host, batch)
     monkeypatch.delenv("VESIN_HIP_GRIDS")
     calculator = NeighborList(cutoff=3.5, full_list=True, sorted=True)
+    _same(_rows(calculator, batch), all_periodic)
     for _ in range(2):
-        _same(_rows(calculator, batch, torch.tensor(periodic)), expected)
-        _same(_rows(calculator, batch), all_periodic)
+        for flags, right in ((torch.tensor(periodic), expected), (True, all_periodic)):
+            rows, picked = _rows_and_where(calculator, batch, capfd, flags)
+            _same(rows, right)
+            assert not picked
     for bad, message in ((0.0, "not invertible"), (1e-3, "too large for this box")):
         calculator = NeighborList(cutoff=3.5, full_list=True, sorted=True)
         boxes = batch[2].copy()

@@ -3972,6 +3972,9 @@ bool pick_grids(
     setup.boxes_of = n_systems;
     setup.picked = true;
     setup.valid = true;
+    if (std::getenv("VESIN_HIP_DEBUG") != nullptr) {
+        std::fprintf(stderr, "batch: %llu cells of %zu systems from grids picked on the device\n", found.total_cells, n_systems);
+    }
     return true;
 }
 
