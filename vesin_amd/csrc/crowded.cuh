@@ -17,9 +17,10 @@
 // A point may have any number of rows; a cell at most CROWDED_LARGE candidates (their sort takes the LDS of a compute
 // unit then). Beyond that, and for shifts or wraps beyond +-255, the host falls back to the radix sort.
 //
-// Measured per call, radix sort -> this: 500,000 points in 50 clusters (82 M rows, P d) 12.7 -> 1.42 ms, (P S d D) 17.9 ->
-// 2.27 ms; 200,000 atoms of diamond, cutoff 6.5 (1480 candidates per tile, P S d) 6.04 -> 1.04 ms; 13,824 atoms, cutoff 5.5
-// 358 -> 167 us; a liquid of 20,000 points, cutoff 7, 649 -> 208 us; 2,000 points, cutoff 7, 180 -> 147 us. On systems that
+// Measured per call, full lists, radix sort -> this: 500,000 points in 50 clusters (82 M rows, P d) 13.2 -> 1.44 ms, (P S d D)
+// 18.5 -> 2.35 ms; 195,112 atoms of diamond, cutoff 6.5 (1480 candidates per tile, P S d) 6.10 -> 1.06 ms; 13,824 atoms, cutoff
+// 5.5, 378 -> 171 us; liquids of 0.1 points per unit of volume, cutoff 7: 20,000 points 560 -> 182 us, 2,000 points 216 -> 152
+// us. On systems that
 // the usual in-order search covers it is the slower one, its passes follow each other where that one sorts beside its
 // counting (1,000,000 atoms of diamond 1.81 against 2.30 ms, 100,000 points of a liquid 274 against 430 us).
 //
@@ -198,8 +199,8 @@ __global__ __launch_bounds__(CROWDED_BLOCK) void crowded_measure_kernel(CrowdedA
 // before its solvent) nearly all would share a few buckets and be compared one by one, and the range of every bucket is
 // shared out again until none holds more than 64. The kernel for most cells and the one for the most crowded are apart
 // because the latter's LDS leaves room for one workgroup per compute unit (clusters of 500,000 points without and with sharing
-// out again: in no order 209 + 121 and 211 + 126 us, blobs numbered one after the other, each along x, 0.2 % of the points
-// before them all 645 + 158 and 346 + 163 us; per call of 2,000,000 points 5.65 and 5.66 ms, 9.41 and 6.06 ms).
+// out again: in no order 208 + 120 and 209 + 121 us, blobs numbered one after the other, each along x, 0.2 % of the points
+// before them all 643 + 153 and 337 + 153 us; per call of 2,000,000 points 5.65 and 5.66 ms, 9.41 and 6.06 ms).
 
 template <uint32_t CAPACITY, int THREADS>
 struct CrowdedSortShared {
@@ -267,9 +268,11 @@ __global__ __launch_bounds__(THREADS) void crowded_sort_kernel(CrowdedArgs args,
         bool out_of_range = false;
 #pragma unroll
         for (uint32_t u = 0; u < OWN; u++) {
-            const uint32_t k = u * THREADS + threadIdx.x;
+            // (the kernel for the most crowded cells is better off without a branch per lane: 127 -> 121 us)
+            const uint32_t own = u * THREADS + threadIdx.x;
+            const uint32_t k = CAPACITY == CROWDED_LARGE ? min(own, n - 1) : own;
             index[u] = at[u] = biased[u] = 0;
-            if (k < n) {
+            if (CAPACITY == CROWDED_LARGE ? u * THREADS < n : own < n) {
                 int32_t packed;
                 locate_candidate(sh.tables, n_stencil, k, at[u], packed);
                 int32_t qx, qy, qz;
@@ -352,30 +355,37 @@ __global__ __launch_bounds__(THREADS) void crowded_sort_kernel(CrowdedArgs args,
             }
             // Some bucket holds many: every bucket's own range of indices is shared out again among as many places as it
             // has keys, which gives an estimate of every key's rank, and the ranks two by two are the new buckets.
-            uint32_t* const low = sh.index;
-            uint32_t* const high = sh.at;
+            // (in rolled loops on LDS that is not in use yet: 337 us in the clumped case, 346 from the registers)
+            uint32_t* const low = sh.at;
+            uint32_t* const high = sh.at + BUCKETS;
             for (uint32_t b = threadIdx.x; b < BUCKETS; b += THREADS) {
                 low[b] = 0xFFFFFFFFu;
                 high[b] = 0;
             }
-            __syncthreads();
 #pragma unroll
             for (uint32_t u = 0; u < OWN; u++) {
-                if (u * THREADS + threadIdx.x < n) {
-                    atomicMin(&low[bucket[u]], index[u]);
-                    atomicMax(&high[bucket[u]], index[u]);
-                }
+                sh.index[u * THREADS + threadIdx.x] = index[u];
+                sh.biased[u * THREADS + threadIdx.x] = bucket[u];
             }
             __syncthreads();
+#pragma unroll 1
+            for (uint32_t k = threadIdx.x; k < n; k += THREADS) { // (each thread its own candidates)
+                atomicMin(&low[sh.biased[k]], sh.index[k]);
+                atomicMax(&high[sh.biased[k]], sh.index[k]);
+            }
+            __syncthreads();
+#pragma unroll 1
+            for (uint32_t k = threadIdx.x; k < n; k += THREADS) {
+                const uint32_t own = sh.biased[k];
+                const uint32_t first = sh.first[own];
+                const uint32_t keys = sh.first[own + 1] - first;
+                const float per_place = static_cast<float>(keys) / (static_cast<float>(high[own] - low[own]) + 1.0f);
+                const uint32_t place = static_cast<uint32_t>(static_cast<float>(sh.index[k] - low[own]) * per_place);
+                sh.biased[k] = (first + min(keys - 1, place)) / 2;
+            }
 #pragma unroll
             for (uint32_t u = 0; u < OWN; u++) {
-                if (u * THREADS + threadIdx.x < n) {
-                    const uint32_t first = sh.first[bucket[u]];
-                    const uint32_t keys = sh.first[bucket[u] + 1] - first;
-                    const uint32_t lowest_here = low[bucket[u]];
-                    const float per_place = static_cast<float>(keys) / (static_cast<float>(high[bucket[u]] - lowest_here) + 1.0f);
-                    bucket[u] = (first + min(keys - 1, static_cast<uint32_t>(static_cast<float>(index[u] - lowest_here) * per_place))) / 2;
-                }
+                bucket[u] = sh.biased[u * THREADS + threadIdx.x];
             }
             __syncthreads();
             for (uint32_t b = threadIdx.x; b <= BUCKETS; b += THREADS) {
