@@ -141,7 +141,7 @@ def test_a_list_that_meets_other_systems(capfd, monkeypatch):
     monkeypatch.setenv("VESIN_HIP_SORT", "crowded")
     calculator = NeighborList(cutoff=3.0, full_list=True, sorted=True)
     # (2600 points: as many candidates around a cell of the smaller box, few in the larger one: the sort for the most
-    # crowded cells is not launched where the call before had none)
+    # crowded cells has something to do in some calls and nothing in others)
     systems = [(500, 12.0), (2000, 12.0), (2000, 9.0), (2000, 20.0), (1000, 8.0), (1000, 8.0)]
     systems += [(2600, 20.0), (2600, 20.0), (2600, 9.0), (2600, 9.0), (2600, 20.0), (2600, 20.0)]
     for n, edge in systems:
