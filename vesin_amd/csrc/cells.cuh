@@ -34,8 +34,18 @@ struct FusedStatus {
 struct alignas(32) SortedPoint {
     double x, y, z;
     uint32_t index; // original point index
-    uint32_t spare;
+    uint32_t wrap;  // packed_wrap of the point
 };
+
+/// The box vectors a point was moved by, in the fields of a biased shift (biased_shift, ordered.cuh): taken off such a shift
+/// in one integer subtraction. For moves within +-255; beyond that it only differs from zero, and the searches that read it
+/// leave such systems to others.
+__device__ __forceinline__ uint32_t packed_wrap(int32_t wx, int32_t wy, int32_t wz) {
+    const int32_t a = min(max(wx, -256), 256);
+    const int32_t b = min(max(wy, -256), 256);
+    const int32_t c = min(max(wz, -256), 256);
+    return (static_cast<uint32_t>(a) << 20) + (static_cast<uint32_t>(b) << 10) + static_cast<uint32_t>(c);
+}
 
 /// Cell-sorted copy of the points. `p` is allocated with SORTED_PADDING extra elements so that the scalar loads of
 /// four consecutive points may run past the last point; the shifts (rarely non-zero, rarely read) keep an array each.
@@ -432,7 +442,7 @@ __global__ __launch_bounds__(BLOCK) void place_direct(
         return;
     }
     const size_t to = static_cast<size_t>(linear) * capacity + k;
-    sorted.p[to] = SortedPoint{x, y, z, i, 0u};
+    sorted.p[to] = SortedPoint{x, y, z, i, packed_wrap(wrap[0], wrap[1], wrap[2])};
     if ((wrap[0] | wrap[1] | wrap[2]) != 0) {
         // (the caller hands the wrap arrays over cleared, as for place_points)
         sorted.wx[to] = wrap[0];
@@ -513,7 +523,7 @@ __global__ __launch_bounds__(BLOCK) void place_points(
     // in a batch (system_of not null) the index counts from the first point of the point's system, and the tile
     // carries the system above its flag bit
     const uint32_t system = system_of != nullptr ? system_of[i] : 0;
-    sorted.p[to] = SortedPoint{x, y, z, system_of != nullptr ? i - first_point[system] : i, 0u};
+    sorted.p[to] = SortedPoint{x, y, z, system_of != nullptr ? i - first_point[system] : i, packed_wrap(wx, wy, wz)};
     if (sorted.l != nullptr) {
         sorted.l[to] = place;
     }
@@ -854,7 +864,7 @@ __global__ __launch_bounds__(BLOCK) void gather_points(
     const int32_t wz = wrap_of[3 * static_cast<size_t>(mine) + 2];
     sorted.p[to] = SortedPoint{
         points[3 * static_cast<size_t>(mine) + 0], points[3 * static_cast<size_t>(mine) + 1],
-        points[3 * static_cast<size_t>(mine) + 2], mine, 0u
+        points[3 * static_cast<size_t>(mine) + 2], mine, packed_wrap(wx, wy, wz)
     };
     sorted.wx[to] = wx;
     sorted.wy[to] = wy;
@@ -992,7 +1002,7 @@ __global__ __launch_bounds__(SMALL_BUILD_THREADS) void build_cells_small(
             const uint32_t first_tile = static_cast<uint32_t>(here >> 32);
             const uint32_t count = cell_count[cell_of[k]];
             const uint32_t to = start + slot_of[k];
-            sorted.p[to] = SortedPoint{x[k], y[k], z[k], i, 0u};
+            sorted.p[to] = SortedPoint{x[k], y[k], z[k], i, packed_wrap(wx[k], wy[k], wz[k])};
             sorted.wx[to] = wx[k];
             sorted.wy[to] = wy[k];
             sorted.wz[to] = wz[k];
@@ -1064,7 +1074,7 @@ __global__ __launch_bounds__(BLOCK) void prepare_single_cell(
             atomicMin(&status->first_bad_coordinate, 3u * i + axis);
         }
         wrapped = (wrap[0] | wrap[1] | wrap[2]) != 0;
-        sorted.p[i] = SortedPoint{x, y, z, i, 0u};
+        sorted.p[i] = SortedPoint{x, y, z, i, packed_wrap(wrap[0], wrap[1], wrap[2])};
         if (sorted.l != nullptr) {
             sorted.l[i] = local_record(pre, inside, wrap);
         }

@@ -29,6 +29,7 @@
 #define VESIN_HIP_CROWDED_CUH
 
 #include "ordered.cuh"
+#include "tile_test.cuh"
 #include "write_tile.cuh"
 
 namespace vesin_hip {
@@ -434,18 +435,108 @@ __global__ __launch_bounds__(THREADS) void crowded_sort_kernel(CrowdedArgs args,
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// COUNT: bound by the fp64 distance tests (clusters of 500,000 points, 282 us). The candidates of a tile are dealt to four
-// waves, pairs of units in turn: the most crowded tiles would otherwise run long after all others are done.
+// COUNT: in single precision (tile_test.cuh). Vector instructions fill two thirds of it, the rest is the latency of its
+// loads and the most crowded tiles, whose candidates are dealt to four waves (they would otherwise run long after all others
+// are done). In double precision -> this: clusters of 500,000 points 270 -> 250 us, 195,112 atoms at cutoff 6.5 298 -> 105 us,
+// 13,824 atoms at cutoff 5.5 33 -> 17 us. Four units at a time 275 us, three 264 (registers).
 
 struct CrowdedCountShared {
     uint32_t tile_index[TILE_POINTS];
     double tile_x[TILE_POINTS], tile_y[TILE_POINTS], tile_z[TILE_POINTS];
     int32_t tile_wx[TILE_POINTS], tile_wy[TILE_POINTS], tile_wz[TILE_POINTS];
     uint32_t rows[TILE_POINTS];
+    TileTests tests;
 };
 
+/// R units of candidates (unit0, unit0 + CROWDED_WAVES, ...) against the tile's points, in single precision but for pairs next to the
+/// cutoff; lane p of `own_rows` adds up the hits of point p.
+template <int R, bool FULL>
+__device__ __forceinline__ void crowded_count_units(
+    CrowdedCountShared& sh, const SortedPoints& sorted, const GridParams& g, const CrowdedCandidate* __restrict__ candidates,
+    uint32_t* __restrict__ columns, uint32_t unit0, uint32_t n, uint32_t first_i, uint32_t n_i, int lane, uint32_t& own_rows
+) {
+    TestCandidates<R> c;
+    CrowdedCandidate candidate[R];
+    SortedPoint point[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        // (lanes past the last candidate read the last one)
+        candidate[r] = candidates[min((unit0 + r * CROWDED_WAVES) * WAVE + lane, n - 1)];
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        point[r] = sorted.p[candidate[r].at];
+    }
+    auto shift_of = [&](uint32_t biased, double& tx, double& ty, double& tz) {
+        shift_vector(
+            g, static_cast<int32_t>((biased >> 20) & 0x3ffu) - 512, static_cast<int32_t>((biased >> 10) & 0x3ffu) - 512,
+            static_cast<int32_t>(biased & 0x3ffu) - 512, tx, ty, tz
+        );
+    };
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const bool valid = (unit0 + r * CROWDED_WAVES) * WAVE + lane < n;
+        double x = point[r].x - sh.tests.origin[0];
+        double y = point[r].y - sh.tests.origin[1];
+        double z = point[r].z - sh.tests.origin[2];
+        if (__ballot(candidate[r].biased != NO_SHIFT) != 0) {
+            double tx, ty, tz;
+            shift_of(candidate[r].biased, tx, ty, tz);
+            x += tx;
+            y += ty;
+            z += tz;
+        }
+        c.x[r] = valid ? static_cast<float>(x) : NOT_THERE;
+        c.y[r] = valid ? static_cast<float>(y) : NOT_THERE;
+        c.z[r] = valid ? static_cast<float>(z) : NOT_THERE;
+        if (!FULL) {
+            // one orientation of every pair: the smaller index first; a point with its own image under the rule of the
+            // reference: the total shift of such a pair is the cell shift
+            const uint32_t cell_shift = candidate[r].biased + point[r].wrap;
+            const bool own_image = cell_shift != NO_SHIFT && half_keeps_self_image(
+                                                                 static_cast<int32_t>((cell_shift >> 20) & 0x3ffu) - 512,
+                                                                 static_cast<int32_t>((cell_shift >> 10) & 0x3ffu) - 512,
+                                                                 static_cast<int32_t>(cell_shift & 0x3ffu) - 512
+                                                             );
+            c.limit[r] = point[r].index + (own_image ? 1u : 0u);
+        }
+    }
+    uint32_t column[R];
+    uint32_t rows;
+    if (test_tile<R, FULL>(sh.tests, sh.tile_index, n_i, c, column, rows) != 0) {
+        resolve_tile<R, FULL>(sh.tests, sh.tile_index, n_i, c, column, rows, [&](int r, uint32_t p) {
+            const CrowdedCandidate again = candidates[min((unit0 + r * CROWDED_WAVES) * WAVE + lane, n - 1)];
+            const SortedPoint there = sorted.p[again.at];
+            double tx, ty, tz;
+            shift_of(again.biased + packed_wrap(sh.tile_wx[p], sh.tile_wy[p], sh.tile_wz[p]), tx, ty, tz);
+            const double vx = (there.x - sh.tile_x[p]) + tx;
+            const double vy = (there.y - sh.tile_y[p]) + ty;
+            const double vz = (there.z - sh.tile_z[p]) + tz;
+            return vx * vx + vy * vy + vz * vz < g.cutoff2;
+        });
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const uint32_t k = (unit0 + r * CROWDED_WAVES) * WAVE + lane;
+        if (FULL) {
+            // a point is no neighbour of itself (of its images it is)
+            const uint32_t own = candidate[r].at - first_i;
+            const uint32_t bit = 1u << ((n_i - 1 - own) % 32u);
+            const bool itself = k < n && own < n_i && candidate[r].biased + point[r].wrap == NO_SHIFT && (column[r] & bit) != 0;
+            column[r] &= itself ? ~bit : ~0u;
+            if (__ballot(itself) != 0) {
+                if (itself) {
+                    atomicSub(&sh.rows[own], 1u);
+                }
+            }
+        }
+        columns[k] = column[r];
+    }
+    own_rows += rows;
+}
+
 template <bool FULL>
-__global__ __launch_bounds__(CROWDED_BLOCK) void crowded_count_kernel(CrowdedArgs args, GridParams g) {
+__global__ __launch_bounds__(CROWDED_BLOCK, 5) void crowded_count_kernel(CrowdedArgs args, GridParams g) {
     constexpr int R = ORDERED_R;
     __shared__ CrowdedCountShared sh;
     const int lane = lane_id();
@@ -467,32 +558,45 @@ __global__ __launch_bounds__(CROWDED_BLOCK) void crowded_count_kernel(CrowdedArg
         const uint32_t n_units = (n + WAVE - 1) / WAVE;
         const bool tile_wrapped = (tile.wrapped & 1u) != 0;
         __syncthreads(); // (the tile before is done with the LDS)
-        bool out_of_range = false;
-        if (threadIdx.x < n_i) {
-            const uint32_t at = tile.first + threadIdx.x;
-            const SortedPoint point = args.sorted.p[at];
-            sh.tile_index[threadIdx.x] = point.index;
-            sh.tile_x[threadIdx.x] = point.x;
-            sh.tile_y[threadIdx.x] = point.y;
-            sh.tile_z[threadIdx.x] = point.z;
-            const int32_t wx = args.sorted.wx[at];
-            const int32_t wy = args.sorted.wy[at];
-            const int32_t wz = args.sorted.wz[at];
-            sh.tile_wx[threadIdx.x] = wx;
-            sh.tile_wy[threadIdx.x] = wy;
-            sh.tile_wz[threadIdx.x] = wz;
-            out_of_range = beyond(wx, wy, wz, ORDERED_SHIFT_LIMIT);
-            sh.rows[threadIdx.x] = 0;
-        }
-        if (__ballot(out_of_range) != 0 && lane == 0) {
-            atomicOr(&args.status->unsuitable, 1u);
+        if (wave == 0) {
+            bool out_of_range = false;
+            SortedPoint point = {0.0, 0.0, 0.0, 0u, 0u};
+            int32_t wx = 0, wy = 0, wz = 0;
+            if (static_cast<uint32_t>(lane) < n_i) {
+                const uint32_t at = tile.first + lane;
+                point = args.sorted.p[at];
+                wx = args.sorted.wx[at];
+                wy = args.sorted.wy[at];
+                wz = args.sorted.wz[at];
+                sh.tile_index[lane] = point.index;
+                sh.tile_x[lane] = point.x;
+                sh.tile_y[lane] = point.y;
+                sh.tile_z[lane] = point.z;
+                sh.tile_wx[lane] = wx;
+                sh.tile_wy[lane] = wy;
+                sh.tile_wz[lane] = wz;
+                out_of_range = beyond(wx, wy, wz, ORDERED_SHIFT_LIMIT);
+                sh.rows[lane] = 0;
+            }
+            prepare_tile_tests(sh.tests, g, lane, n_i, point.x, point.y, point.z, wx, wy, wz);
+            if (__ballot(out_of_range) != 0 && lane == 0) {
+                atomicOr(&args.status->unsuitable, 1u);
+            }
         }
         __syncthreads();
 
         const CrowdedCandidate* candidates = args.candidates + static_cast<size_t>(cell.first_candidate) * WAVE;
         uint32_t* columns = args.columns + (static_cast<size_t>(cell.first_column) + static_cast<size_t>(t - first_tile) * n_units) * WAVE;
         uint32_t own_rows = 0;
-        for (uint32_t unit0 = wave * R; unit0 < n_units; unit0 += CROWDED_WAVES * R) {
+        const bool single = uniform(sh.tests.usable) != 0;
+        uint32_t unit = wave;
+        for (; single && unit + (R - 1) * CROWDED_WAVES < n_units; unit += R * CROWDED_WAVES) {
+            crowded_count_units<R, FULL>(sh, args.sorted, g, candidates, columns, unit, n, tile.first, n_i, lane, own_rows);
+        }
+        for (; single && unit < n_units; unit += CROWDED_WAVES) {
+            crowded_count_units<1, FULL>(sh, args.sorted, g, candidates, columns, unit, n, tile.first, n_i, lane, own_rows);
+        }
+        for (uint32_t unit0 = wave * R; !single && unit0 < n_units; unit0 += CROWDED_WAVES * R) {
             SweepCandidates<R> c;
             uint32_t original[R], column[R];
             int32_t bx[R], by[R], bz[R];
@@ -604,11 +708,14 @@ __global__ void clear_crowded_status(CrowdedStatus* status) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// WRITE
+// WRITE: only the candidates with a hit go through the chunks (clusters of 500,000 points, P d, 700 -> 615 us; 200,000
+// points, 55 per cell, half P S d D 440 -> 345 us).
 
-template <bool STAGED>
+template <bool STAGED, TileStores STORES>
 __global__ __launch_bounds__(TILE_BLOCK, STAGED ? 4 : 5) void crowded_write_kernel(CrowdedArgs args, GridParams g) {
     __shared__ TileWriteShared<STAGED> sh;
+    __shared__ uint32_t hits_of[4 * TILE_WAVES];
+    __shared__ uint32_t beyond_chunk;
     const uint32_t lane = static_cast<uint32_t>(lane_id());
     const uint32_t wave = uniform(threadIdx.x / WAVE);
     const CrowdedStatus found = *args.status;
@@ -636,32 +743,79 @@ __global__ __launch_bounds__(TILE_BLOCK, STAGED ? 4 : 5) void crowded_write_kern
         const CrowdedCandidate* candidates = args.candidates + static_cast<size_t>(cell.first_candidate) * WAVE;
         const uint32_t* columns =
             args.columns + (static_cast<size_t>(cell.first_column) + static_cast<size_t>(t - first_tile) * n_units) * WAVE;
-        for (uint32_t first = 0; first < n; first += TILE_CHUNK) {
-            const uint32_t in_chunk = min(n - first, TILE_CHUNK);
-            const uint32_t units_here = (in_chunk + WAVE - 1) / WAVE;
+        // The candidates that some point of the tile has for a neighbour (about two thirds), TILE_CHUNK of them at a time: each
+        // thread looks at one in TILE_BLOCK of the next 4 TILE_BLOCK candidates.
+        constexpr uint32_t LOOK = 4;
+        for (uint32_t first = 0; first < n;) {
             if (first != 0) {
                 __syncthreads();
             }
-            bool shifted = moved;
-            for (uint32_t k = threadIdx.x; k < units_here * WAVE; k += TILE_BLOCK) {
-                uint32_t column = 0;
-                if (k < in_chunk) {
-                    column = columns[first + k];
-                    const CrowdedCandidate candidate = candidates[first + k];
-                    const SortedPoint point = args.sorted.p[candidate.at];
-                    sh.x[k] = point.x;
-                    sh.y[k] = point.y;
-                    sh.z[k] = point.z;
-                    sh.index[k] = point.index;
-                    sh.biased[k] = candidate.biased;
-                    shifted = shifted || candidate.biased != NO_SHIFT;
+            uint32_t column[LOOK];
+            CrowdedCandidate candidate[LOOK];
+            uint64_t mask[LOOK];
+#pragma unroll
+            for (uint32_t u = 0; u < LOOK; u++) {
+                const uint32_t k = first + u * TILE_BLOCK + threadIdx.x;
+                column[u] = 0;
+                if (k < n) {
+                    column[u] = columns[k];
+                    candidate[u] = candidates[k];
                 }
-                sh.column[k] = column;
             }
-            if (__syncthreads_or(shifted) != 0) {
-                write_tile_chunk<true, STAGED>(sh, wave, g, args.out, n_i, units_here, n > TILE_CHUNK, lane);
+#pragma unroll
+            for (uint32_t u = 0; u < LOOK; u++) {
+                mask[u] = __ballot(column[u] != 0);
+                if (lane == 0) {
+                    hits_of[u * TILE_WAVES + wave] = __popcll(mask[u]);
+                }
+            }
+            __syncthreads();
+            uint32_t found = 0;
+            uint32_t next = min(first + LOOK * TILE_BLOCK, n);
+            bool shifted = moved;
+#pragma unroll
+            for (uint32_t u = 0; u < LOOK; u++) {
+                uint32_t slot = found + rank_in_mask(mask[u]);
+#pragma unroll
+                for (uint32_t w = 0; w < TILE_WAVES; w++) {
+                    const uint32_t hits = uniform(hits_of[u * TILE_WAVES + w]);
+                    slot += w < wave ? hits : 0u;
+                    found += hits;
+                }
+                const uint32_t k = first + u * TILE_BLOCK + threadIdx.x;
+                if (column[u] != 0 && slot < TILE_CHUNK) {
+                    const SortedPoint point = args.sorted.p[candidate[u].at];
+                    sh.x[slot] = point.x;
+                    sh.y[slot] = point.y;
+                    sh.z[slot] = point.z;
+                    sh.index[slot] = point.index;
+                    sh.biased[slot] = candidate[u].biased;
+                    sh.column[slot] = column[u];
+                    shifted = shifted || candidate[u].biased != NO_SHIFT;
+                }
+                if (column[u] != 0 && slot == TILE_CHUNK) {
+                    beyond_chunk = k; // the first that did not fit
+                }
+            }
+            const uint32_t in_chunk = min(found, TILE_CHUNK);
+            const uint32_t units_here = (in_chunk + WAVE - 1) / WAVE;
+            // (the columns of the last unit beyond the last candidate)
+            if (threadIdx.x < units_here * WAVE - in_chunk) {
+                sh.column[in_chunk + threadIdx.x] = 0;
+            }
+            const bool any_shifted = __syncthreads_or(shifted) != 0;
+            if (found > TILE_CHUNK) {
+                next = uniform(beyond_chunk);
+            }
+            const bool more_chunks = first != 0 || next < n;
+            first = next;
+            if (in_chunk == 0) {
+                continue;
+            }
+            if (any_shifted) {
+                write_tile_chunk<true, STAGED, STORES>(sh, wave, g, args.out, n_i, units_here, more_chunks, lane);
             } else {
-                write_tile_chunk<false, STAGED>(sh, wave, g, args.out, n_i, units_here, n > TILE_CHUNK, lane);
+                write_tile_chunk<false, STAGED, STORES>(sh, wave, g, args.out, n_i, units_here, more_chunks, lane);
             }
         }
     }

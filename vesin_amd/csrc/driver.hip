@@ -38,6 +38,7 @@
 #include "images.cuh"
 #include "molecules.cuh"
 #include "ordered.cuh"
+#include "ordered_tile.cuh"
 #include "small.cuh"
 #include "policy.hpp"
 #include "scan.cuh"
@@ -203,6 +204,20 @@ static bool radix_sort_only() {
 
 /// VESIN_HIP_SORT=crowded sends every sorted list of one system to the in-order search for crowded cells (for
 /// comparisons and tests).
+template <bool VECTORS>
+static auto ordered_write_kernel_for(TileStores stores) {
+    return stores == STORE_CACHED       ? ordered_write_kernel<VECTORS, STORE_CACHED>
+           : stores == STORE_BY_GRANULE ? ordered_write_kernel<VECTORS, STORE_BY_GRANULE>
+                                        : ordered_write_kernel<VECTORS, STORE_STREAMED>;
+}
+
+template <bool VECTORS>
+static auto crowded_write_kernel_for(TileStores stores) {
+    return stores == STORE_CACHED       ? crowded_write_kernel<VECTORS, STORE_CACHED>
+           : stores == STORE_BY_GRANULE ? crowded_write_kernel<VECTORS, STORE_BY_GRANULE>
+                                        : crowded_write_kernel<VECTORS, STORE_STREAMED>;
+}
+
 static bool crowded_search_only() {
     const char* text = std::getenv("VESIN_HIP_SORT");
     return text != nullptr && std::strcmp(text, "crowded") == 0;
@@ -1074,12 +1089,14 @@ struct HipExtras {
     int in_order_rest = 0;            // calls left before the in-order search is tried again on a system it did not cover
     int crowded_rest = 0;             // the same for the in-order search for crowded cells (crowded.cuh)
     size_t crowded_points = 0;        // the last system that search covered: its number of points ...
-    CrowdedRoom crowded_room;         // ... and the room for its candidates and hit columns
+    CrowdedRoom crowded_room;         // ... and the room for its candidates and hit columns, and its rows
+    size_t crowded_rows = 0;
     int one_launch_rest = 0;          // calls left before a small system is tried in one launch again
     WaitRest meeting_rest;            // ... after workgroups of that launch gave up waiting for the others
     WaitRest chain_rest;              // the same for the chain of the single-pass search (rows in work-item order)
     uint32_t ordered_tiles = 0;       // tiles of the last call through the in-order search, and its number of points:
-    size_t ordered_tiles_points = 0;  // how the next one deals its writing pass to the waves (see write_split)
+    size_t ordered_tiles_points = 0;  // which kernels the next one takes, and how it deals its passes to the waves
+    size_t ordered_rows = 0;          // and its rows: how the next one stores them (see tile_stores)
     /// Extent of the points along the directions that are not periodic, as the last call found it: a small system
     /// that went through the one launch reports it on the way, and the next call of the same kind (see BoxGuess) on
     /// the same box picks its grid from it without a pass over the points and a round trip to the host first. A
@@ -2022,6 +2039,10 @@ bool compute(
         ordered_points_per_item = wanted;
     }
     const uint32_t ordered_items_per_tile = TILE_POINTS / ordered_points_per_item;
+    // (from a list's second call on the same number of points: a workgroup per tile, ordered_tile.cuh)
+    const size_t tiles_known = extras.ordered_tiles_points == n_points ? extras.ordered_tiles : 0;
+    const bool by_tiles = std::getenv("VESIN_HIP_WRITE_SPLIT") == nullptr && std::getenv("VESIN_HIP_COUNT_SPLIT") == nullptr &&
+                          std::getenv("VESIN_HIP_ORDERED_SHARE") == nullptr && ordered_by_tiles(n_points, tiles_known);
     const uint32_t ordered_blocks =
         static_cast<uint32_t>((tiles_bound * ordered_items_per_tile + ORDERED_WAVES - 1) / ORDERED_WAVES);
     const size_t ordered_record_bytes =
@@ -2071,8 +2092,9 @@ bool compute(
         }
         sorted.p = carver.take<SortedPoint>(sorted_slots + SORTED_PADDING);
         // (the places of the points inside their cells, for the single-precision pre-test of the in-order search's
-        // counting pass; the cell builds of small systems and of the reproducible order do not fill them in)
-        sorted.l = try_in_order && pre.use32 != 0 && !small_build && !ordered_rows()
+        // counting pass of a wave per tile; the cell builds of small systems and of the reproducible order do not fill
+        // them in)
+        sorted.l = try_in_order && !by_tiles && pre.use32 != 0 && !small_build && !ordered_rows()
                        ? carver.take<float4>(sorted_slots + SORTED_PADDING)
                        : nullptr;
         counts = carver.take<uint32_t>(std::max(n_slots, direct_slots * n_slices));
@@ -2085,7 +2107,7 @@ bool compute(
         if (try_in_order) {
             candidate_records = carver.take<CandidateRecord>(static_cast<size_t>(ordered_blocks) * ORDERED_WAVES * ORDERED_UNITS * WAVE);
             candidates_of_item = carver.take<uint32_t>(static_cast<size_t>(ordered_blocks) * ORDERED_WAVES);
-            if (ordered_items_per_tile == 1) {
+            if (ordered_items_per_tile == 1 && !by_tiles) {
                 candidate_order = carver.take<uint16_t>(tiles_bound * ORDERED_CANDIDATES);
             }
 
@@ -2510,21 +2532,14 @@ bool compute(
         // How many waves share a tile in either pass follows the number of tiles the call before had on the same
         // number of points (policy.hpp); a list's first call on a system keeps one wave per tile.
         const bool presorted = ordered_items_per_tile == 1;
-        const size_t tiles_before = presorted && extras.ordered_tiles_points == n_points ? extras.ordered_tiles : 0;
-        oargs.write_split = ordered_write_split(n_points, tiles_before);
-        // well-filled tiles whose candidates come in one chunk: a workgroup per tile (write_tile.cuh)
-        const bool tile_writer =
-            presorted && std::getenv("VESIN_HIP_WRITE_SPLIT") == nullptr &&
-            ordered_write_by_tiles(n_points, n_cells, tiles_before, full_stencil, options.return_vectors);
-        if (tile_writer) {
-            oargs.write_split = TILE_WAVES;
-        }
+        const size_t tiles_before = presorted ? tiles_known : 0;
+        oargs.write_split = by_tiles ? TILE_WAVES : ordered_write_split(n_points, tiles_before);
         if (const char* text = std::getenv("VESIN_HIP_WRITE_SPLIT")) {
             oargs.write_split = static_cast<uint32_t>(std::max(1, std::min(4, std::atoi(text))));
         }
         // (the waves of a tile add their rows in memory that the cell build cleared)
         const bool rows_cleared = !single_cell && !small_build;
-        oargs.count_split = rows_cleared ? ordered_count_split(n_points, tiles_before) : 1;
+        oargs.count_split = by_tiles ? TILE_WAVES : rows_cleared ? ordered_count_split(n_points, tiles_before) : 1;
         if (const char* text = std::getenv("VESIN_HIP_COUNT_SPLIT")) {
             oargs.count_split = rows_cleared ? static_cast<uint32_t>(std::max(1, std::min(4, std::atoi(text)))) : 1u;
         }
@@ -2547,10 +2562,13 @@ bool compute(
                 dim3(ORDER_BLOCK), 0, where, oargs, g
             );
         };
-        auto launch_write = [&]() {
-            if (tile_writer) {
-                auto kernel = oargs.out.vectors != nullptr ? ordered_write_kernel<true> : ordered_write_kernel<false>;
-                hipLaunchKernelGGL(kernel, dim3(blocks * ORDERED_WAVES), dim3(TILE_BLOCK), 0, stream, oargs, g);
+        // (`rows`: as far as they are known: those of the call before, where this one's were not counted yet)
+        auto launch_write = [&](size_t rows) {
+            if (by_tiles) {
+                const TileStores stores =
+                    tile_stores(n_points, rows, options.return_shifts, options.return_distances, options.return_vectors);
+                auto kernel = options.return_vectors ? ordered_write_kernel_for<true>(stores) : ordered_write_kernel_for<false>(stores);
+                hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(tiles_bound)), dim3(TILE_BLOCK), 0, stream, oargs, g);
                 return;
             }
             auto kernel = presorted ? (options.full ? ordered_search_kernel<true, true, true> : ordered_search_kernel<true, false, true>)
@@ -2571,6 +2589,14 @@ bool compute(
             oargs.guarded = 1;
         }
         auto launch_count_and_scan = [&]() {
+            if (by_tiles) {
+                auto kernel = options.full ? ordered_tile_kernel<true> : ordered_tile_kernel<false>;
+                hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(tiles_bound)), dim3(TILE_BLOCK), 0, stream, oargs, g);
+                mark(T_COUNT);
+                exclusive_scan<SCAN_U32>(rows_of_point, n_points, first_row_of_point, scan_scratch, stream);
+                mark(T_SCAN);
+                return;
+            }
             hipStream_t side = presorted && !ordered_one_stream() ? extras.side() : nullptr;
             if (side != nullptr) {
                 HIP_CHECK(hipEventRecord(extras.side_fork, stream));
@@ -2599,7 +2625,7 @@ bool compute(
                 oargs.publish_to = &extras.mail_device->ordered;
                 oargs.build_status = extras.d_status;
                 mark(T_WRITE_BEGIN);
-                launch_write();
+                launch_write(extras.ordered_rows);
                 mark(T_WRITE);
                 oargs.publish_to = nullptr;
                 QueuedOutcome outcome = queued_outcome(2);
@@ -2625,16 +2651,23 @@ bool compute(
         }
         extras.ordered_tiles = found.n_tiles;
         extras.ordered_tiles_points = n_points;
+        extras.ordered_rows = found.total_rows;
         const bool suitable = found.found.max_rows <= ORDERED_MAX_ROWS &&
                               found.found.max_candidates <= ORDERED_CANDIDATES && found.found.unsuitable == 0;
         if (std::getenv("VESIN_HIP_DEBUG") != nullptr) {
+            // (well-filled tiles whose candidates come to the writing pass's LDS in one go, also where all of them have a
+            // hit: 10 points per tile, 16 when there are vectors, and 665 candidates on average)
+            const bool one_chunk =
+                tiles_before > 0 &&
+                static_cast<double>(n_points) >= (options.return_vectors ? 16.0 : 10.0) * static_cast<double>(tiles_before) &&
+                static_cast<double>(full_stencil) * static_cast<double>(n_points) <= 665.0 * static_cast<double>(n_cells);
             std::fprintf(
                 stderr,
                 "in-order search: rows %llu, most rows of a point %u, most candidates of a tile %u, unsuitable %u, "
                 "candidates of %u tiles ordered by window and of %u by buckets, %u tiles written by %u waves each%s and counted by %u: %s\n",
                 found.total_rows, found.found.max_rows, found.found.max_candidates, found.found.unsuitable,
                 found.found.windowed, found.found.bucketed, found.n_tiles, oargs.write_split,
-                tile_writer ? " (candidates in LDS)" : "", oargs.count_split, suitable ? "used" : "not covered"
+                by_tiles && one_chunk ? " (candidates in LDS)" : "", oargs.count_split, suitable ? "used" : "not covered"
             );
         }
         if (suitable) {
@@ -2647,7 +2680,7 @@ bool compute(
                 oargs.guarded = 0;
                 mark(T_WRITE_BEGIN);
                 if (total > 0) {
-                    launch_write();
+                    launch_write(total);
                 }
                 mark(T_WRITE);
                 mark(T_SORT);
@@ -2711,8 +2744,10 @@ bool compute(
             cargs.candidate_units = static_cast<uint32_t>(room.candidate_units);
             cargs.column_units = static_cast<uint32_t>(room.column_units);
             const bool early_write = known && extras.capacity > 0;
-            auto launch_write = [&]() {
-                auto kernel = cargs.out.vectors != nullptr ? crowded_write_kernel<true> : crowded_write_kernel<false>;
+            auto launch_write = [&](size_t rows) {
+                const TileStores stores =
+                    crowded_stores(n_points, rows, options.return_shifts, options.return_distances, options.return_vectors);
+                auto kernel = options.return_vectors ? crowded_write_kernel_for<true>(stores) : crowded_write_kernel_for<false>(stores);
                 hipLaunchKernelGGL(kernel, dim3(tile_blocks), dim3(TILE_BLOCK), 0, stream, cargs, g);
             };
             if (attempt > 0) {
@@ -2748,7 +2783,7 @@ bool compute(
                 cargs.out = outputs_of();
                 cargs.capacity = early_capacity;
                 mark(T_WRITE_BEGIN);
-                launch_write();
+                launch_write(extras.crowded_rows);
                 mark(T_WRITE);
             }
             extras.wait(stream);
@@ -2786,6 +2821,7 @@ bool compute(
             }
             extras.crowded_points = pays ? n_points : 0; // (0: the next call counts, and decides, before it does anything else)
             extras.crowded_room = crowded_room_kept(n_points, room, counted);
+            extras.crowded_rows = found.total_rows;
             const size_t total = found.total_rows;
             check_pair_limit(total);
             if (!(early_write && total <= early_capacity)) {
@@ -2795,7 +2831,7 @@ bool compute(
                 cargs.capacity = extras.capacity;
                 mark(T_WRITE_BEGIN);
                 if (total > 0) {
-                    launch_write();
+                    launch_write(total);
                 }
                 mark(T_WRITE);
                 HIP_CHECK(hipStreamSynchronize(stream));

@@ -354,13 +354,12 @@ __device__ __forceinline__ bool ordered_sweep_pair32(
     return true;
 }
 
-template <bool FULL, bool WRAPPED, typename Shared>
+template <bool FULL, bool WRAPPED, int R = ORDERED_R, typename Shared>
 __device__ __forceinline__ void ordered_sweep_pair(
     const Shared& sh, const SortedPoints& sorted, const GridParams& g, uint32_t unit0, uint32_t n_stencil,
-    uint32_t n_candidates, uint32_t first_i, uint32_t n_i, int lane, uint32_t (&column)[ORDERED_R], uint32_t& rows,
-    bool& out_of_range, uint32_t (&at)[ORDERED_R], uint32_t (&original)[ORDERED_R], uint32_t (&biased)[ORDERED_R]
+    uint32_t n_candidates, uint32_t first_i, uint32_t n_i, int lane, uint32_t (&column)[R], uint32_t& rows,
+    bool& out_of_range, uint32_t (&at)[R], uint32_t (&original)[R], uint32_t (&biased)[R]
 ) {
-    constexpr int R = ORDERED_R;
     SweepCandidates<R> c;
     int32_t packed_q[R];
     bool any_shift = false;
@@ -951,111 +950,6 @@ __global__ __launch_bounds__(ORDERED_BLOCK) __attribute__((amdgpu_waves_per_eu(4
                 sh, PointsByIndex{system_points}, g, args.out, columns, cand_index, cand_index, cand_biased, n_units, n_i - 1 - p, wrap_i,
                 sh.tile_x[p], sh.tile_y[p], sh.tile_z[p], sh.tile_index[p], sh.tile_row[p], lane
             );
-        }
-    }
-}
-
-/// WRITE for well-filled tiles (ordered_write_by_tiles, policy.hpp), with the candidates in the order ordered_sort_kernel
-/// left for the tile: one workgroup per tile (see write_tile.cuh).
-///
-/// Bound half by its stores, half by latency. 1,000,000 atoms of diamond (23 points and 630 candidates per tile, full list),
-/// ordered_search_kernel<true, ...> -> this: P S d 1.11 -> 0.93 ms (3.4 TB/s; without its stores the kernel takes 0.57 ms,
-/// a copy of that many bytes 0.67), P 0.80 -> 0.56 ms, P S d D 1.56 -> 1.50 ms; in random order P S d 1.35 -> 1.04 ms,
-/// P S d D 1.87 -> 1.59 ms. Eight waves per tile 1.16 ms, two 1.01, two steps of rows side by side 1.01 (registers).
-template <bool STAGED>
-__global__ __launch_bounds__(TILE_BLOCK, STAGED ? 4 : 5) void ordered_write_kernel(OrderedArgs args, GridParams g) {
-    __shared__ TileWriteShared<STAGED> sh;
-    const uint32_t lane = static_cast<uint32_t>(lane_id());
-    const uint32_t wave = uniform(threadIdx.x / WAVE);
-    if (args.publish_to != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
-        OrderedHostStatus report;
-        report.found = *args.status;
-        report.total_rows = args.first_row[g.n_points];
-        report.first_bad_coordinate = args.build_status->first_bad_coordinate;
-        report.n_tiles = static_cast<unsigned int>(args.cell_scan[g.n_cells] >> 32);
-        *args.publish_to = report;
-    }
-    if (args.guarded != 0) {
-        const OrderedStatus found = *args.status;
-        const bool suitable = found.max_rows <= ORDERED_MAX_ROWS && found.max_candidates <= ORDERED_CANDIDATES &&
-                              found.unsuitable == 0 && args.first_row[g.n_points] <= args.capacity;
-        if (!suitable) {
-            return;
-        }
-    }
-    // the work item of the counting pass that this tile was: tiles in the same order, on the same XCD
-    const uint32_t n_tiles = static_cast<uint32_t>(args.cell_scan[g.n_cells] >> 32);
-    const uint32_t per_xcd = (n_tiles + N_XCD - 1) / N_XCD;
-    const uint32_t xcd = blockIdx.x % N_XCD;
-    const uint32_t within = blockIdx.x / N_XCD;
-    const uint32_t tile_id = xcd * per_xcd + within;
-    if (within >= per_xcd || tile_id >= n_tiles) {
-        return;
-    }
-    const uint32_t work = ((within / ORDERED_WAVES) * N_XCD + xcd) * ORDERED_WAVES + within % ORDERED_WAVES;
-    // What the first chunk needs comes through a chain of loads (place in the order, record, point), each of which takes
-    // microseconds beside the stores of the other workgroups: they are issued as early as they can be, before the tile is
-    // known (the arrays hold ORDERED_CANDIDATES entries per tile, whatever the tile uses).
-    const CandidateRecord* records = args.records + static_cast<size_t>(work) * ORDERED_CANDIDATES;
-    const uint16_t* order = args.order + static_cast<size_t>(tile_id) * ORDERED_CANDIDATES;
-    constexpr uint32_t OWN = (TILE_CHUNK + TILE_BLOCK - 1) / TILE_BLOCK; // candidates of a chunk that a thread brings
-    uint32_t place[OWN];
-#pragma unroll
-    for (uint32_t u = 0; u < OWN; u++) {
-        place[u] = order[u * TILE_BLOCK + threadIdx.x];
-    }
-    const uint32_t n = uniform(args.candidates_of_item[work]);
-    const Tile tile = args.tiles[tile_id];
-    const uint32_t n_i = uniform(tile.count);
-    CandidateRecord record[OWN];
-    double x[OWN], y[OWN], z[OWN];
-    auto load_chunk = [&](uint32_t first) {
-#pragma unroll
-        for (uint32_t u = 0; u < OWN; u++) {
-            const uint32_t k = u * TILE_BLOCK + threadIdx.x;
-            record[u] = CandidateRecord{0u, 0u, NO_SHIFT};
-            if (k < TILE_CHUNK && first + k < n) {
-                record[u] = records[min(place[u], n - 1)];
-            }
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < OWN; u++) {
-            const double* point = args.points + 3 * static_cast<size_t>(record[u].index);
-            x[u] = point[0];
-            y[u] = point[1];
-            z[u] = point[2];
-        }
-    };
-    load_chunk(0);
-    const bool moved = load_tile(sh, args.sorted, tile.first, n_i, args.first_row);
-    for (uint32_t first = 0; first < n; first += TILE_CHUNK) {
-        if (first != 0) {
-#pragma unroll
-            for (uint32_t u = 0; u < OWN; u++) {
-                place[u] = order[min(first + u * TILE_BLOCK + threadIdx.x, ORDERED_CANDIDATES - 1)];
-            }
-            load_chunk(first);
-            __syncthreads();
-        }
-        bool shifted = moved;
-#pragma unroll
-        for (uint32_t u = 0; u < OWN; u++) {
-            const uint32_t k = u * TILE_BLOCK + threadIdx.x;
-            if (k < TILE_CHUNK) {
-                sh.x[k] = x[u];
-                sh.y[k] = y[u];
-                sh.z[k] = z[u];
-                sh.index[k] = record[u].index;
-                sh.biased[k] = record[u].biased;
-                sh.column[k] = record[u].column;
-            }
-            shifted = shifted || record[u].biased != NO_SHIFT;
-        }
-        const uint32_t units_here = (min(n - first, TILE_CHUNK) + WAVE - 1) / WAVE;
-        if (__syncthreads_or(shifted) != 0) {
-            write_tile_chunk<true, STAGED>(sh, wave, g, args.out, n_i, units_here, n > TILE_CHUNK, lane);
-        } else {
-            write_tile_chunk<false, STAGED>(sh, wave, g, args.out, n_i, units_here, n > TILE_CHUNK, lane);
         }
     }
 }

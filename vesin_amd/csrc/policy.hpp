@@ -231,8 +231,9 @@ inline bool crowded_search_pays(size_t n_points, size_t n_tiles) {
     return n_tiles <= 16384 || n_points >= 5 * n_tiles;
 }
 
-/// Waves that share the points of a tile in the writing pass (1 or 4), from the number of tiles the call before had
-/// on the same points (0: not known, one wave).
+/// Waves that share the points of a tile in the writing pass of a wave per tile or share (1 or 4), from the number of tiles the
+/// call before had on the same points (0: not known, one wave). Such tiles have a workgroup each since (ordered_by_tiles),
+/// unless one of the two numbers of waves is forced.
 ///
 /// The pass keeps four waves per SIMD resident, 4096 on this GPU. A system of a few more tiles than that leaves the
 /// stragglers running alone for as long as everything before them took (100,000 atoms, 4,260 tiles: 172 us where a
@@ -255,31 +256,6 @@ inline unsigned int ordered_write_split(size_t n_points, size_t tiles_before) {
     return tiles > 0.85 * resident && tiles <= 5.0 * resident ? 4 : 1;
 }
 
-/// Whether the writing pass gives every tile a workgroup that brings the candidates' coordinates to LDS (write_tile.cuh),
-/// from the same number. Bringing them pays when enough rows are made of them: 10 points per tile, or 16 when vectors are
-/// returned (their way through LDS leaves room for fewer workgroups). Candidates beyond 704 come in a second chunk,
-/// which costs more than it gives: 665 on average at most, so that few tiles have more. Writing pass, the other kernel with
-/// a wave per tile -> this, cutoff 5, liquids of 300,000 points with 8 / 10 / 16 / 20 / 28 points per cell: full lists P S d
-/// 220 -> 227, 228 -> 207, 307 -> 250, 328 -> 277, 388 -> 421 us; half lists P S d D 206 -> 299, 211 -> 278, 288 -> 260,
-/// 298 -> 291, 350 -> 439 us; 60,000 points with 6 / 10 / 16 / 20: full 57 -> 56, 68 -> 50, 81 -> 60, 89 -> 70 us, half 54 ->
-/// 74, 63 -> 64, 79 -> 66, 87 -> 70 us.
-///
-/// The same against the kernel it takes the place of (ordered_write_split: four waves per tile from 3,482 to 20,480 tiles, one
-/// below), cutoff 5, 2,197 / 4,096 / 9,261 / 19,683 cells; cutoffs 4 and 6 differ by 1-2 %. Liquids with 20 points per cell:
-/// half P S d 70 -> 42, 85 -> 66, 175 -> 131, 372 -> 260 us; half P S d D 70 -> 60, 100 -> 98, 196 -> 193, 394 -> 389; full
-/// P S d D 105 -> 84, 150 -> 147, 294 -> 308, 597 -> 609. Lattices in order, 22.4 per cell: half P S d D 64 -> 56, 111 -> 104,
-/// 224 -> 211, 405 -> 393; full P S d D 99 -> 79, 191 -> 167, 380 -> 343, 711 -> 643. The one shape that loses (full lists with
-/// vectors, points in no order, 9,000 to 20,480 tiles: up to 5 % of the pass, 1 % of a call) cannot be told from the one
-/// that wins a tenth, the same list of points in order.
-inline bool ordered_write_by_tiles(size_t n_points, size_t n_cells, size_t tiles_before, size_t stencil_cells, bool vectors) {
-    if (tiles_before == 0 || n_cells == 0) {
-        return false;
-    }
-    const double points = static_cast<double>(n_points);
-    return points >= (vectors ? 16.0 : 10.0) * static_cast<double>(tiles_before) &&
-           static_cast<double>(stencil_cells) * points <= 665.0 * static_cast<double>(n_cells);
-}
-
 /// Waves that share the candidates of a tile in the counting pass (1 or 2), decided like the other.
 ///
 /// That pass runs seven waves per SIMD (7168 at a time) and lasts as long as its slowest wave, the one of the tile
@@ -293,6 +269,60 @@ inline unsigned int ordered_count_split(size_t n_points, size_t tiles_before) {
         return 1;
     }
     return static_cast<double>(n_points) >= 16.0 * static_cast<double>(tiles_before) ? 2 : 1;
+}
+
+/// Whether the search gives every tile a workgroup (ordered_tile.cuh) in place of a wave or several (ordered.cuh), from the
+/// number of tiles the call before had on the same points (0: not known, and a wave per tile).
+///
+/// Its kernels are the faster ones but for many tiles of few points, where most of a workgroup has nothing to do. Per call, a
+/// wave per tile or share of a tile -> a workgroup per tile, cutoff 5, liquids with 1.5 / 3 / 5 / 7 / 9 / 12 points per cell:
+/// 20,000 points full P S d 160 -> 147, 139 -> 130, 181 -> 109, 141 -> 106, 134 -> 103, 143 -> 100 us, half P S d D 161 -> 156,
+/// 135 -> 129, 139 -> 119, 138 -> 114, 127 -> 109, 125 -> 102; 60,000 points full 258 -> 273, 264 -> 202, 204 -> 170, 247 ->
+/// 150, 194 -> 147, 249 -> 137, half 252 -> 289, 212 -> 217, 205 -> 179, 200 -> 155, 191 -> 152, 208 -> 144; 300,000 points
+/// with 3 / 5 / 7 / 9 / 12 full 655 -> 751, 602 -> 541, 547 -> 453, 575 -> 413, 531 -> 487, half 642 -> 830, 558 -> 590, 525 ->
+/// 559, 514 -> 496, 512 -> 486. Well-filled tiles: 100,000 points, 26 per cell, half P S d D 297 -> 201 us; 1,000,000 atoms
+/// of diamond, full P S d 1615 -> 1287 us.
+inline bool ordered_by_tiles(size_t n_points, size_t tiles_before) {
+    const double points = static_cast<double>(n_points);
+    const double tiles = static_cast<double>(tiles_before);
+    return tiles_before > 0 && points >= (tiles_before <= 16384 ? 1.5 : 6.0) * tiles;
+}
+
+/// How the writing passes with a workgroup per tile (write_tile.cuh) store their rows.
+enum TileStores : int {
+    STORE_CACHED,     // through the caches
+    STORE_STREAMED,   // past them (non-temporal)
+    STORE_BY_GRANULE, // past them, but for the granules of 16 rows that a run of consecutive rows starts or ends in
+};
+
+/// A run of consecutive rows starts and ends in the middle of 64-byte pieces that other workgroups write the rest of. Stored
+/// past the caches, such a piece is written to memory twice, in parts, which costs several times what a whole one does;
+/// stored through them it is put together, in the L2 or in the 256 MB behind it, if both parts come while it is there.
+/// Whole pieces of lists larger than that are better off past the caches. Writing pass, past / through / by granule, us:
+///  - up to 200 MB: 60,000 points, 12 per cell, full P S d 48 / 36 / 44, P S d D 68 / 48 / 55; 100,000 points, 15 per cell,
+///    half P S d 57 / 44 / 56, 25 per cell, half P S 58 / 43 / 51; 30,000 points, 20 per cell, full P S d 37 / 30 / 33;
+///  - beyond, with vectors: 100,000 points, 26 per cell, half P S d D 108 / 88 / 78; 300,000 points, 20 per cell, full P S D
+///    377 / 428 / 309, P S d D 452 / 508 / 356;
+///  - with distances: 150,000 points, 20 per cell, full P S d 146 / 151 / 106, 300,000 points 285 / 318 / 278, diamond of
+///    110,592 atoms 107 / 101 / 84 and of 1,000,000 atoms 909 / 1030 / 840 (in random order 988 / 1255 / 1004); but 500,000
+///    points, 12 per cell, half (25 rows per point) 252 / 242 / 295: with nearly every row in such a granule, sorting them
+///    out is all that is left;
+///  - pairs alone 122 / 175 / 150, pairs and shifts 217 / 246 / 224 (300,000 points): the second set of stores costs more
+///    than it saves.
+inline TileStores tile_stores(size_t n_points, size_t rows, bool shifts, bool distances, bool vectors) {
+    const size_t row_bytes = 16 + (shifts ? 12 : 0) + (distances ? 8 : 0) + (vectors ? 24 : 0);
+    if (rows <= (size_t(200) << 20) / row_bytes) {
+        return STORE_CACHED;
+    }
+    return (vectors || distances) && rows / 40 >= n_points ? STORE_BY_GRANULE : STORE_STREAMED;
+}
+
+/// The same for crowded cells, whose points have their rows in many pieces, a chunk of candidates each: with distances alone
+/// what is sorted out costs more than it saves (clusters of 500,000 points, past the caches / by granule: P d 667 / 803, P S d
+/// 997 / 1004, P S d D 1603 / 1425 us).
+inline TileStores crowded_stores(size_t n_points, size_t rows, bool shifts, bool distances, bool vectors) {
+    const TileStores stores = tile_stores(n_points, rows, shifts, distances, vectors);
+    return stores == STORE_BY_GRANULE && !vectors ? STORE_STREAMED : stores;
 }
 
 } // namespace vesin_hip
