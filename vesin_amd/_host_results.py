@@ -1,0 +1,90 @@
+"""Results for callers that hold numpy arrays: the arrays of a call come to pinned host memory in one go, without a wait in
+between, and from there to memory of their own, each while the next ones are still on the way. (They are not handed out where
+they landed: pinned memory is not there for forked processes, and stays locked for as long as an array made of it lives.)
+
+The pinned memory is kept in a pool of at most ``LIMIT`` bytes for the whole process. Results that do not fit are copied one
+by one, and so are those of a calculator's first call (it does not pay for the pinned memory).
+"""
+
+import threading
+
+import numpy as np
+
+LIMIT = 64 << 20      # bytes of pinned memory, in use and kept
+SMALLEST = 1 << 20    # bytes of a block at least
+ALIGNMENT = 64        # of the arrays in a block
+# Results of up to this are waited for together: an event for each costs more than the overlap gives (216 atoms, 0.7 MB, per
+# call 256 us with, 160 without; the copies one by one 190. 1,728 atoms, 5.5 MB: 530 -> 400, 8,000 atoms 1710 -> 820 us)
+SMALL = 2 << 20
+
+
+class HostStaging:
+    def __init__(self):
+        self._lock = threading.Lock()
+        self._kept = []
+        self._held = 0
+
+    def _take(self, needed):
+        import torch
+
+        with self._lock:
+            fitting = [block for block in self._kept if block.numel() >= needed]
+            if fitting:
+                block = min(fitting, key=lambda b: b.numel())
+                self._kept = [other for other in self._kept if other is not block]
+                return block
+            size = max(SMALLEST, 1 << (needed - 1).bit_length())
+            while self._kept and self._held + size > LIMIT:
+                self._held -= self._kept.pop(0).numel()
+            if self._held + size > LIMIT:
+                return None
+            block = torch.empty(size, dtype=torch.uint8, pin_memory=True)
+            self._held += size
+            return block
+
+    def _give_back(self, block):
+        with self._lock:
+            self._kept.append(block)
+
+    def to_host(self, tensors, dtypes):
+        """The device tensors (contiguous, of one device) as numpy arrays of the given types of the same size, or None when
+        they do not fit."""
+        import torch
+
+        starts, needed = [], 0
+        for tensor in tensors:
+            starts.append(needed)
+            size = tensor.numel() * tensor.element_size()
+            needed += (size + ALIGNMENT - 1) // ALIGNMENT * ALIGNMENT
+        block = self._take(needed) if 0 < needed <= LIMIT else None
+        if block is None:
+            return None
+        stream = torch.cuda.current_stream(tensors[0].device)
+        in_one_go = needed <= SMALL
+        try:
+            landing, landed = [], []
+            for start, tensor in zip(starts, tensors):
+                size = tensor.numel() * tensor.element_size()
+                landing.append(block[start : start + size].view(tensor.dtype).view(tensor.shape))
+                landing[-1].copy_(tensor, non_blocking=True)
+                if not in_one_go:
+                    landed.append(stream.record_event())
+            if in_one_go:
+                stream.synchronize()
+                return [source.numpy().view(dtype).copy() for source, dtype in zip(landing, dtypes)]
+            arrays = []
+            for source, event, dtype in zip(landing, landed, dtypes):
+                array = np.empty(tuple(source.shape), dtype=dtype)
+                event.synchronize()
+                # (torch's copy: by several threads where the array is large)
+                torch.from_numpy(array.view(np.int64 if dtype == np.uint64 else dtype)).copy_(source)
+                arrays.append(array)
+            return arrays
+        except BaseException:
+            stream.synchronize() # (nothing is on its way into the block when it is given back)
+            raise
+        finally:
+            self._give_back(block)
+
+
+STAGING = HostStaging()

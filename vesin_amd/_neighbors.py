@@ -40,6 +40,7 @@ from ._c_api import (
     VesinUnknownDevice,
     get_library,
 )
+from ._host_results import STAGING as HOST_STAGING
 
 _HANDOVER = None
 
@@ -419,24 +420,54 @@ class NeighborList:
         if taken is not None:
             taken[1]()  # (the pairs of a call that asked for none of "ijP")
 
-        data = []
-        for quantity in quantities:
-            if quantity == "P":
-                data.append(to_result(pairs))
-            elif quantity == "i":
-                data.append(to_result(pairs[:, 0]))
-            elif quantity == "j":
-                data.append(to_result(pairs[:, 1]))
-            elif quantity == "S":
-                data.append(to_result(shifts))
-            elif quantity == "d":
-                data.append(to_result(distances))
-            elif quantity == "D":
-                data.append(to_result(vectors))
+        data = None
+        if not is_torch and n_pairs > 0:
+            data = self._host_results(quantities, pairs, shifts, distances, vectors)
+        if data is None:
+            data = []
+            for quantity in quantities:
+                if quantity == "P":
+                    data.append(to_result(pairs))
+                elif quantity == "i":
+                    data.append(to_result(pairs[:, 0]))
+                elif quantity == "j":
+                    data.append(to_result(pairs[:, 1]))
+                elif quantity == "S":
+                    data.append(to_result(shifts))
+                elif quantity == "d":
+                    data.append(to_result(distances))
+                elif quantity == "D":
+                    data.append(to_result(vectors))
         data = tuple(data)
         if not copy and n_pairs != 0:
             self._last_views = (result_key, data)
         return data
+
+    def _host_results(self, quantities, pairs, shifts, distances, vectors):
+        """The results as numpy arrays by way of pinned memory (from a calculator's second such call on), or None."""
+        import torch
+
+        if not self.__dict__.get("_host_called", False):
+            self._host_called = True
+            return None
+        tensors, dtypes = [], []
+        columns = None
+        for quantity in quantities:
+            if quantity in "ij":
+                if columns is None:
+                    columns = pairs.view(torch.int64).t().contiguous()
+                tensors.append(columns[0 if quantity == "i" else 1])
+                dtypes.append(np.uint64)
+            elif quantity == "P":
+                tensors.append(pairs.view(torch.int64))
+                dtypes.append(np.uint64)
+            elif quantity == "S":
+                tensors.append(shifts)
+                dtypes.append(np.int32)
+            elif quantity in "dD":
+                tensors.append(distances if quantity == "d" else vectors)
+                dtypes.append(np.float32 if tensors[-1].dtype == torch.float32 else np.float64)
+        return HOST_STAGING.to_host(tensors, dtypes) if tensors else None
 
     def compute_batch(self, points, first_point, boxes, periodic=True, quantities: str = "ij", copy: bool = True):
         """Neighbor lists of many systems in one go (``vesin_hip_neighbors_batch``).
