@@ -11,6 +11,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <type_traits>
 
 #include "device_common.cuh"
 
@@ -20,6 +21,11 @@ namespace vesin_hip {
 // 58 KB of LDS, so two workgroups share a compute unit: with 256 threads each, too few loads are in flight, with 1024
 // the waves wait for each other where the table is filled and emptied (89 M rows, gradient of the distances: 1484 /
 // 1056 / 1115 us with 256 / 512 / 1024 threads).
+//
+// With the next rows read while these go to the table, and runs of one first point summed without the LDS (shuffles do go
+// through it), 89 M rows, gradient of the distances, by the order of the list: unsorted 1095 -> 1042 us, sorted 1148 -> 974;
+// the reads alone take 810 and 890 us. Fewer bytes do not help any more (distances computed again from the vectors: the
+// same), nor do 1024 threads (1090, 1180) or half the table for a third workgroup (1065, 1220).
 constexpr int BACKWARD_THREADS = 512;
 
 struct BackwardArgs {
@@ -46,23 +52,34 @@ __device__ inline double wave_sum(double value) {
     return value;
 }
 
-/// Sums a run of lanes that name the same point into the first lane of the run. `heads` has one bit per lane that
-/// starts a run; afterwards the sums of a run stand in its first lane.
+/// One step of a sum over runs: adds what the lane `CTRL` names (a DPP control, for the rows of `ROW_MASK`) holds, where that
+/// lane belongs to the same run.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ double add_from(double value, bool same_run) {
+    const uint64_t there = dpp_or_zero64<CTRL, ROW_MASK>(static_cast<uint64_t>(__double_as_longlong(value)));
+    return value + (same_run ? __longlong_as_double(static_cast<long long>(there)) : 0.0);
+}
+
+/// Sums a run of lanes that name the same point into the last lane of the run. `heads` has one bit per lane that starts a
+/// run. (Data moves with DPP only: with shuffles, which go through the LDS that the table is in, see pairs_backward_kernel.)
 __device__ inline void sum_runs(uint64_t heads, double& gx, double& gy, double& gz) {
     const uint32_t lane = static_cast<uint32_t>(lane_id());
-    const uint64_t after = lane == 63 ? 0 : (heads >> (lane + 1)) << (lane + 1);
-    const uint32_t run_end = after == 0 ? 64u : static_cast<uint32_t>(__builtin_ctzll(after));
-#pragma unroll
-    for (int offset = 1; offset < 64; offset <<= 1) {
-        const double ox = __shfl_down(gx, offset, WAVE);
-        const double oy = __shfl_down(gy, offset, WAVE);
-        const double oz = __shfl_down(gz, offset, WAVE);
-        if (lane + offset < run_end) {
-            gx += ox;
-            gy += oy;
-            gz += oz;
-        }
-    }
+    const uint64_t up_to_here = heads & (~0ull >> (63 - lane));
+    const uint32_t start = 63u - static_cast<uint32_t>(__builtin_clzll(up_to_here)); // (lane 0 starts a run)
+    auto step = [&](auto control, auto row_mask, bool same_run) {
+        constexpr int CTRL = decltype(control)::value;
+        constexpr int ROW_MASK = decltype(row_mask)::value;
+        gx = add_from<CTRL, ROW_MASK>(gx, same_run);
+        gy = add_from<CTRL, ROW_MASK>(gy, same_run);
+        gz = add_from<CTRL, ROW_MASK>(gz, same_run);
+    };
+    const uint32_t in_row = lane % 16;
+    step(std::integral_constant<int, 0x111>(), std::integral_constant<int, 0xf>(), in_row >= 1 && start + 1 <= lane);
+    step(std::integral_constant<int, 0x112>(), std::integral_constant<int, 0xf>(), in_row >= 2 && start + 2 <= lane);
+    step(std::integral_constant<int, 0x114>(), std::integral_constant<int, 0xf>(), in_row >= 4 && start + 4 <= lane);
+    step(std::integral_constant<int, 0x118>(), std::integral_constant<int, 0xf>(), in_row >= 8 && start + 8 <= lane);
+    step(std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xa>(), lane / 16 % 2 == 1 && start < lane - in_row);
+    step(std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xc>(), lane >= 32 && start < 32);
 }
 
 /// Sums of one workgroup, by point, in LDS: rows that follow each other in a list name few different points (the
@@ -143,36 +160,57 @@ __global__ __launch_bounds__(BACKWARD_THREADS) void pairs_backward_kernel(Backwa
     // over runs use the whole wave)
     const size_t block_first = static_cast<size_t>(blockIdx.x) * args.rows_per_block;
     const size_t block_end = min(block_first + args.rows_per_block, args.n_pairs);
-    for (size_t base = block_first + (threadIdx.x & ~(WAVE - 1)); base < block_end; base += BACKWARD_THREADS) {
+    // (the next row of a lane is read while the sums of this one go to the table)
+    struct Row {
+        size_t i, j;
+        double dg, d, vx, vy, vz, gx, gy, gz;
+    };
+    auto read = [&](size_t row) {
+        Row r = {~size_t(0), 0, 0.0, 1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        if (row < block_end) {
+            r.i = args.pairs[row][0];
+            r.j = args.pairs[row][1];
+            if (args.vectors_grad != nullptr) {
+                r.gx = args.vectors_grad[row][0];
+                r.gy = args.vectors_grad[row][1];
+                r.gz = args.vectors_grad[row][2];
+            }
+            if (args.distances_grad != nullptr) {
+                r.dg = args.distances_grad[row];
+                r.d = args.distances[row];
+                r.vx = args.vectors[row][0];
+                r.vy = args.vectors[row][1];
+                r.vz = args.vectors[row][2];
+            }
+        }
+        return r;
+    };
+    const size_t wave_first = block_first + (threadIdx.x & ~(WAVE - 1));
+    Row next = read(wave_first + lane);
+    for (size_t base = wave_first; base < block_end; base += BACKWARD_THREADS) {
         const size_t row = base + lane;
+        const Row here = next;
+        next = read(row + BACKWARD_THREADS);
         bool active = row < block_end;
         // rows that do not count carry an index no point has, so that they never join the run of a neighbour
-        size_t i = ~size_t(0);
-        size_t j = 0;
+        size_t i = here.i;
+        const size_t j = here.j;
         double gx = 0.0;
         double gy = 0.0;
         double gz = 0.0;
-        if (active) {
-            i = args.pairs[row][0];
-            j = args.pairs[row][1];
-            if (i >= args.n_points || j >= args.n_points) {
-                *args.bad_index = 1;
-                active = false;
-                i = ~size_t(0);
-            }
+        if (active && (i >= args.n_points || j >= args.n_points)) {
+            *args.bad_index = 1;
+            active = false;
+            i = ~size_t(0);
         }
         if (active) {
-            if (args.vectors_grad != nullptr) {
-                gx = args.vectors_grad[row][0];
-                gy = args.vectors_grad[row][1];
-                gz = args.vectors_grad[row][2];
-            }
+            gx = here.gx;
+            gy = here.gy;
+            gz = here.gz;
             if (args.distances_grad != nullptr) {
-                const double dg = args.distances_grad[row];
-                const double d = args.distances[row];
-                gx += dg * args.vectors[row][0] / d;
-                gy += dg * args.vectors[row][1] / d;
-                gz += dg * args.vectors[row][2] / d;
+                gx += here.dg * here.vx / here.d;
+                gy += here.dg * here.vy / here.d;
+                gz += here.dg * here.vz / here.d;
             }
             if (args.shifts != nullptr) {
                 const int32_t s0 = args.shifts[row][0];
@@ -205,7 +243,7 @@ __global__ __launch_bounds__(BACKWARD_THREADS) void pairs_backward_kernel(Backwa
             bool add = active;
             if (__popcll(heads) <= 32) {
                 sum_runs(heads, mx, my, mz);
-                add = active && head;
+                add = active && (lane == 63 || (heads >> (lane + 1) & 1u) != 0);
             }
             if (add) {
                 add_to_point(shared, args.points_grad, i, mx, my, mz);
