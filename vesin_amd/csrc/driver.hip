@@ -238,7 +238,7 @@ static bool fresh_extent_only() {
 }
 
 /// VESIN_HIP_STREAMS=one keeps every kernel of a call on the call's stream (for comparisons and tests); otherwise the
-/// in-order search orders the candidates of the tiles on a second stream while it counts the rows.
+/// in-order search with a wave per tile orders the candidates of the tiles on a second stream while it counts the rows.
 static bool ordered_one_stream() {
     const char* text = std::getenv("VESIN_HIP_STREAMS");
     return text != nullptr && std::strcmp(text, "one") == 0;

@@ -21,6 +21,9 @@
 // +-255 are reported in the status and the host goes on with the search for crowded cells (crowded.cuh) where that covers the
 // system, or with the unsorted search followed by the radix sort.
 //
+// From a list's second call on a system most systems take COUNT and SORT in one kernel and a workgroup per tile
+// (ordered_tile.cuh), with the same layout of points and records.
+//
 // Arithmetic as everywhere (vesin/src/cpu_cell_list.cpp:135-138, vesin/src/types.hpp:232-243):
 // S = cell shift - wrap_j + wrap_i, T = S . H left to right, v = (r_j - r_i) + T, d2 = vx*vx + vy*vy + vz*vz,
 // keep iff d2 < cutoff^2.
