@@ -48,6 +48,8 @@ def probe(tmp_path_factory):
     for name in ("probe_ordered_write_split", "probe_ordered_count_split"):
         getattr(lib, name).argtypes = [ctypes.c_size_t, ctypes.c_size_t]
         getattr(lib, name).restype = ctypes.c_uint
+    lib.probe_ordered_by_tiles.argtypes = [ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int]
+    lib.probe_ordered_by_tiles.restype = ctypes.c_int
     return lib
 
 
@@ -387,6 +389,21 @@ def test_waves_per_tile_of_the_two_passes(probe):
             assert count(tiles * per_tile, tiles) in (1, 2)
             if per_tile < 16:
                 assert write(tiles * per_tile, tiles) == 1 and count(tiles * per_tile, tiles) == 1
+
+
+# (points, tiles, vectors returned, time of a call with a workgroup per tile over that with a wave per tile or share of one):
+# liquids, measured in turn; the largest ratio of full and half lists
+@pytest.mark.parametrize("n_points, tiles, vectors, ratio", [
+    (30_000, 16_355, True, 1.16), (30_000, 16_355, False, 1.12), (25_000, 15_639, True, 1.14), (30_000, 15_396, False, 1.09),
+    (40_000, 14_417, True, 1.12), (20_000, 12_558, True, 1.07), (50_000, 14_988, True, 1.07), (60_000, 18_749, False, 1.05),
+    (300_000, 72_796, True, 1.25), (300_000, 72_796, False, 1.12), (400_000, 63_876, True, 1.05), (60_000, 30_652, False, 1.24),
+    (6_000, 3_985, True, 0.85), (10_000, 6_116, True, 0.90), (15_000, 9_176, False, 0.97), (20_000, 9_806, False, 0.94),
+    (60_000, 13_644, False, 0.93), (60_000, 10_600, True, 0.91), (150_000, 24_337, True, 0.88), (300_000, 39_285, True, 0.92),
+    (1_000_000, 165_967, False, 0.93), (100_000, 4_260, True, 0.70), (1_000_000, 43_000, False, 0.80),
+])
+def test_a_workgroup_per_tile_where_it_is_faster(probe, n_points, tiles, vectors, ratio):
+    assert bool(probe.probe_ordered_by_tiles(n_points, tiles, int(vectors))) == (ratio < 1.0)
+    assert not probe.probe_ordered_by_tiles(n_points, 0, int(vectors))  # not known
 
 
 def run_wait_rest(probe, gives_up):

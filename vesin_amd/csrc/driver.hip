@@ -2042,7 +2042,8 @@ bool compute(
     // (from a list's second call on the same number of points: a workgroup per tile, ordered_tile.cuh)
     const size_t tiles_known = extras.ordered_tiles_points == n_points ? extras.ordered_tiles : 0;
     const bool by_tiles = std::getenv("VESIN_HIP_WRITE_SPLIT") == nullptr && std::getenv("VESIN_HIP_COUNT_SPLIT") == nullptr &&
-                          std::getenv("VESIN_HIP_ORDERED_SHARE") == nullptr && ordered_by_tiles(n_points, tiles_known);
+                          std::getenv("VESIN_HIP_ORDERED_SHARE") == nullptr &&
+                          ordered_by_tiles(n_points, tiles_known, options.return_vectors);
     const uint32_t ordered_blocks =
         static_cast<uint32_t>((tiles_bound * ordered_items_per_tile + ORDERED_WAVES - 1) / ORDERED_WAVES);
     const size_t ordered_record_bytes =

@@ -3,6 +3,7 @@
 #ifndef VESIN_HIP_POLICY_HPP
 #define VESIN_HIP_POLICY_HPP
 
+#include <algorithm>
 #include <cstddef>
 
 namespace vesin_hip {
@@ -274,18 +275,24 @@ inline unsigned int ordered_count_split(size_t n_points, size_t tiles_before) {
 /// Whether the search gives every tile a workgroup (ordered_tile.cuh) in place of a wave or several (ordered.cuh), from the
 /// number of tiles the call before had on the same points (0: not known, and a wave per tile).
 ///
-/// Its kernels are the faster ones but for many tiles of few points, where most of a workgroup has nothing to do. Per call, a
-/// wave per tile or share of a tile -> a workgroup per tile, cutoff 5, liquids with 1.5 / 3 / 5 / 7 / 9 / 12 points per cell:
-/// 20,000 points full P S d 160 -> 147, 139 -> 130, 181 -> 109, 141 -> 106, 134 -> 103, 143 -> 100 us, half P S d D 161 -> 156,
-/// 135 -> 129, 139 -> 119, 138 -> 114, 127 -> 109, 125 -> 102; 60,000 points full 258 -> 273, 264 -> 202, 204 -> 170, 247 ->
-/// 150, 194 -> 147, 249 -> 137, half 252 -> 289, 212 -> 217, 205 -> 179, 200 -> 155, 191 -> 152, 208 -> 144; 300,000 points
-/// with 3 / 5 / 7 / 9 / 12 full 655 -> 751, 602 -> 541, 547 -> 453, 575 -> 413, 531 -> 487, half 642 -> 830, 558 -> 590, 525 ->
-/// 559, 514 -> 496, 512 -> 486. Well-filled tiles: 100,000 points, 26 per cell, half P S d D 297 -> 201 us; 1,000,000 atoms
-/// of diamond, full P S d 1615 -> 1287 us.
-inline bool ordered_by_tiles(size_t n_points, size_t tiles_before) {
+/// Its kernels are the faster ones but for many tiles of few points, where most of a workgroup has nothing to do: the more
+/// tiles, the better the waves of the other way fill the chip by themselves, and the kernels of lists with vectors leave room
+/// for fewer workgroups (write_tile.cuh). Full and half lists cross at the same points per tile. The line follows where both
+/// ways took the same for liquids of 3,000 to 1,000,000 points (cutoffs 3.5 and 5): without vectors 1.5 points per tile at
+/// 9,000 tiles, 2.8 at 14,400, 3.5 at 18,700, 5 from 59,000 on; with vectors 1.5 at 8,000, 2.4 at 10,600, 3.5 at 11,700, 5 to 6
+/// from 16,400 on, 6.3 at 64,000. Calls, a wave per tile or share of one -> a workgroup per tile, us:
+///  - below the line: full P S d D, 1.8 points in each of 16,400 tiles 162 -> 187, 2.8 of 14,400 164 -> 183, 4.1 of 72,800 588 ->
+///    698; half P S d D, 2.0 of 15,400 153 -> 174, 6.3 of 63,900 657 -> 689; full P S d, 2.0 of 15,400 152 -> 163;
+///  - above it: full P S d D, 5.7 of 10,600 193 -> 172; half P S d D, 7.6 of 39,300 524 -> 466; full P S d, 3.2 of 4,700 126 ->
+///    105, 4.4 of 13,600 193 -> 172, 6.0 of 166,000 1725 -> 1518; 100,000 points, 26 per cell, half P S d D 297 -> 201;
+///    1,000,000 atoms of diamond, full P S d 1615 -> 1287.
+inline bool ordered_by_tiles(size_t n_points, size_t tiles_before, bool vectors) {
     const double points = static_cast<double>(n_points);
     const double tiles = static_cast<double>(tiles_before);
-    return tiles_before > 0 && points >= (tiles_before <= 16384 ? 1.5 : 6.0) * tiles;
+    const double wanted = !vectors         ? std::min(5.0, 1.5 + (tiles - 9000.0) / 4000.0)
+                          : tiles > 40000.0 ? 6.5
+                                            : std::min(6.0, 1.5 + (tiles - 8000.0) / 1300.0);
+    return tiles_before > 0 && points >= std::max(1.5, wanted) * tiles;
 }
 
 /// How the writing passes with a workgroup per tile (write_tile.cuh) store their rows.
