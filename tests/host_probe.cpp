@@ -195,6 +195,8 @@ extern "C" void probe_crowded_room(size_t n_points, const size_t* counted, size_
     }
 }
 
+extern "C" size_t probe_backward_rows_per_block(size_t n_pairs) { return vesin_hip::backward_rows_per_block(n_pairs); }
+
 extern "C" int probe_ordered_records_fit(size_t n_points, size_t record_bytes) {
     return vesin_hip::ordered_records_fit(n_points, record_bytes) ? 1 : 0;
 }

@@ -50,6 +50,8 @@ def probe(tmp_path_factory):
         getattr(lib, name).restype = ctypes.c_uint
     lib.probe_ordered_by_tiles.argtypes = [ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int]
     lib.probe_ordered_by_tiles.restype = ctypes.c_int
+    lib.probe_backward_rows_per_block.argtypes = [ctypes.c_size_t]
+    lib.probe_backward_rows_per_block.restype = ctypes.c_size_t
     return lib
 
 
@@ -404,6 +406,23 @@ def test_waves_per_tile_of_the_two_passes(probe):
 def test_a_workgroup_per_tile_where_it_is_faster(probe, n_points, tiles, vectors, ratio):
     assert bool(probe.probe_ordered_by_tiles(n_points, tiles, int(vectors))) == (ratio < 1.0)
     assert not probe.probe_ordered_by_tiles(n_points, 0, int(vectors))  # not known
+
+
+def test_rows_of_a_gradient_are_dealt_out_in_whole_rounds(probe):
+    """512 workgroups run at a time: the last round of a list of more than two rounds' smallest workgroups is nearly full, where
+    one that holds a third of them (6.3 M rows in 767 workgroups) cost as much as a full one."""
+    for n_pairs in [1, 511, 512, 513, 262_144, 524_288, 4_194_304, 4_194_305, 8_388_608, 8_388_609, 2**32 + 7] + [
+        int(n) for n in np.geomspace(600_000, 2e9, 400)
+    ]:
+        rows = probe.probe_backward_rows_per_block(n_pairs)
+        assert rows % 512 == 0 and 512 <= rows <= 8192
+        workgroups = -(-n_pairs // rows)
+        # (rounding up to 512 rows leaves out up to 512 / rows of the workgroups)
+        rounds = max(2, -(-n_pairs // (512 * 8192)))
+        assert workgroups <= 512 * rounds
+        if rows > 512:
+            assert workgroups > 512 * rounds * (1 - 512 / rows)
+    assert probe.probe_backward_rows_per_block(6_284_114) == 6_144  # not 767 workgroups of 8192
 
 
 def run_wait_rest(probe, gives_up):

@@ -14,6 +14,7 @@
 #include <type_traits>
 
 #include "device_common.cuh"
+#include "policy.hpp"
 
 namespace vesin_hip {
 
@@ -27,6 +28,7 @@ namespace vesin_hip {
 // the reads alone take 810 and 890 us. Fewer bytes do not help any more (distances computed again from the vectors: the
 // same), nor do 1024 threads (1090, 1180) or half the table for a third workgroup (1065, 1220).
 constexpr int BACKWARD_THREADS = 512;
+static_assert(BACKWARD_ROWS % BACKWARD_THREADS == 0 && BACKWARD_STEP % BACKWARD_THREADS == 0, "whole rounds of the threads");
 
 struct BackwardArgs {
     const size_t (*pairs)[2];
@@ -40,7 +42,7 @@ struct BackwardArgs {
     double* points_grad;           // [n_points][3] or nullptr
     double* box_grad;              // [3][3] or nullptr
     uint32_t* bad_index;           // set to 1 when a pair names a point that does not exist
-    size_t rows_per_block;         // a multiple of BACKWARD_THREADS (see backward_rows_per_block)
+    size_t rows_per_block;         // a multiple of BACKWARD_THREADS (backward_rows_per_block, policy.hpp)
 };
 
 /// Sum over the 64 lanes of a wave, result in every lane.
@@ -96,18 +98,6 @@ constexpr uint32_t BACKWARD_SLOTS = 2048;
 constexpr uint32_t BACKWARD_GROUP = 8;
 constexpr uint32_t BACKWARD_PROBES = 8;
 constexpr uint32_t BACKWARD_EMPTY = 0xFFFFFFFFu;
-
-/// Rows that one workgroup takes. Many rows let more additions meet in the table (1,000,000 atoms of diamond, 89 M rows,
-/// gradient of the distances: 1190 / 1098 / 1064 us with 2048 / 4096 / 8192 rows, 1101 with 16384); lists of fewer rows
-/// go for two workgroups on every one of the 256 compute units (50,000 atoms, 2.1 M rows, everything asked for: 55.6 /
-/// 47.7 / 46.1 / 57.4 us with 1024 / 2048 / 4096 / 8192 rows; sorted, of atoms in no order: 147 / 157 / 211 / 250 us).
-inline size_t backward_rows_per_block(size_t n_pairs) {
-    size_t rows = 8192;
-    while (rows > static_cast<size_t>(BACKWARD_THREADS) && n_pairs / rows < 512) {
-        rows /= 2;
-    }
-    return rows;
-}
 
 struct BackwardShared {
     uint32_t keys[BACKWARD_SLOTS];

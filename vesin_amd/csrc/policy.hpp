@@ -332,6 +332,25 @@ inline TileStores crowded_stores(size_t n_points, size_t rows, bool shifts, bool
     return stores == STORE_BY_GRANULE && !vectors ? STORE_STREAMED : stores;
 }
 
+constexpr size_t BACKWARD_ROWS = 8192;    // of a workgroup at most
+constexpr size_t BACKWARD_STEP = 512;     // and a multiple of this
+constexpr size_t BACKWARD_RESIDENT = 512; // workgroups at a time: two on each of 256 compute units
+
+/// Rows that one workgroup of the gradient's kernel (backward.cuh) takes. Many rows let more additions meet in its table
+/// (1,000,000 atoms of diamond, 89 M rows, gradient of the distances: 1190 / 1098 / 1064 us with 2048 / 4096 / 8192 rows, 1101
+/// with 16384). The rows are dealt out evenly over as few times BACKWARD_RESIDENT workgroups as that allows, but at least
+/// two: a last round of a few workgroups takes as long as a full one. Powers of two, 512 to 1,023 workgroups up to 8.4 M rows
+/// -> dealt out evenly, us: 0.7 M rows, half list, gradient of the distances and the box 46 -> 46; 2.7 M rows, full list,
+/// distances 74 -> 66, vectors 75 -> 66; 4.5 M rows 113 -> 92 and 110 -> 90; 6.3 M rows 144 -> 122 and 138 -> 114, points in no
+/// order 728 -> 688; 13.6 M rows 244 -> 231; 36 M rows 584 -> 580. (At least one round: half lists of 0.7 M rows 46 -> 38, but
+/// points in no order 1.4 M rows 106 -> 124, where two rounds take 100.)
+inline size_t backward_rows_per_block(size_t n_pairs) {
+    const size_t most = BACKWARD_RESIDENT * BACKWARD_ROWS;
+    const size_t rounds = std::max<size_t>(2, n_pairs / most + (n_pairs % most != 0));
+    const size_t rows = (n_pairs - 1) / (BACKWARD_RESIDENT * rounds) + 1;
+    return (rows + BACKWARD_STEP - 1) / BACKWARD_STEP * BACKWARD_STEP;
+}
+
 } // namespace vesin_hip
 
 #endif
