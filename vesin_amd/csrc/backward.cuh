@@ -23,10 +23,11 @@ namespace vesin_hip {
 // the waves wait for each other where the table is filled and emptied (89 M rows, gradient of the distances: 1484 /
 // 1056 / 1115 us with 256 / 512 / 1024 threads).
 //
-// With the next rows read while these go to the table, and runs of one first point summed without the LDS (shuffles do go
-// through it), 89 M rows, gradient of the distances, by the order of the list: unsorted 1095 -> 1042 us, sorted 1148 -> 974;
-// the reads alone take 810 and 890 us. Fewer bytes do not help any more (distances computed again from the vectors: the
-// same), nor do 1024 threads (1090, 1180) or half the table for a third workgroup (1065, 1220).
+// Runs of one first point are summed without the LDS (shuffles do go through it), and all loads of a row are issued before
+// its indices are looked at: 89 M rows, gradient of the distances, whole calls by the order of the list, unsorted 1436 -> 1334
+// (sums) -> 1268 us (loads), sorted 1144 -> 1056 -> 963; the reads alone take 810 and 890 us. Reading the next rows ahead
+// gives nothing on top (1274, 975), fewer bytes do not help any more (distances computed again from the vectors: the same),
+// nor do 1024 threads or half the table for a third workgroup (5 to 25 % slower).
 constexpr int BACKWARD_THREADS = 512;
 static_assert(BACKWARD_ROWS % BACKWARD_THREADS == 0 && BACKWARD_STEP % BACKWARD_THREADS == 0, "whole rounds of the threads");
 
@@ -150,57 +151,40 @@ __global__ __launch_bounds__(BACKWARD_THREADS) void pairs_backward_kernel(Backwa
     // over runs use the whole wave)
     const size_t block_first = static_cast<size_t>(blockIdx.x) * args.rows_per_block;
     const size_t block_end = min(block_first + args.rows_per_block, args.n_pairs);
-    // (the next row of a lane is read while the sums of this one go to the table)
-    struct Row {
-        size_t i, j;
-        double dg, d, vx, vy, vz, gx, gy, gz;
-    };
-    auto read = [&](size_t row) {
-        Row r = {~size_t(0), 0, 0.0, 1.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        if (row < block_end) {
-            r.i = args.pairs[row][0];
-            r.j = args.pairs[row][1];
-            if (args.vectors_grad != nullptr) {
-                r.gx = args.vectors_grad[row][0];
-                r.gy = args.vectors_grad[row][1];
-                r.gz = args.vectors_grad[row][2];
-            }
-            if (args.distances_grad != nullptr) {
-                r.dg = args.distances_grad[row];
-                r.d = args.distances[row];
-                r.vx = args.vectors[row][0];
-                r.vy = args.vectors[row][1];
-                r.vz = args.vectors[row][2];
-            }
-        }
-        return r;
-    };
-    const size_t wave_first = block_first + (threadIdx.x & ~(WAVE - 1));
-    Row next = read(wave_first + lane);
-    for (size_t base = wave_first; base < block_end; base += BACKWARD_THREADS) {
+    for (size_t base = block_first + (threadIdx.x & ~(WAVE - 1)); base < block_end; base += BACKWARD_THREADS) {
         const size_t row = base + lane;
-        const Row here = next;
-        next = read(row + BACKWARD_THREADS);
         bool active = row < block_end;
         // rows that do not count carry an index no point has, so that they never join the run of a neighbour
-        size_t i = here.i;
-        const size_t j = here.j;
-        double gx = 0.0;
-        double gy = 0.0;
-        double gz = 0.0;
-        if (active && (i >= args.n_points || j >= args.n_points)) {
-            *args.bad_index = 1;
-            active = false;
-            i = ~size_t(0);
+        size_t i = ~size_t(0);
+        size_t j = 0;
+        double gx = 0.0, gy = 0.0, gz = 0.0;
+        double dg = 0.0, d = 1.0, vx = 0.0, vy = 0.0, vz = 0.0;
+        if (active) { // (all loads of the row, none of which waits for another)
+            i = args.pairs[row][0];
+            j = args.pairs[row][1];
+            if (args.vectors_grad != nullptr) {
+                gx = args.vectors_grad[row][0];
+                gy = args.vectors_grad[row][1];
+                gz = args.vectors_grad[row][2];
+            }
+            if (args.distances_grad != nullptr) {
+                dg = args.distances_grad[row];
+                d = args.distances[row];
+                vx = args.vectors[row][0];
+                vy = args.vectors[row][1];
+                vz = args.vectors[row][2];
+            }
+            if (i >= args.n_points || j >= args.n_points) {
+                *args.bad_index = 1;
+                active = false;
+                i = ~size_t(0);
+            }
         }
         if (active) {
-            gx = here.gx;
-            gy = here.gy;
-            gz = here.gz;
             if (args.distances_grad != nullptr) {
-                gx += here.dg * here.vx / here.d;
-                gy += here.dg * here.vy / here.d;
-                gz += here.dg * here.vz / here.d;
+                gx += dg * vx / d;
+                gy += dg * vy / d;
+                gz += dg * vz / d;
             }
             if (args.shifts != nullptr) {
                 const int32_t s0 = args.shifts[row][0];
