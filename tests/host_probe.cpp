@@ -195,6 +195,10 @@ extern "C" void probe_crowded_room(size_t n_points, const size_t* counted, size_
     }
 }
 
+extern "C" int probe_crowded_stores(size_t n_points, size_t rows, int shifts, int distances, int vectors) {
+    return vesin_hip::crowded_stores(n_points, rows, shifts != 0, distances != 0, vectors != 0);
+}
+
 extern "C" size_t probe_backward_rows_per_block(size_t n_pairs) { return vesin_hip::backward_rows_per_block(n_pairs); }
 
 extern "C" int probe_ordered_records_fit(size_t n_points, size_t record_bytes) {

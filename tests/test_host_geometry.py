@@ -50,6 +50,8 @@ def probe(tmp_path_factory):
         getattr(lib, name).restype = ctypes.c_uint
     lib.probe_ordered_by_tiles.argtypes = [ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int]
     lib.probe_ordered_by_tiles.restype = ctypes.c_int
+    lib.probe_crowded_stores.argtypes = [ctypes.c_size_t, ctypes.c_size_t] + [ctypes.c_int] * 3
+    lib.probe_crowded_stores.restype = ctypes.c_int
     lib.probe_backward_rows_per_block.argtypes = [ctypes.c_size_t]
     lib.probe_backward_rows_per_block.restype = ctypes.c_size_t
     return lib
@@ -423,6 +425,24 @@ def test_rows_of_a_gradient_are_dealt_out_in_whole_rounds(probe):
         if rows > 512:
             assert workgroups > 512 * rounds * (1 - 512 / rows)
     assert probe.probe_backward_rows_per_block(6_284_114) == 6_144  # not 767 workgroups of 8192
+
+
+CACHED, STREAMED, BY_GRANULE = range(3)
+
+
+@pytest.mark.parametrize("n_points, rows, quantities, stores", [
+    (500_000, 39_112_722, "SdD", STREAMED),   # by granule 1.07 times as long as streamed
+    (500_000, 57_912_212, "SdD", STREAMED),   # 1.09
+    (500_000, 37_524_730, "D", STREAMED),     # 1.06
+    (300_000, 24_760_394, "D", STREAMED),     # 1.05
+    (300_000, 24_760_394, "SdD", STREAMED),   # 1.04
+    (100_000, 16_484_976, "SdD", BY_GRANULE), # 0.95
+    (50_000, 20_267_794, "SdD", BY_GRANULE),  # 0.95
+    (50_000, 20_267_794, "Sd", STREAMED),
+    (100_000, 2_000_000, "SdD", CACHED),
+])
+def test_how_the_rows_of_crowded_cells_are_stored(probe, n_points, rows, quantities, stores):
+    assert probe.probe_crowded_stores(n_points, rows, *(int(q in quantities) for q in "SdD")) == stores
 
 
 def run_wait_rest(probe, gives_up):

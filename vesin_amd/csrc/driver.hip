@@ -202,8 +202,6 @@ static bool radix_sort_only() {
     return text != nullptr && std::strcmp(text, "radix") == 0;
 }
 
-/// VESIN_HIP_SORT=crowded sends every sorted list of one system to the in-order search for crowded cells (for
-/// comparisons and tests).
 template <bool VECTORS>
 static auto ordered_write_kernel_for(TileStores stores) {
     return stores == STORE_CACHED       ? ordered_write_kernel<VECTORS, STORE_CACHED>
@@ -211,13 +209,18 @@ static auto ordered_write_kernel_for(TileStores stores) {
                                         : ordered_write_kernel<VECTORS, STORE_STREAMED>;
 }
 
-template <bool VECTORS>
-static auto crowded_write_kernel_for(TileStores stores) {
-    return stores == STORE_CACHED       ? crowded_write_kernel<VECTORS, STORE_CACHED>
-           : stores == STORE_BY_GRANULE ? crowded_write_kernel<VECTORS, STORE_BY_GRANULE>
-                                        : crowded_write_kernel<VECTORS, STORE_STREAMED>;
+/// (crowded_stores, policy.hpp: by granule with vectors only)
+static auto crowded_write_kernel_for(TileStores stores, bool vectors) {
+    if (!vectors) {
+        return stores == STORE_CACHED ? crowded_write_kernel<false, STORE_CACHED> : crowded_write_kernel<false, STORE_STREAMED>;
+    }
+    return stores == STORE_CACHED       ? crowded_write_kernel<true, STORE_CACHED>
+           : stores == STORE_BY_GRANULE ? crowded_write_kernel<true, STORE_BY_GRANULE>
+                                        : crowded_write_kernel<true, STORE_STREAMED>;
 }
 
+/// VESIN_HIP_SORT=crowded sends every sorted list of one system to the in-order search for crowded cells (for
+/// comparisons and tests).
 static bool crowded_search_only() {
     const char* text = std::getenv("VESIN_HIP_SORT");
     return text != nullptr && std::strcmp(text, "crowded") == 0;
@@ -2748,7 +2751,7 @@ bool compute(
             auto launch_write = [&](size_t rows) {
                 const TileStores stores =
                     crowded_stores(n_points, rows, options.return_shifts, options.return_distances, options.return_vectors);
-                auto kernel = options.return_vectors ? crowded_write_kernel_for<true>(stores) : crowded_write_kernel_for<false>(stores);
+                auto kernel = crowded_write_kernel_for(stores, options.return_vectors);
                 hipLaunchKernelGGL(kernel, dim3(tile_blocks), dim3(TILE_BLOCK), 0, stream, cargs, g);
             };
             if (attempt > 0) {

@@ -324,12 +324,17 @@ inline TileStores tile_stores(size_t n_points, size_t rows, bool shifts, bool di
     return (vectors || distances) && rows / 40 >= n_points ? STORE_BY_GRANULE : STORE_STREAMED;
 }
 
-/// The same for crowded cells, whose points have their rows in many pieces, a chunk of candidates each: with distances alone
-/// what is sorted out costs more than it saves (clusters of 500,000 points, past the caches / by granule: P d 667 / 803, P S d
-/// 997 / 1004, P S d D 1603 / 1425 us).
+/// The same for crowded cells, whose tiles are written in the order of the cells: the two runs that share a granule are most
+/// often far apart in time, so the granules that wait for their second part, one per point, have to stay in the 256 MB
+/// behind the L2 together with what else goes there. Without vectors sorting them out costs more than it saves. Calls on
+/// clusters, past the caches / by granule, us: full P S d D, 50,000 points (20 M rows) 675 / 638, 100,000 (16 M) 589 / 559,
+/// 300,000 (25 M) 843 / 872, 500,000 (58 M) 1349 / 1470, (82 M) 1782 / 1825; half 100,000 (11 M) 552 / 516, 500,000 (29 M) 1157 / 1260;
+/// full P D, 300,000 (25 M) 802 / 838; P d, 500,000 points, writing pass 667 / 803.
 inline TileStores crowded_stores(size_t n_points, size_t rows, bool shifts, bool distances, bool vectors) {
     const TileStores stores = tile_stores(n_points, rows, shifts, distances, vectors);
-    return stores == STORE_BY_GRANULE && !vectors ? STORE_STREAMED : stores;
+    const size_t granule_bytes = 16 * (16 + (shifts ? 12 : 0) + (distances ? 8 : 0) + 24);
+    const bool stay = n_points <= (size_t(128) << 20) / granule_bytes;
+    return stores == STORE_BY_GRANULE && !(vectors && stay) ? STORE_STREAMED : stores;
 }
 
 constexpr size_t BACKWARD_ROWS = 8192;    // of a workgroup at most
