@@ -39,6 +39,29 @@ def test_beyond_the_limit_and_without_rows(monkeypatch):
         assert i.shape == (0,) and S.shape == (0, 3) and d.shape == (0,)
 
 
+@pytest.mark.parametrize("quantities", ["ij", "jd", "PSdDi"])
+def test_nothing_is_made_for_results_that_do_not_fit(quantities, monkeypatch):
+    """Results beyond the limit take no more device memory than the copies one by one do."""
+    import torch
+
+    points, box, _ = configs.diamond(12, seed=2)
+
+    def peak_and_results(limit):
+        monkeypatch.setattr(_host_results, "LIMIT", limit)
+        calculator = NeighborList(cutoff=5.0, full_list=True, sorted=True)
+        for _ in range(3):
+            torch.cuda.reset_peak_memory_stats()
+            results = calculator.compute(points, box, True, quantities)
+        return torch.cuda.max_memory_allocated(), results
+
+    monkeypatch.setattr(NeighborList, "_host_results", lambda self, *arguments: None)
+    one_by_one, expected = peak_and_results(0)
+    monkeypatch.undo()
+    beyond, results = peak_and_results(1000)
+    assert beyond <= one_by_one
+    assert all(np.array_equal(a, b) for a, b in zip(expected, results))
+
+
 def test_several_threads():
     systems = [configs.diamond(replicas, seed=replicas)[:2] for replicas in (2, 3, 4, 5)]
     expected = [NeighborList(cutoff=5.0, full_list=True, sorted=True).compute(p, b, True, "PSd") for p, b in systems]

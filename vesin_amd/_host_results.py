@@ -46,25 +46,33 @@ class HostStaging:
         with self._lock:
             self._kept.append(block)
 
+    @staticmethod
+    def _places(sizes):
+        """Where arrays of these sizes start in a block, and where the last one ends."""
+        starts, end = [], 0
+        for size in sizes:
+            starts.append(end)
+            end += (size + ALIGNMENT - 1) // ALIGNMENT * ALIGNMENT
+        return starts, end
+
+    def fits(self, sizes):
+        return 0 < self._places(sizes)[1] <= LIMIT
+
     def to_host(self, tensors, dtypes):
         """The device tensors (contiguous, of one device) as numpy arrays of the given types of the same size, or None when
         they do not fit."""
         import torch
 
-        starts, needed = [], 0
-        for tensor in tensors:
-            starts.append(needed)
-            size = tensor.numel() * tensor.element_size()
-            needed += (size + ALIGNMENT - 1) // ALIGNMENT * ALIGNMENT
-        block = self._take(needed) if 0 < needed <= LIMIT else None
+        sizes = [tensor.numel() * tensor.element_size() for tensor in tensors]
+        starts, needed = self._places(sizes)
+        block = self._take(needed) if self.fits(sizes) else None
         if block is None:
             return None
         stream = torch.cuda.current_stream(tensors[0].device)
         in_one_go = needed <= SMALL
         try:
             landing, landed = [], []
-            for start, tensor in zip(starts, tensors):
-                size = tensor.numel() * tensor.element_size()
+            for start, size, tensor in zip(starts, sizes, tensors):
                 landing.append(block[start : start + size].view(tensor.dtype).view(tensor.shape))
                 landing[-1].copy_(tensor, non_blocking=True)
                 if not in_one_go:

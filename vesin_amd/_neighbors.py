@@ -450,6 +450,10 @@ class NeighborList:
         if not self.__dict__.get("_host_called", False):
             self._host_called = True
             return None
+        arrays = {"i": pairs, "j": pairs, "P": pairs, "S": shifts, "d": distances, "D": vectors}
+        sizes = [arrays[q].numel() * arrays[q].element_size() // (2 if q in "ij" else 1) for q in quantities if q in arrays]
+        if not HOST_STAGING.fits(sizes):
+            return None  # (before anything is made for it)
         tensors, dtypes = [], []
         columns = None
         for quantity in quantities:
