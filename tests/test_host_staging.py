@@ -1,0 +1,29 @@
+"""Which results of numpy callers come by way of pinned memory (vesin_amd/_host_results.py), without a GPU."""
+
+import pytest
+
+from vesin_amd import _host_results
+from vesin_amd._host_results import HostStaging
+
+MB = 1_000_000
+BYTES = {"i": 8, "j": 8, "P": 16, "S": 12, "d": 8, "D": 24}
+
+
+# (quantities, bytes, time of a call through the pinned block over that of the copies one by one, whichever way through the
+# block is the faster one)
+@pytest.mark.parametrize("quantities, size, ratio", [
+    ("d", 0.04 * MB, 1.07), ("d", 0.42 * MB, 1.08), ("d", 1.05 * MB, 1.04), ("d", 1.68 * MB, 0.89), ("d", 26.8 * MB, 0.53),
+    ("PSdD", 0.31 * MB, 1.05), ("PSdD", 1.42 * MB, 1.06), ("PSdD", 1.88 * MB, 1.07), ("PSdD", 3.14 * MB, 0.90),
+    ("PSdD", 50.3 * MB, 0.43), ("ijSd", 0.05 * MB, 0.77), ("ijSd", 0.85 * MB, 0.93), ("ijSd", 3.24 * MB, 0.88),
+    ("ij", 0.18 * MB, 0.92), ("ij", 2.1 * MB, 0.87), ("ij", 53.6 * MB, 0.43), ("ij", 100 * MB, 1.0), ("PSdD", 100 * MB, 1.0),
+])
+def test_results_come_the_faster_way(quantities, size, ratio):
+    rows = size / sum(BYTES[q] for q in quantities)
+    sizes = [int(rows) * BYTES[q] for q in quantities]
+    assert HostStaging().pays(sizes, columns="i" in quantities) == (ratio < 1.0)
+
+
+def test_no_rows_and_the_limit():
+    staging = HostStaging()
+    assert not staging.pays([0, 0], True)
+    assert staging.pays([_host_results.LIMIT], False) and not staging.pays([_host_results.LIMIT + 1], False)

@@ -13,9 +13,13 @@ import numpy as np
 LIMIT = 64 << 20      # bytes of pinned memory, in use and kept
 SMALLEST = 1 << 20    # bytes of a block at least
 ALIGNMENT = 64        # of the arrays in a block
-# Results of up to this are waited for together: an event for each costs more than the overlap gives (216 atoms, 0.7 MB, per
-# call 256 us with, 160 without; the copies one by one 190. 1,728 atoms, 5.5 MB: 530 -> 400, 8,000 atoms 1710 -> 820 us)
-SMALL = 2 << 20
+# Small results are waited for together, as an event for each array costs more than the overlap gives. That way through the
+# block then only pays where it spares a copy of its own for the columns i and j. Up to 1 MB and three eighths of one per array
+# (calls, copies one by one / together / each with an event, us: i j S d, 0.9 MB 220 / 204 / 234, 2.4 MB 316 / 300 / 291, 4.7 MB
+# 429 / 417 / 345; P S d D, 0.7 MB 180 / 190 / 220, 2.5 MB 257 / 273 / 260, 3.1 MB 305 / 315 / 276; d, 0.2 MB 105 / 115 / 121, 1.1 MB
+# 175 / 190 / 182, 1.7 MB 219 / 229 / 193; beyond, 8 to 50 MB, the last takes about half as long as the first)
+SMALL = 1 << 20
+SMALL_PER_ARRAY = 3 << 17
 
 
 class HostStaging:
@@ -55,8 +59,16 @@ class HostStaging:
             end += (size + ALIGNMENT - 1) // ALIGNMENT * ALIGNMENT
         return starts, end
 
+    @staticmethod
+    def _small(size, number):
+        return size <= SMALL + number * SMALL_PER_ARRAY
+
     def fits(self, sizes):
         return 0 < self._places(sizes)[1] <= LIMIT
+
+    def pays(self, sizes, columns):
+        """Whether arrays of these sizes, some of them columns of the pairs or not, come faster this way than one by one."""
+        return self.fits(sizes) and (columns or not self._small(self._places(sizes)[1], len(sizes)))
 
     def to_host(self, tensors, dtypes):
         """The device tensors (contiguous, of one device) as numpy arrays of the given types of the same size, or None when
@@ -69,7 +81,7 @@ class HostStaging:
         if block is None:
             return None
         stream = torch.cuda.current_stream(tensors[0].device)
-        in_one_go = needed <= SMALL
+        in_one_go = self._small(needed, len(sizes))
         try:
             landing, landed = [], []
             for start, size, tensor in zip(starts, sizes, tensors):

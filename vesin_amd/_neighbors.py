@@ -452,7 +452,7 @@ class NeighborList:
             return None
         arrays = {"i": pairs, "j": pairs, "P": pairs, "S": shifts, "d": distances, "D": vectors}
         sizes = [arrays[q].numel() * arrays[q].element_size() // (2 if q in "ij" else 1) for q in quantities if q in arrays]
-        if not HOST_STAGING.fits(sizes):
+        if not HOST_STAGING.pays(sizes, "i" in quantities or "j" in quantities):
             return None  # (before anything is made for it)
         tensors, dtypes = [], []
         columns = None
