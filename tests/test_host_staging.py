@@ -1,6 +1,8 @@
 """Which results of numpy callers come by way of pinned memory (vesin_amd/_host_results.py), without a GPU."""
 
+import numpy as np
 import pytest
+import torch
 
 from vesin_amd import _host_results
 from vesin_amd._host_results import HostStaging
@@ -27,3 +29,48 @@ def test_no_rows_and_the_limit():
     staging = HostStaging()
     assert not staging.pays([0, 0], True)
     assert staging.pays([_host_results.LIMIT], False) and not staging.pays([_host_results.LIMIT + 1], False)
+
+
+class _Event:
+    def synchronize(self):
+        pass
+
+
+class _Stream(_Event):
+    def record_event(self):
+        return _Event()
+
+
+@pytest.fixture
+def no_gpu(monkeypatch):
+    """Blocks of ordinary memory, copies that are done when they return."""
+    empty = torch.empty
+
+    def unpinned(*shape, pin_memory=False, device=None, **options):
+        if pin_memory and torch.device(device or torch.get_default_device()).type != "cpu":
+            raise RuntimeError("Only dense CPU tensors can be pinned")
+        return empty(*shape, device=device, **options)
+
+    monkeypatch.setattr(torch, "empty", unpinned)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: _Stream())
+
+
+def test_pinned_memory_that_is_refused(monkeypatch):
+    """The results are copied one by one then, and the pool is as it was."""
+    def refuse(*shape, **options):
+        raise RuntimeError("out of memory")
+
+    staging = HostStaging()
+    monkeypatch.setattr(torch, "empty", refuse)
+    assert staging.to_host([torch.arange(10)], [np.int64]) is None
+    assert staging._held == 0 and staging._kept == []
+
+
+@pytest.mark.parametrize("rows", [1000, 1_000_000])
+def test_blocks_made_under_another_default_device(rows, no_gpu):
+    values = torch.arange(rows, dtype=torch.float64)
+    staging = HostStaging()
+    with torch.device("meta"):
+        assert np.array_equal(staging.to_host([values], [np.float64])[0], values.numpy())
+    assert np.array_equal(staging.to_host([values], [np.float64])[0], values.numpy())
+    assert staging._held > 0

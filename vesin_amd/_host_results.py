@@ -28,9 +28,18 @@ class HostStaging:
         self._kept = []
         self._held = 0
 
-    def _take(self, needed):
+    @staticmethod
+    def _pinned(size):
+        """A new block, or None when there is no pinned memory for it (a limit of the machine)."""
         import torch
 
+        try:
+            # (on the CPU, whatever torch's default device is)
+            return torch.empty(size, dtype=torch.uint8, device="cpu", pin_memory=True)
+        except RuntimeError:
+            return None
+
+    def _take(self, needed):
         with self._lock:
             fitting = [block for block in self._kept if block.numel() >= needed]
             if fitting:
@@ -42,8 +51,8 @@ class HostStaging:
                 self._held -= self._kept.pop(0).numel()
             if self._held + size > LIMIT:
                 return None
-            block = torch.empty(size, dtype=torch.uint8, pin_memory=True)
-            self._held += size
+            block = self._pinned(size)
+            self._held += size if block is not None else 0
             return block
 
     def _give_back(self, block):
