@@ -74,3 +74,21 @@ def test_blocks_made_under_another_default_device(rows, no_gpu):
         assert np.array_equal(staging.to_host([values], [np.float64])[0], values.numpy())
     assert np.array_equal(staging.to_host([values], [np.float64])[0], values.numpy())
     assert staging._held > 0
+
+
+def test_the_pool_never_locks_more_than_it_says(no_gpu, monkeypatch):
+    """Counted at the allocator, which keeps pinned memory locked when a block is dropped."""
+    locked = []
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda size, **options: locked.append(size) or empty(size, **options))
+    staging = HostStaging()
+    mb = 1 << 20
+    # results of every size, growing and shrinking; several threads at once
+    for sizes in [[k * mb] for k in (1, 2, 3, 9, 20, 40, 64, 30, 5)] + [[40 * mb, 40 * mb], [3 * mb] * 9, [64 * mb], [25 * mb] * 3]:
+        blocks = [staging._take(size) for size in sizes]
+        assert all(block is None or block.numel() >= size for block, size in zip(blocks, sizes))
+        assert blocks[0] is not None  # (one thread always finds a block)
+        for block in blocks:
+            if block is not None:
+                staging._give_back(block)
+    assert sum(locked) == staging._held <= _host_results.POOL == 2 * _host_results.LIMIT

@@ -2,15 +2,17 @@
 between, and from there to memory of their own, each while the next ones are still on the way. (They are not handed out where
 they landed: pinned memory is not there for forked processes, and stays locked for as long as an array made of it lives.)
 
-The pinned memory is kept in a pool of at most ``LIMIT`` bytes for the whole process. Results that do not fit are copied one
-by one, and so are those of a calculator's first call (it does not pay for the pinned memory).
+The pinned memory is kept in a pool of at most ``POOL`` bytes for the whole process, until it ends: blocks are never dropped, as
+PyTorch's allocator would keep them locked. Results of more than ``LIMIT`` bytes, or that find no block, are copied one by one,
+and so are those of a calculator's first call (it does not pay for the pinned memory).
 """
 
 import threading
 
 import numpy as np
 
-LIMIT = 64 << 20      # bytes of pinned memory, in use and kept
+LIMIT = 64 << 20      # bytes of results at most
+POOL = 2 * LIMIT      # bytes of pinned memory, in use and kept: one block of every size, as blocks are powers of two
 SMALLEST = 1 << 20    # bytes of a block at least
 ALIGNMENT = 64        # of the arrays in a block
 # Small results are waited for together, as an event for each array costs more than the overlap gives. That way through the
@@ -26,7 +28,7 @@ class HostStaging:
     def __init__(self):
         self._lock = threading.Lock()
         self._kept = []
-        self._held = 0
+        self._held = 0 # bytes of all blocks, none of which is ever dropped
 
     @staticmethod
     def _pinned(size):
@@ -47,9 +49,7 @@ class HostStaging:
                 self._kept = [other for other in self._kept if other is not block]
                 return block
             size = max(SMALLEST, 1 << (needed - 1).bit_length())
-            while self._kept and self._held + size > LIMIT:
-                self._held -= self._kept.pop(0).numel()
-            if self._held + size > LIMIT:
+            if self._held + size > POOL:
                 return None
             block = self._pinned(size)
             self._held += size if block is not None else 0
