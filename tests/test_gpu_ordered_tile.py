@@ -15,7 +15,7 @@ NAMES = {"P": "pairs", "S": "shifts", "d": "distances", "D": "vectors"}
 EVERY = (True, True, True)
 
 
-def _check(points, box, periodic, cutoff, full, quantities, capfd, monkeypatch, by_tiles=True):
+def _check(points, box, periodic, cutoff, full, quantities, capfd, monkeypatch):
     import torch
 
     expected = oracle.canonicalize(oracle.neighbors(points, box, list(periodic), cutoff, full, False, "ijSdD"))
@@ -27,10 +27,9 @@ def _check(points, box, periodic, cutoff, full, quantities, capfd, monkeypatch, 
         capfd.readouterr()
         outputs = calculator.compute(device_points, device_box, periodic, quantities)
         err = capfd.readouterr().err
-        found = re.findall(r"tiles written by (\d+) waves each.* and counted by (\d+): used", err)
+        found = re.findall(r"tiles written by \d+ waves each(.*) and counted by \d+: used", err)
         assert len(found) == 1, err
-        if call > 0:
-            assert (found[0] == ("4", "4")) == by_tiles, err
+        assert ("a workgroup per tile" in found[0]) == (call > 0), err
         for q, out in zip(quantities, outputs):
             assert np.array_equal(out.cpu().numpy(), expected[NAMES[q]]), (call, q)
     return expected

@@ -258,10 +258,9 @@ def test_any_number_of_waves_per_tile_writes_the_same_rows(waves, full, capfd, m
     _check(points, box, (True, False, True), 3.0, full, capfd, monkeypatch, "used")
 
 
-def test_well_filled_tiles_that_barely_exceed_the_resident_waves_get_four_waves_each(capfd, monkeypatch):
-    """110,592 atoms in 4,096 cells, 729 candidates around a tile on average (more than the kernel that brings them to
-    LDS is for): the list's first call learns the number of tiles, the calls after it deal every tile's points to four
-    waves; both give the oracle's list."""
+def test_well_filled_tiles_get_a_workgroup_each_from_the_second_call_on(capfd, monkeypatch):
+    """110,592 atoms in 4,096 cells, 729 candidates around a tile on average: the list's first call learns the number of
+    tiles, the calls after it give every tile a workgroup; both give the oracle's list."""
     import torch
 
     points, box = _lattice(24, 24, 24, seed=12)
@@ -276,13 +275,13 @@ def test_well_filled_tiles_that_barely_exceed_the_resident_waves_get_four_waves_
         P, S, d, D = calculator.compute(device_points, device_box, True, "PSdD")
         err = capfd.readouterr().err
         tiles, each = _waves_per_tile(err)
-        assert 4096 < tiles < 6144 and "candidates in LDS" not in err
-        waves.append(each)
+        assert 4096 < tiles < 6144
+        waves.append((each, "a workgroup per tile" in err))
         assert np.array_equal(P.cpu().numpy(), expected["pairs"])
         assert np.array_equal(S.cpu().numpy(), expected["shifts"])
         assert np.array_equal(d.cpu().numpy(), expected["distances"])
         assert np.array_equal(D.cpu().numpy(), expected["vectors"])
-    assert waves == [1, 4, 4]
+    assert waves == [(1, False), (4, True), (4, True)]
 
 
 @pytest.mark.parametrize("waves", [2, 3, 4])

@@ -2659,19 +2659,17 @@ bool compute(
         const bool suitable = found.found.max_rows <= ORDERED_MAX_ROWS &&
                               found.found.max_candidates <= ORDERED_CANDIDATES && found.found.unsuitable == 0;
         if (std::getenv("VESIN_HIP_DEBUG") != nullptr) {
-            // (well-filled tiles whose candidates come to the writing pass's LDS in one go, also where all of them have a
-            // hit: 10 points per tile, 16 when there are vectors, and 665 candidates on average)
-            const bool one_chunk =
-                tiles_before > 0 &&
-                static_cast<double>(n_points) >= (options.return_vectors ? 16.0 : 10.0) * static_cast<double>(tiles_before) &&
-                static_cast<double>(full_stencil) * static_cast<double>(n_points) <= 665.0 * static_cast<double>(n_cells);
+            char workgroups[64] = "";
+            if (by_tiles) {
+                std::snprintf(workgroups, sizeof(workgroups), " (a workgroup per tile, %u hits at most)", found.found.max_hits);
+            }
             std::fprintf(
                 stderr,
                 "in-order search: rows %llu, most rows of a point %u, most candidates of a tile %u, unsuitable %u, "
                 "candidates of %u tiles ordered by window and of %u by buckets, %u tiles written by %u waves each%s and counted by %u: %s\n",
                 found.total_rows, found.found.max_rows, found.found.max_candidates, found.found.unsuitable,
                 found.found.windowed, found.found.bucketed, found.n_tiles, oargs.write_split,
-                by_tiles && one_chunk ? " (candidates in LDS)" : "", oargs.count_split, suitable ? "used" : "not covered"
+                workgroups, oargs.count_split, suitable ? "used" : "not covered"
             );
         }
         if (suitable) {

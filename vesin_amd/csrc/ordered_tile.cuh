@@ -420,6 +420,7 @@ __global__ __launch_bounds__(TILE_BLOCK, 6) void ordered_tile_kernel(OrderedArgs
     }
     if (args.report_order != 0 && threadIdx.x == 0) {
         atomicAdd(window ? &args.status->windowed : &args.status->bucketed, 1u);
+        atomicMax(&args.status->max_hits, n);
     }
     if (window) {
         uint32_t offset[TILE_SORT_OWN];
