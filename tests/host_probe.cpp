@@ -112,16 +112,8 @@ extern "C" unsigned int probe_ordered_share(size_t n_points, size_t n_cells, siz
     return vesin_hip::ordered_share(n_points, n_cells, tile_slots, coarse != 0);
 }
 
-extern "C" unsigned int probe_ordered_write_split(size_t n_points, size_t tiles_before) {
-    return vesin_hip::ordered_write_split(n_points, tiles_before);
-}
-
 extern "C" int probe_ordered_by_tiles(size_t n_points, size_t tiles_before, int vectors) {
     return vesin_hip::ordered_by_tiles(n_points, tiles_before, vectors != 0) ? 1 : 0;
-}
-
-extern "C" unsigned int probe_ordered_count_split(size_t n_points, size_t tiles_before) {
-    return vesin_hip::ordered_count_split(n_points, tiles_before);
 }
 
 /// Runs the bookkeeping of a launch with waiting workgroups (vesin_hip::WaitRest) over a sequence of calls:

@@ -45,9 +45,6 @@ def probe(tmp_path_factory):
     lib.probe_candidate_lifetime.restype = None
     lib.probe_ordered_share.argtypes = [ctypes.c_size_t, ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int]
     lib.probe_ordered_share.restype = ctypes.c_uint
-    for name in ("probe_ordered_write_split", "probe_ordered_count_split"):
-        getattr(lib, name).argtypes = [ctypes.c_size_t, ctypes.c_size_t]
-        getattr(lib, name).restype = ctypes.c_uint
     lib.probe_ordered_by_tiles.argtypes = [ctypes.c_size_t, ctypes.c_size_t, ctypes.c_int]
     lib.probe_ordered_by_tiles.restype = ctypes.c_int
     lib.probe_crowded_stores.argtypes = [ctypes.c_size_t, ctypes.c_size_t] + [ctypes.c_int] * 3
@@ -369,30 +366,6 @@ def test_share_of_a_tile_per_wave(probe):
             assert found in (1, 2, 4, 8, 16, 32)
             if not coarse:
                 assert found <= share(n_points, n_cells, True) or found in (4, 8)
-
-
-def test_waves_per_tile_of_the_two_passes(probe):
-    write = probe.probe_ordered_write_split
-    count = probe.probe_ordered_count_split
-    # nothing known about the system yet
-    assert write(100_000, 0) == 1 and count(100_000, 0) == 1
-    # the 100,000-atom benchmark: 4,260 tiles of 23.5 points
-    assert write(100_000, 4260) == 4 and count(100_000, 4260) == 2
-    # twice and four times the size at the same filling
-    assert write(200_000, 9000) == 4 and count(200_000, 9000) == 2
-    assert write(400_000, 19_000) == 4 and count(400_000, 19_000) == 1
-    assert write(800_000, 39_000) == 1 and count(800_000, 39_000) == 1
-    # few tiles: the writing pass has room for all of them at once
-    assert write(50_000, 2300) == 1 and count(50_000, 2300) == 2
-    # 12 points per tile: one wave each, whatever the number of tiles
-    assert write(100_000, 8100) == 1 and count(100_000, 8100) == 1
-    assert write(50_000, 4200) == 1 and count(50_000, 4200) == 1
-    for tiles in range(1, 40_000, 97):
-        for per_tile in (3, 15, 16, 31):
-            assert write(tiles * per_tile, tiles) in (1, 4)
-            assert count(tiles * per_tile, tiles) in (1, 2)
-            if per_tile < 16:
-                assert write(tiles * per_tile, tiles) == 1 and count(tiles * per_tile, tiles) == 1
 
 
 # (points, tiles, vectors returned, time of a call with a workgroup per tile over that with a wave per tile or share of one):

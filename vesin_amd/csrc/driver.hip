@@ -2533,20 +2533,18 @@ bool compute(
         oargs.rows_of_point = rows_of_point;
         oargs.records = candidate_records;
         oargs.candidates_of_item = candidates_of_item;
-        // How many waves share a tile in either pass follows the number of tiles the call before had on the same
-        // number of points (policy.hpp); a list's first call on a system keeps one wave per tile.
         const bool presorted = ordered_items_per_tile == 1;
-        const size_t tiles_before = presorted ? tiles_known : 0;
-        oargs.write_split = by_tiles ? TILE_WAVES : ordered_write_split(n_points, tiles_before);
-        if (const char* text = std::getenv("VESIN_HIP_WRITE_SPLIT")) {
-            oargs.write_split = static_cast<uint32_t>(std::max(1, std::min(4, std::atoi(text))));
-        }
+        // Waves that share a tile: a workgroup's (by_tiles), or one; VESIN_HIP_WRITE_SPLIT and VESIN_HIP_COUNT_SPLIT (for
+        // measurements and tests) deal the points of a tile to several in the writing pass, its candidates in the counting pass.
+        auto waves_per_tile = [&](const char* name) {
+            const char* text = std::getenv(name);
+            return by_tiles ? static_cast<uint32_t>(TILE_WAVES)
+                            : static_cast<uint32_t>(text != nullptr ? std::max(1, std::min(4, std::atoi(text))) : 1);
+        };
+        oargs.write_split = waves_per_tile("VESIN_HIP_WRITE_SPLIT");
         // (the waves of a tile add their rows in memory that the cell build cleared)
         const bool rows_cleared = !single_cell && !small_build;
-        oargs.count_split = by_tiles ? TILE_WAVES : rows_cleared ? ordered_count_split(n_points, tiles_before) : 1;
-        if (const char* text = std::getenv("VESIN_HIP_COUNT_SPLIT")) {
-            oargs.count_split = rows_cleared ? static_cast<uint32_t>(std::max(1, std::min(4, std::atoi(text)))) : 1u;
-        }
+        oargs.count_split = by_tiles || rows_cleared ? waves_per_tile("VESIN_HIP_COUNT_SPLIT") : 1;
         oargs.points = reinterpret_cast<const double*>(points);
         oargs.pre = pre;
         oargs.order = candidate_order;

@@ -232,46 +232,6 @@ inline bool crowded_search_pays(size_t n_points, size_t n_tiles) {
     return n_tiles <= 16384 || n_points >= 5 * n_tiles;
 }
 
-/// Waves that share the points of a tile in the writing pass of a wave per tile or share (1 or 4), from the number of tiles the
-/// call before had on the same points (0: not known, one wave). Such tiles have a workgroup each since (ordered_by_tiles),
-/// unless one of the two numbers of waves is forced.
-///
-/// The pass keeps four waves per SIMD resident, 4096 on this GPU. A system of a few more tiles than that leaves the
-/// stragglers running alone for as long as everything before them took (100,000 atoms, 4,260 tiles: 172 us where a
-/// wave lives 110 us; four waves per tile 121 us). With four waves per tile a workgroup is a tile: its waves fetch
-/// the tile's records together and each writes the rows of a quarter of the points, so the work comes in shorter
-/// pieces at little extra cost. It pays for well-filled tiles up to about five times as many tiles as resident
-/// waves (half lists at 24 points per tile, cutoff 6, per call with one wave -> four: 4,500 tiles 318 -> 283 us,
-/// 9,000 tiles 551 -> 515 us, 19,000 tiles 833 -> 794 us, 39,000 tiles 1613 -> 1613 us; full lists at 23 points per
-/// tile, 52,000 tiles: 2.04 -> 2.07 ms) and not for tiles of few points (12 per tile, full lists: 8,000 tiles 276 ->
-/// 311 us, 27,000 tiles 483 -> 606 us).
-inline unsigned int ordered_write_split(size_t n_points, size_t tiles_before) {
-    if (tiles_before == 0) {
-        return 1;
-    }
-    const double resident = 4096.0;
-    const double tiles = static_cast<double>(tiles_before);
-    if (static_cast<double>(n_points) < 16.0 * tiles) {
-        return 1;
-    }
-    return tiles > 0.85 * resident && tiles <= 5.0 * resident ? 4 : 1;
-}
-
-/// Waves that share the candidates of a tile in the counting pass (1 or 2), decided like the other.
-///
-/// That pass runs seven waves per SIMD (7168 at a time) and lasts as long as its slowest wave, the one of the tile
-/// with the most points and candidates. While the tiles of a system do not fill those slots much more than once, the
-/// candidates of every well-filled tile are dealt to two waves, pairs of units of 64 in turn, that add up their rows
-/// per point (half lists, cutoff 6, per call: 24 points per tile, 25,000 / 50,000 / 100,000 / 200,000 atoms 168 ->
-/// 155, 217 -> 201, 312 -> 304, 529 -> 519 us; 400,000 atoms, 17,576 tiles: 833 -> 841 us; 12 points per tile,
-/// 30,000 / 100,000 atoms: 137 -> 143, 275 -> 282 us).
-inline unsigned int ordered_count_split(size_t n_points, size_t tiles_before) {
-    if (tiles_before == 0 || tiles_before > 9216) {
-        return 1;
-    }
-    return static_cast<double>(n_points) >= 16.0 * static_cast<double>(tiles_before) ? 2 : 1;
-}
-
 /// Whether the search gives every tile a workgroup (ordered_tile.cuh) in place of a wave or several (ordered.cuh), from the
 /// number of tiles the call before had on the same points (0: not known, and a wave per tile).
 ///
