@@ -222,3 +222,74 @@ def test_the_rest_after_a_refused_system_ends(capfd, monkeypatch):
     assert tried == [False] * 64 + [True] * 2
     for q, out in zip("PSdD", outputs):
         assert np.array_equal(out.cpu().numpy(), expected[NAMES[q]]), q
+
+
+@pytest.mark.parametrize("full", [True, False])
+@pytest.mark.parametrize("periodic,far", [(False, 0.0), (False, 1.0e6), (True, 0.0), (True, 4.0e3)])
+def test_pairs_next_to_the_cutoff(periodic, far, full, capfd, monkeypatch):
+    """Pairs within a few units in the last place of the cutoff, on either side, which single precision cannot decide; far from
+    the origin, and with points moved by box vectors, so that shifts and wraps take part in the decision."""
+    rng = np.random.default_rng(9)
+    cutoff, box = 3.0, np.array([[38.0, 0.0, 0.0], [4.0, 39.0, 0.0], [-3.0, 2.0, 40.0]])
+    grid = np.stack(np.meshgrid(*[np.arange(12)] * 3, indexing="ij"), axis=-1).reshape(-1, 3)
+    first = (grid + 0.5 + rng.uniform(-0.05, 0.05, size=grid.shape)) / 12 @ box
+    direction = rng.normal(size=first.shape)
+    direction /= np.linalg.norm(direction, axis=1)[:, None]
+    steps = rng.integers(-6, 7, size=len(first)).astype(np.float64)
+    second = first + direction * (cutoff * (1.0 + steps * 2.0**-52))[:, None]
+    points = np.concatenate([first, second])
+    if periodic:
+        points[::3] += rng.integers(-3, 4, size=points[::3].shape) @ box
+    points = (points + far)[rng.permutation(len(points))]
+    _check(points, box, periodic, cutoff, full, capfd, monkeypatch)
+    expected = _expected(points, box, periodic, cutoff, full)
+    assert (np.abs(expected["distances"] - cutoff) < 1e-8).sum() > 300
+    assert not periodic or (expected["shifts"] != 0).any(axis=1).sum() > 300
+
+
+@pytest.mark.parametrize("scale", [1e-6, 1e9, 1e12])
+@pytest.mark.parametrize("full", [True, False])
+def test_small_and_large_cutoffs(full, scale, capfd, monkeypatch):
+    """The largest is left to double precision altogether (a square of 9e24); of points moved by box vectors too, and of tiles
+    of which none was moved."""
+    for outside in (0.0, 0.6):
+        points, box = _liquid(4000, 20.0, 10, outside, 0.2)
+        _check(points * scale, box * scale, True, 3.0 * scale, full, capfd, monkeypatch)
+
+
+@pytest.mark.parametrize("periodic", [False, True])
+@pytest.mark.parametrize("full", [True, False])
+def test_tiles_too_wide_for_single_precision(full, periodic, capfd, monkeypatch):
+    """Pairs of points in a box of 4,000 cutoffs, whose cells are 222 cutoffs wide (no more cells than points): the points of
+    tiles with two pairs and more are too far apart for the tests in single precision, those of one pair are not."""
+    rng = np.random.default_rng(14)
+    first = 4000.0 * rng.random((1500, 3))
+    points = np.concatenate([first, first + 0.6 * rng.normal(size=first.shape)])[rng.permutation(3000)]
+    expected = _expected(points, 4000.0 * np.eye(3), periodic, 1.0, full)
+    assert len(expected["pairs"]) > 500
+    _check(points, 4000.0 * np.eye(3), periodic, 1.0, full, capfd, monkeypatch)
+
+
+@pytest.mark.parametrize(
+    "n,quantities,full,streamed",
+    [
+        (150_000, "P", True, True), (150_000, "PSd", True, True), (150_000, "PSdD", False, True),
+        (100_000, "PSdD", False, False), # (by granule: see crowded_stores)
+    ],
+)
+def test_lists_beyond_the_caches(n, quantities, full, streamed, capfd, monkeypatch):
+    """More than 200 MB of rows: stored past the caches, with vectors only of systems whose shared pieces would not stay there."""
+    points, box = _liquid(n, 3.03 * (n / 25.0) ** (1.0 / 3.0), 13, 0.0, 0.1)
+    expected = _expected(points, box, True, 3.0, full)
+    row_bytes = 16 + 12 * ("S" in quantities) + 8 * ("d" in quantities) + 24 * ("D" in quantities)
+    assert len(expected["pairs"]) * row_bytes > 200 << 20 and len(expected["pairs"]) >= 40 * n
+    assert streamed == ("D" not in quantities or n * 16 * row_bytes > 128 << 20)
+    monkeypatch.setenv("VESIN_HIP_SORT", "crowded")
+    monkeypatch.setenv("VESIN_HIP_DEBUG", "1")
+    calculator = NeighborList(cutoff=3.0, full_list=full, sorted=True)
+    for call in range(2):
+        capfd.readouterr()
+        result = _compute(calculator, points, box, True, quantities)
+        assert "crowded search:" in capfd.readouterr().err
+        for key in result:
+            assert np.array_equal(result[key], expected[key]), (call, key)

@@ -32,7 +32,7 @@ def _check(points, box, periodic, cutoff, full, quantities, capfd, monkeypatch):
         assert ("a workgroup per tile" in found[0]) == (call > 0), err
         for q, out in zip(quantities, outputs):
             assert np.array_equal(out.cpu().numpy(), expected[NAMES[q]]), (call, q)
-    return expected
+    return expected, err
 
 
 def _liquid(n, per_cell, cutoff, skew, seed):
@@ -94,7 +94,7 @@ def test_pairs_next_to_the_cutoff(far, full, capfd, monkeypatch):
     steps = rng.integers(-6, 7, size=len(first)).astype(np.float64)
     second = first + direction * (cutoff * (1.0 + steps * 2.0**-52))[:, None]
     points = np.concatenate([first, second]) + far
-    expected = _check(points, box, (False, False, False), cutoff, full, "PSd", capfd, monkeypatch)
+    expected, _ = _check(points, box, (False, False, False), cutoff, full, "PSd", capfd, monkeypatch)
     assert (np.abs(expected["distances"] - cutoff) < 1e-9).sum() > 300
 
 
@@ -106,35 +106,67 @@ def test_small_and_large_cutoffs(scale, capfd, monkeypatch):
 
 
 def test_more_rows_than_a_line_holds(capfd, monkeypatch):
-    """About 230 rows for each of up to 32 points of a tile, in order of the cells (runs of many rows) and in none."""
+    """A blob of 37 points in every cell, about 150 rows for each of the 32 points of its first tile, where a line holds 2,560
+    rows: two lines, of points in order of the cells (runs of many rows) and in none."""
     rng = np.random.default_rng(11)
     edge = 4 * 3.003
     centres = np.stack(np.meshgrid(*[np.arange(4)] * 3, indexing="ij"), axis=-1).reshape(-1, 3) * 3.003 + 1.5
-    ball = rng.normal(size=(64, 15, 3)) * 0.35
+    ball = np.clip(rng.normal(size=(64, 37, 3)) * 0.35, -1.4, 1.4)
     points = (centres[:, None, :] + ball).reshape(-1, 3)
     box = np.eye(3) * edge
     for order in (np.arange(len(points)), rng.permutation(len(points))):
-        _check(points[order], box, EVERY, 3.0, True, "PSdD", capfd, monkeypatch)
+        expected, _ = _check(points[order], box, EVERY, 3.0, True, "PSdD", capfd, monkeypatch)
+        rows = np.empty(len(points), dtype=int)
+        rows[order] = np.bincount(expected["pairs"][:, 0].astype(int), minlength=len(points))
+        assert np.sort(rows.reshape(64, 37), axis=1)[:, :32].sum(axis=1).min() > 2560 and rows.max() <= 256
+
+
+def _spans_of_cells(pairs, points, shape, n):
+    """Of the neighbours of the points of every cell of the search: the range of their indices, as it is and counted from the
+    last index on to the first where that is shorter."""
+    cells = np.floor(points / (np.array(shape) * 3.567) * np.floor(np.array(shape) * 3.567 / 5.0)).astype(int)
+    _, cell = np.unique(cells, axis=0, return_inverse=True)
+    cell = cell.reshape(-1)
+    first = np.full(cell.max() + 1, n)
+    np.minimum.at(first, cell, np.arange(n))
+    i, j = pairs.astype(np.int64).T
+    ranges = []
+    for index in (j, (j - first[cell[i]] + n // 2) % n):
+        low, high = np.full(len(first), n), np.full(len(first), -1)
+        np.minimum.at(low, cell[i], index)
+        np.maximum.at(high, cell[i], index)
+        ranges.append(high - low + 1)
+    return ranges[0], np.minimum(*ranges)
 
 
 @pytest.mark.parametrize("order", ["lattice", "none", "around the end"])
 def test_orders_of_the_indices(order, capfd, monkeypatch):
-    """Ranked through the bit set (one round, several, from the last index on to the first) or through buckets."""
+    """Ranked through the bit set (65,536 indices at a time: one round, two, from the last index on to the first) or through
+    buckets."""
     basis = np.array([[0, 0, 0], [0, 2, 2], [2, 0, 2], [2, 2, 0], [1, 1, 1], [1, 3, 3], [3, 1, 3], [3, 3, 1]]) / 4.0
-    shape = (9, 44, 44) if order == "around the end" else (27, 27, 27)
+    shape = (8, 46, 46) if order == "around the end" else (27, 27, 27)
     cells = np.stack(np.meshgrid(*[np.arange(k) for k in shape], indexing="ij"), axis=-1).reshape(-1, 3)
     points = (cells[:, None, :] + basis[None, :, :]).reshape(-1, 3) * 3.567
     rng = np.random.default_rng(12)
     points += rng.normal(scale=0.05, size=points.shape)
     if order == "none":
         points = points[rng.permutation(len(points))]
-    _check(points, np.diag(np.array(shape) * 3.567), EVERY, 5.0, True, "PSd", capfd, monkeypatch)
+    expected, err = _check(points, np.diag(np.array(shape) * 3.567), EVERY, 5.0, True, "PSd", capfd, monkeypatch)
+    windowed, bucketed = (int(k) for k in re.search(r"candidates of (\d+) tiles ordered by window and of (\d+) by buckets", err).groups())
+    as_it_is, around = _spans_of_cells(expected["pairs"], points, shape, len(points))
+    if order == "none":
+        assert windowed == 0 and bucketed > 4096 and around.min() > 2 * 65_536
+    else:
+        # (most of the cells, as the points on their edges may be in the next one)
+        assert windowed > 4096 and bucketed == 0
+        assert np.mean(around < 65_536) > 0.99 if order == "lattice" else np.mean((around > 65_536) & (around < 2 * 65_536)) > 0.5
+        assert np.sum(as_it_is > 2 * 65_536) > 100
 
 
 @pytest.mark.parametrize("quantities,full", [("P", True), ("PSd", True), ("PSdD", False)])
 def test_lists_beyond_the_caches(quantities, full, capfd, monkeypatch):
     """More than 200 MB of rows: stored past the caches, all of them (pairs alone) or but for the ends of the runs."""
     points, box = _liquid(150_000, 25.0, 3.0, 0.1, 13)
-    expected = _check(points, box, EVERY, 3.0, full, quantities, capfd, monkeypatch)
+    expected, _ = _check(points, box, EVERY, 3.0, full, quantities, capfd, monkeypatch)
     row_bytes = 16 + 12 * ("S" in quantities) + 8 * ("d" in quantities) + 24 * ("D" in quantities)
     assert len(expected["pairs"]) * row_bytes > 200 << 20
