@@ -2,6 +2,8 @@
 list of the oracle, in the order (i, j, S), bit for bit; and the systems that the usual in-order search does not cover
 come to it by themselves."""
 
+import re
+
 import numpy as np
 import pytest
 
@@ -42,6 +44,7 @@ def _check(points, box, periodic, cutoff, full, capfd, monkeypatch, covered=True
         assert result["pairs"].shape == expected["pairs"].shape
         for key in result:
             assert np.array_equal(result[key], expected[key]), (call, key)
+    return int(re.search(r"(\d+) tiles in double precision", lines[-1]).group(1)) if lines else None
 
 
 def _liquid(n, edge, seed, outside=0.0, skew=0.0):
@@ -254,7 +257,19 @@ def test_small_and_large_cutoffs(full, scale, capfd, monkeypatch):
     of which none was moved."""
     for outside in (0.0, 0.6):
         points, box = _liquid(4000, 20.0, 10, outside, 0.2)
-        _check(points * scale, box * scale, True, 3.0 * scale, full, capfd, monkeypatch)
+        in_double = _check(points * scale, box * scale, True, 3.0 * scale, full, capfd, monkeypatch)
+        assert (in_double > 0) == (scale == 1e12)
+
+
+@pytest.mark.parametrize("full", [True, False])
+def test_every_pair_in_double_precision(full, capfd, monkeypatch):
+    """VESIN_HIP_TESTS=double."""
+    points, box = _liquid(4000, 20.0, 10, 0.0, 0.2)
+    moved = np.random.default_rng(16).integers(-2, 3, size=points.shape)
+    moved[points[:, 0] < np.median(points[:, 0])] = 0
+    assert _check(points + moved @ box, box, True, 3.0, full, capfd, monkeypatch) == 0
+    monkeypatch.setenv("VESIN_HIP_TESTS", "double")
+    assert _check(points + moved @ box, box, True, 3.0, full, capfd, monkeypatch) > 0
 
 
 @pytest.mark.parametrize("periodic", [False, True])
@@ -267,7 +282,7 @@ def test_tiles_too_wide_for_single_precision(full, periodic, capfd, monkeypatch)
     points = np.concatenate([first, first + 0.6 * rng.normal(size=first.shape)])[rng.permutation(3000)]
     expected = _expected(points, 4000.0 * np.eye(3), periodic, 1.0, full)
     assert len(expected["pairs"]) > 500
-    _check(points, 4000.0 * np.eye(3), periodic, 1.0, full, capfd, monkeypatch)
+    assert 0 < _check(points, 4000.0 * np.eye(3), periodic, 1.0, full, capfd, monkeypatch)
 
 
 @pytest.mark.parametrize(

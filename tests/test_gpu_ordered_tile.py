@@ -35,6 +35,14 @@ def _check(points, box, periodic, cutoff, full, quantities, capfd, monkeypatch):
     return expected, err
 
 
+def _tiles(err):
+    return int(re.search(r"(\d+) tiles written by", err).group(1))
+
+
+def _in_double(err):
+    return int(re.search(r"of (\d+) by a workgroup in double precision", err).group(1))
+
+
 def _liquid(n, per_cell, cutoff, skew, seed):
     rng = np.random.default_rng(seed)
     box = np.array([[1.0, 0.0, 0.0], [0.6 * skew, 1.05, 0.0], [skew, 0.4 * skew, 1.1]])
@@ -102,7 +110,21 @@ def test_pairs_next_to_the_cutoff(far, full, capfd, monkeypatch):
 def test_small_and_large_cutoffs(scale, capfd, monkeypatch):
     """The largest is left to double precision altogether (a square of 9e24)."""
     points, box = _liquid(4_000, 12.0, 3.0, 0.2, 10)
-    _check(points * scale, box * scale, EVERY, 3.0 * scale, True, "PSdD", capfd, monkeypatch)
+    _, err = _check(points * scale, box * scale, EVERY, 3.0 * scale, True, "PSdD", capfd, monkeypatch)
+    assert _in_double(err) == (_tiles(err) if scale == 1e12 else 0)
+
+
+@pytest.mark.parametrize("full", [True, False])
+def test_every_pair_in_double_precision(full, capfd, monkeypatch):
+    """VESIN_HIP_TESTS=double, on points of which some were moved by box vectors, and others are in tiles of none that was."""
+    points, box = _liquid(8_000, 12.0, 3.0, 0.3, 15)
+    moved = np.random.default_rng(16).integers(-2, 3, size=points.shape)
+    moved[points[:, 0] < np.median(points[:, 0])] = 0
+    _, err = _check(points + moved @ box, box, EVERY, 3.0, full, "PSdD", capfd, monkeypatch)
+    assert _in_double(err) == 0
+    monkeypatch.setenv("VESIN_HIP_TESTS", "double")
+    _, err = _check(points + moved @ box, box, EVERY, 3.0, full, "PSdD", capfd, monkeypatch)
+    assert _in_double(err) == _tiles(err) > 0
 
 
 def test_more_rows_than_a_line_holds(capfd, monkeypatch):

@@ -63,7 +63,7 @@ struct CrowdedStatus {
     unsigned int max_candidates;
     unsigned int unsuitable; // a shift or wrap outside of the key's range
     unsigned int overflow;   // cells that found no room left
-    unsigned int padding;
+    unsigned int in_double;  // tiles whose pairs were all tested in double precision (where it is reported)
 };
 
 /// What the host reads after COUNT and the scan (pinned host memory).
@@ -88,6 +88,8 @@ struct CrowdedArgs {
     const uint64_t* first_row;    // WRITE: [n_points + 1], their exclusive scan
     uint64_t capacity;            // WRITE: rows that the output arrays hold; nothing is written when there are more
     SearchOutputs out;
+    uint32_t double_only;         // COUNT: not zero: every pair is tested in double precision (for tests)
+    uint32_t report;              // COUNT: count the tiles where they are (an atomic on one word: for tests)
 };
 
 /// Number `turn` of the tiles that a workgroup takes (n_tiles or beyond: none): every XCD walks a contiguous range of
@@ -578,7 +580,10 @@ __global__ __launch_bounds__(CROWDED_BLOCK, 5) void crowded_count_kernel(Crowded
                 out_of_range = beyond(wx, wy, wz, ORDERED_SHIFT_LIMIT);
                 sh.rows[lane] = 0;
             }
-            prepare_tile_tests(sh.tests, g, lane, n_i, point.x, point.y, point.z, wx, wy, wz);
+            prepare_tile_tests(sh.tests, g, lane, n_i, point.x, point.y, point.z, wx, wy, wz, args.double_only);
+            if (args.report != 0 && lane == 0 && sh.tests.usable == 0) {
+                atomicAdd(&args.status->in_double, 1u);
+            }
             if (__ballot(out_of_range) != 0 && lane == 0) {
                 atomicOr(&args.status->unsuitable, 1u);
             }

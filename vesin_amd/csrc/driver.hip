@@ -2551,6 +2551,7 @@ bool compute(
         oargs.first_row = first_row_of_point;
         oargs.status = ordered_status;
         oargs.report_order = std::getenv("VESIN_HIP_DEBUG") != nullptr ? 1u : 0u;
+        oargs.double_only = double_precision_only() ? 1u : 0u;
         const uint32_t blocks = ordered_blocks;
         // The order of every tile's candidates, for the writing pass (wasted when the counting pass finds the
         // system unsuitable, which the host only knows after both). Small systems do without: one more launch
@@ -2664,9 +2665,10 @@ bool compute(
             std::fprintf(
                 stderr,
                 "in-order search: rows %llu, most rows of a point %u, most candidates of a tile %u, unsuitable %u, "
-                "candidates of %u tiles ordered by window and of %u by buckets, %u tiles written by %u waves each%s and counted by %u: %s\n",
+                "candidates of %u tiles ordered by window and of %u by buckets, those of %u by a workgroup in double precision, "
+                "%u tiles written by %u waves each%s and counted by %u: %s\n",
                 found.total_rows, found.found.max_rows, found.found.max_candidates, found.found.unsuitable,
-                found.found.windowed, found.found.bucketed, found.n_tiles, oargs.write_split,
+                found.found.windowed, found.found.bucketed, found.found.in_double, found.n_tiles, oargs.write_split,
                 workgroups, oargs.count_split, suitable ? "used" : "not covered"
             );
         }
@@ -2720,6 +2722,8 @@ bool compute(
         cargs.status = crowded_status;
         cargs.rows_of_point = rows_of_point;
         cargs.first_row = first_row_of_point;
+        cargs.double_only = double_precision_only() ? 1u : 0u;
+        cargs.report = std::getenv("VESIN_HIP_DEBUG") != nullptr ? 1u : 0u;
         // workgroups of the passes, a multiple of the XCDs: each goes through as many tiles as there are for it (the
         // number of tiles, known on the device, may be far below its bound where most cells are empty)
         const uint32_t tile_blocks = static_cast<uint32_t>(std::min<size_t>((tiles_bound + N_XCD - 1) / N_XCD * N_XCD, 16384));
@@ -2799,8 +2803,8 @@ bool compute(
             };
             if (std::getenv("VESIN_HIP_DEBUG") != nullptr) {
                 std::fprintf(
-                    stderr, "crowded search: rows %llu, most candidates of a cell %u, unsuitable %u, %zu + %zu units of candidates and columns, room for %zu + %zu\n",
-                    found.total_rows, found.found.max_candidates, found.found.unsuitable, counted.candidate_units, counted.column_units,
+                    stderr, "crowded search: rows %llu, most candidates of a cell %u, unsuitable %u, %u tiles in double precision, %zu + %zu units of candidates and columns, room for %zu + %zu\n",
+                    found.total_rows, found.found.max_candidates, found.found.unsuitable, found.found.in_double, counted.candidate_units, counted.column_units,
                     room.candidate_units, room.column_units
                 );
             }

@@ -64,6 +64,8 @@ struct OrderedStatus {
     unsigned int arrived;        // one-launch search, in the host's copy: workgroups of the launch
     unsigned int gave_up;        // one-launch search, in the host's copy: the workgroups did not wait for each other
     unsigned int max_hits;       // most candidates with a hit of one tile (a workgroup per tile, where it is reported)
+    unsigned int in_double;      // tiles of a workgroup whose pairs were all tested in double precision (the same)
+    unsigned int padding;
 };
 
 /// What the host reads after the counting pass (pinned host memory, or a copy of it).
@@ -93,6 +95,7 @@ struct OrderedArgs {
     uint32_t count_split;       // COUNT: waves that share the candidates of one work item (at least 1; more than 1:
                                 // `rows_of_point` is zero on entry and the waves add to it)
     uint32_t report_order;      // SORT: count the tiles ordered either way, and so on (atomics on one word: for tests)
+    uint32_t double_only;       // COUNT by a workgroup per tile: not zero: every pair is tested in double precision (for tests)
     uint32_t guarded;           // WRITE launched before the host has seen what COUNT found: write nothing unless the
                                 // system suits this search and the rows fit the `capacity` of the arrays
     uint64_t capacity;

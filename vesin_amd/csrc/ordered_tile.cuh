@@ -287,7 +287,7 @@ __global__ __launch_bounds__(TILE_BLOCK, 6) void ordered_tile_kernel(OrderedArgs
             sh.tile_wrap[lane] = point.wrap;
             sh.rows[lane] = 0;
         }
-        prepare_tile_tests(sh.tests, g, lane, n_i, point.x, point.y, point.z, wx, wy, wz);
+        prepare_tile_tests(sh.tests, g, lane, n_i, point.x, point.y, point.z, wx, wy, wz, args.double_only);
         if (lane < 4) {
             sh.range[lane] = 0;
         }
@@ -326,6 +326,9 @@ __global__ __launch_bounds__(TILE_BLOCK, 6) void ordered_tile_kernel(OrderedArgs
             count_units<4, FULL>(sh, sorted, g, wave, n_candidates, first_i, n_i, lane, out_of_range, range);
         }
     } else {
+        if (args.report_order != 0 && threadIdx.x == 0) {
+            atomicAdd(&args.status->in_double, 1u);
+        }
         uint32_t rows = 0;
         for (uint32_t unit = wave; unit < n_units; unit += TILE_WAVES) {
             uint32_t column[1], at[1], original[1], biased[1];

@@ -627,6 +627,8 @@ __global__ __launch_bounds__(WAVES * WAVE) void small_system_kernel(SmallArgs ar
     found.arrived = gridDim.x;
     found.gave_up = 0;
     found.max_hits = 0;
+    found.in_double = 0;
+    found.padding = 0;
     const bool suitable = found.max_rows <= ORDERED_MAX_ROWS && found.max_candidates <= ORDERED_CANDIDATES &&
                           found.unsuitable == 0 && shared.first_bad == 0xFFFFFFFFu;
     if (blockIdx.x == 0 && t == 0) {

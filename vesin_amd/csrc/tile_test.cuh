@@ -41,8 +41,10 @@ struct TileTests {
 };
 
 /// By one wave, whose lane p < n_i holds point p of the tile: coordinates and the box vectors that it was moved by.
+/// `double_only`: not zero: they are not used.
 __device__ __forceinline__ void prepare_tile_tests(
-    TileTests& tests, const GridParams& g, uint32_t lane, uint32_t n_i, double x, double y, double z, int32_t wx, int32_t wy, int32_t wz
+    TileTests& tests, const GridParams& g, uint32_t lane, uint32_t n_i, double x, double y, double z, int32_t wx, int32_t wy, int32_t wz,
+    uint32_t double_only
 ) {
     double tx, ty, tz;
     shift_vector(g, -wx, -wy, -wz, tx, ty, tz);
@@ -80,7 +82,7 @@ __device__ __forceinline__ void prepare_tile_tests(
         tests.origin[1] = oy;
         tests.origin[2] = oz;
         // (also not for cutoffs whose squares come near the range of single precision)
-        tests.usable = eps < 0.01 * g.cutoff2 && g.cutoff2 > 1e-20 && g.cutoff2 < 1e+20 ? 1u : 0u;
+        tests.usable = double_only == 0 && eps < 0.01 * g.cutoff2 && g.cutoff2 > 1e-20 && g.cutoff2 < 1e+20 ? 1u : 0u;
     }
 }
 
