@@ -26,12 +26,18 @@
 namespace vesin_hip {
 
 /// `values` with `value` in lane `where` (both the same in every lane): one vector instruction, where a comparison and a
-/// selection take three. (The compiler has no builtin of its own for its intrinsic.)
+/// selection take three. (The compiler has no builtin of its own for its intrinsic: the build tries its name first.)
+#ifdef VESIN_HIP_NO_WRITE_LANE
+__device__ __forceinline__ uint32_t with_lane(uint32_t values, uint32_t value, uint32_t where) {
+    return static_cast<uint32_t>(lane_id()) == where ? value : values;
+}
+#else
 extern "C" __device__ uint32_t vesin_write_lane(uint32_t value, uint32_t where, uint32_t values) __asm("llvm.amdgcn.writelane.i32");
 
 __device__ __forceinline__ uint32_t with_lane(uint32_t values, uint32_t value, uint32_t where) {
     return vesin_write_lane(uniform(value), uniform(where), values);
 }
+#endif
 
 struct TileTests {
     float4 point[TILE_POINTS]; // -2 a, lower bound
