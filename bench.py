@@ -42,12 +42,12 @@ if ROOT not in sys.path:
 HBM_PEAK_GBS = 8000.0
 
 # HBM bytes moved by ONE launch of the single-pass search kernel on the 1M-atom workload, from rocprofv3 --pmc
-# FETCH_SIZE and WRITE_SIZE runs scaled by a device copy of known size (166.9 MB fetched + 3238.4 MB written). The figure belongs to the kernel sources whose
+# FETCH_SIZE and WRITE_SIZE runs scaled by a device copy of known size (167.0 MB fetched + 3238.0 MB written). The figure belongs to the kernel sources whose
 # digest is recorded with it: a run with other sources reports no traffic instead of a stale one.
 SEARCH_KERNEL_TRAFFIC = {
     "bytes": 3_405_000_000,
     "profile": "profiles/fused_search_config1_pmc.txt",
-    "kernel_sources_sha256": "513a8433a61ddf2ed07aec567bf181e7871bb8a2ca9aac13fd804b6f264a0a4d",
+    "kernel_sources_sha256": "ac11e80ccfdf95c6dd36635a91c586df26f280197fc365dcba7360b688ef456b",
 }
 KERNEL_SOURCES = ["device_common.cuh", "geometry.hpp", "cells.cuh", "search.cuh", "fused.cuh"]
 
