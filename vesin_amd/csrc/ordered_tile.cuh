@@ -6,8 +6,8 @@
 //   a scan over the points gives every point its first row;
 //   WRITE  (ordered_write_kernel) takes the records as they come, write_tile.cuh does the rest.
 // Against COUNT and SORT side by side, which order all candidates, and a WRITE that looks its candidates up by their place in
-// that order (us, COUNT and SORT -> COUNT and ORDER; WRITE): 1,000,000 atoms of diamond, full P S d 590 -> 340; 930 -> 840;
-// 100,000 points, 26 per cell, half P S d D 115 -> 60; 123 -> 78; 10,000 points, 29 per cell 30 -> 22; 40 -> 18.
+// that order (us, COUNT and SORT -> COUNT and ORDER; WRITE): 1,000,000 atoms of diamond, full P S d 590 -> 365; 930 -> 810;
+// 100,000 points, 26 per cell, half P S d D 115 -> 64; 123 -> 78; 10,000 points, 29 per cell 30 -> 22; 40 -> 18.
 #ifndef VESIN_HIP_ORDERED_TILE_CUH
 #define VESIN_HIP_ORDERED_TILE_CUH
 
@@ -217,9 +217,9 @@ __device__ __forceinline__ void count_units(
 }
 
 /// COUNT and ORDER. Bound by its vector instructions, which are 86 % of what the compute units can issue (1,000,000 atoms of
-/// diamond, 340 us): two thirds of them tests, the rest the order. Six workgroups per compute unit, 393 us with five. The
+/// diamond, 365 us): two thirds of them tests, the rest the order. Six workgroups per compute unit, 15 % slower with five. The
 /// places come from a bit per original index while two rounds of 65,536 indices cover the tile, and from buckets otherwise:
-/// indices without order take as long either way, runs of consecutive ones crowd a few buckets (340 us, 490 with one round).
+/// indices without order take as long either way, runs of consecutive ones crowd a few buckets (44 % slower with one round).
 template <bool FULL>
 __global__ __launch_bounds__(TILE_BLOCK, 6) void ordered_tile_kernel(OrderedArgs args, GridParams g) {
     constexpr int R = ORDERED_R;
@@ -575,7 +575,7 @@ __global__ __launch_bounds__(TILE_BLOCK, 6) void ordered_tile_kernel(OrderedArgs
     }
 }
 
-/// WRITE. Bound by its stores: 1,000,000 atoms of diamond, P S d, 840 us, 310 without them; see tile_stores, policy.hpp.
+/// WRITE. Bound by its stores: 1,000,000 atoms of diamond, P S d, 810 us, 460 without them; see tile_stores, policy.hpp.
 template <bool STAGED, TileStores STORES>
 __global__ __launch_bounds__(TILE_BLOCK, STAGED ? 4 : 5) void ordered_write_kernel(OrderedArgs args, GridParams g) {
     __shared__ TileWriteShared<STAGED> sh;

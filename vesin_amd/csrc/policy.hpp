@@ -271,7 +271,7 @@ enum TileStores : int {
 ///  - beyond, with vectors: 100,000 points, 26 per cell, half P S d D 108 / 88 / 78; 300,000 points, 20 per cell, full P S D
 ///    377 / 428 / 309, P S d D 452 / 508 / 356;
 ///  - with distances: 150,000 points, 20 per cell, full P S d 146 / 151 / 106, 300,000 points 285 / 318 / 278, diamond of
-///    110,592 atoms 107 / 101 / 84 and of 1,000,000 atoms 909 / 1030 / 840 (in random order 988 / 1255 / 1004); but 500,000
+///    110,592 atoms 107 / 101 / 84 and of 1,000,000 atoms 910 / 1020 / 810 (in random order 988 / 1255 / 1004); but 500,000
 ///    points, 12 per cell, half (25 rows per point) 252 / 242 / 295: with nearly every row in such a granule, sorting them
 ///    out is all that is left;
 ///  - pairs alone 122 / 175 / 150, pairs and shifts 217 / 246 / 224 (300,000 points): the second set of stores costs more

@@ -20,7 +20,7 @@
 namespace vesin_hip {
 
 // LDS and registers leave room for five workgroups per compute unit, four with vectors (six and five by spilling registers:
-// 1,000,000 atoms of diamond, P S d, 1008 against 806 us).
+// 1,000,000 atoms of diamond, P S d, 1010 against 810 us).
 constexpr int TILE_WAVES = 4;
 constexpr int TILE_BLOCK = TILE_WAVES * WAVE;
 constexpr uint32_t TILE_CHUNK = 512;
