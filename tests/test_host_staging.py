@@ -25,6 +25,14 @@ def test_results_come_the_faster_way(quantities, size, ratio):
     assert HostStaging().pays(sizes, columns="i" in quantities) == (ratio < 1.0)
 
 
+@pytest.mark.parametrize("quantities", ["d", "D", "PS", "PSdD", "SSSSD"])
+def test_what_is_surely_small_comes_one_by_one(quantities):
+    """At the last number of rows of which that is said, and the sizes that it is said of differ from those that are not."""
+    rows = max(k for k in range(1, 200_000) if HostStaging.surely_small(k, len(quantities)))
+    assert not HostStaging().pays([rows * BYTES[q] for q in quantities], columns=False)
+    assert 10_000 < rows < 100_000
+
+
 def test_no_rows_and_the_limit():
     staging = HostStaging()
     assert not staging.pays([0, 0], True)

@@ -72,6 +72,11 @@ class HostStaging:
     def _small(size, number):
         return size <= SMALL + number * SMALL_PER_ARRAY
 
+    @classmethod
+    def surely_small(cls, rows, number):
+        """Whether `number` arrays of so many rows, of 24 bytes at most, are small whatever they are."""
+        return cls._small((24 * rows + ALIGNMENT) * number, number)
+
     def fits(self, sizes):
         return 0 < self._places(sizes)[1] <= LIMIT
 

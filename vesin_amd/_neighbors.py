@@ -422,7 +422,7 @@ class NeighborList:
 
         data = None
         if not is_torch and n_pairs > 0:
-            data = self._host_results(quantities, pairs, shifts, distances, vectors)
+            data = self._host_results(quantities, n_pairs, pairs, shifts, distances, vectors)
         if data is None:
             data = []
             for quantity in quantities:
@@ -443,16 +443,19 @@ class NeighborList:
             self._last_views = (result_key, data)
         return data
 
-    def _host_results(self, quantities, pairs, shifts, distances, vectors):
+    def _host_results(self, quantities, n_pairs, pairs, shifts, distances, vectors):
         """The results as numpy arrays by way of pinned memory (from a calculator's second such call on), or None."""
-        import torch
-
         if not self.__dict__.get("_host_called", False):
             self._host_called = True
             return None
+        columns_wanted = "i" in quantities or "j" in quantities
+        if not columns_wanted and HOST_STAGING.surely_small(n_pairs, len(quantities)):
+            return None  # (before anything else: such calls take 100 us and less)
+        import torch
+
         arrays = {"i": pairs, "j": pairs, "P": pairs, "S": shifts, "d": distances, "D": vectors}
         sizes = [arrays[q].numel() * arrays[q].element_size() // (2 if q in "ij" else 1) for q in quantities if q in arrays]
-        if not HOST_STAGING.pays(sizes, "i" in quantities or "j" in quantities):
+        if not HOST_STAGING.pays(sizes, columns_wanted):
             return None  # (before anything is made for it)
         tensors, dtypes = [], []
         columns = None
