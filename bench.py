@@ -28,6 +28,7 @@ config3_single, config4a, config4b.
 """
 
 import argparse
+import gc
 import hashlib
 import json
 import os
@@ -174,6 +175,8 @@ def measure(workload, steps, warmup, torch, np):
     """First call, warm-up, the timed region of exactly `steps` calls, then per-call series (wall clock; HIP events)."""
     from vesin_amd import configs, enable_timings
 
+    # (a full collection of Python's takes 40 ms with PyTorch loaded, and would come in the middle of some region otherwise)
+    gc.collect()
     start = time.perf_counter()
     outputs = workload.call()
     torch.cuda.synchronize()
