@@ -25,12 +25,15 @@ def test_results_come_the_faster_way(quantities, size, ratio):
     assert HostStaging().pays(sizes, columns="i" in quantities) == (ratio < 1.0)
 
 
-@pytest.mark.parametrize("quantities", ["d", "D", "PS", "PSdD", "SSSSD"])
-def test_what_is_surely_small_comes_one_by_one(quantities):
-    """At the last number of rows of which that is said, and the sizes that it is said of differ from those that are not."""
-    rows = max(k for k in range(1, 200_000) if HostStaging.surely_small(k, len(quantities)))
-    assert not HostStaging().pays([rows * BYTES[q] for q in quantities], columns=False)
-    assert 10_000 < rows < 100_000
+@pytest.mark.parametrize("quantities", ["d", "D", "PS", "PSdD", "SSSSD", "i", "ijSd", "ijPSdD"])
+def test_what_is_said_at_a_glance_is_what_the_sizes_say(quantities):
+    staging, columns = HostStaging(), "i" in quantities
+    said = set()
+    for rows in [1, 2, 1000, *range(10_000, 60_000, 1000), *range(400_000, 9_000_000, 100_000)]:
+        glance = staging.pays_at_a_glance(rows, len(quantities), columns)
+        said.add(glance)
+        assert glance is None or glance == staging.pays([rows * BYTES[q] for q in quantities], columns)
+    assert said == {None, columns}
 
 
 def test_no_rows_and_the_limit():

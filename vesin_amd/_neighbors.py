@@ -449,14 +449,15 @@ class NeighborList:
             self._host_called = True
             return None
         columns_wanted = "i" in quantities or "j" in quantities
-        if not columns_wanted and HOST_STAGING.surely_small(n_pairs, len(quantities)):
-            return None  # (before anything else: such calls take 100 us and less)
+        pays = HOST_STAGING.pays_at_a_glance(n_pairs, len(quantities), columns_wanted)
+        if pays is None:
+            arrays = {"i": pairs, "j": pairs, "P": pairs, "S": shifts, "d": distances, "D": vectors}
+            sizes = [arrays[q].numel() * arrays[q].element_size() // (2 if q in "ij" else 1) for q in quantities if q in arrays]
+            pays = HOST_STAGING.pays(sizes, columns_wanted)
+        if not pays:
+            return None  # (before anything is made for it)
         import torch
 
-        arrays = {"i": pairs, "j": pairs, "P": pairs, "S": shifts, "d": distances, "D": vectors}
-        sizes = [arrays[q].numel() * arrays[q].element_size() // (2 if q in "ij" else 1) for q in quantities if q in arrays]
-        if not HOST_STAGING.pays(sizes, columns_wanted):
-            return None  # (before anything is made for it)
         tensors, dtypes = [], []
         columns = None
         for quantity in quantities:
